@@ -47,6 +47,7 @@ __global__ void pad_rows_kernel(float* __restrict__ q, int from, int m, int D)
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef int int4_t __attribute__((ext_vector_type(4)));
 
 /**
  * Four consecutive fp16 at columns k..k+3 of `row` (a row pointer, or row 0 of the matrix when the row is past
@@ -388,38 +389,70 @@ __device__ __forceinline__ int hash_log_dev(int total, int log_cap)
   return e < kMinLogHash ? kMinLogHash : (e > log_cap ? log_cap : e);
 }
 
+/** x of the lane whose number differs in bit o (1, 2, 4, 8 or 16): 1 and 2 as DPP moves, the others through the LDS
+ * crossbar. */
+template <int O>
+__device__ __forceinline__ float lane_xor(float x)
+{
+  if constexpr (O == 1)
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true));  // quad_perm 1 0 3 2
+  else if constexpr (O == 2)
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, true));  // quad_perm 2 3 0 1
+  else
+    return __shfl_xor(x, O);
+}
+
+/** The sum over an aligned group of G lanes by an xor butterfly from G / 2 down. */
+template <int G>
+__device__ __forceinline__ float group_sum(float x)
+{
+  if constexpr (G > 1) {
+    x += lane_xor<G / 2>(x);
+    return group_sum<G / 2>(x);
+  }
+  return x;
+}
+
+constexpr int kChunkPitch = 18;  // float2 words of a chunk of 16 coordinates in LDS: two chunks start in other banks
+
+/** LDS words (float2) of the scales and the query sketch of S coordinates. */
+__host__ __device__ constexpr auto sketch_lds_words(int S) -> int { return S / 16 * kChunkPitch; }
+
 /**
- * Sketch scores of a query's candidates 0..n-1 (search_kernels.cuh:227-251): an LR-lane group (LR = the
- * next power of two >= S / 16, at most 32) scores a candidate, lane `sub` reducing the 16-element chunks
- * sub, sub + LR, ... as u = fma(code, scale, -qs), d = fma(u, u, d), then an xor butterfly over the
- * group; the group's lane 0 hands (j, id, score) to put.  id_of(j) gives candidate j's id.  A
- * candidate's row is read by one load instruction of its group (one address translation per row: rows
- * lie anywhere in a sketch of many GB), and every group has kRows candidates' loads in flight before it
- * computes.
+ * Sketch scores of a query's candidates 0..n-1 (search_kernels.cuh:227-251): with LR = the next power of two >= S / 16
+ * (at most 32), the 16-element chunks sub, sub + LR, ... of a row are summed as u = fma(code, scale, -qs),
+ * d = fma(u, u, d), and the LR sums by an xor butterfly from LR / 2 down; put(j, id, score) takes them.  id_of(j) gives
+ * candidate j's id.
+ *
+ * A group of G lanes scores a candidate, lane sub taking the NJ chunks sub, sub + G, ... (chunk numbers differ in the
+ * butterfly's high bits, so a lane's own sums are combined first).  Where rows come from the caches it is bound by the
+ * arithmetic, 3 instructions a code, and small batches by a wavefront's rows in flight: an LR-lane group with one chunk a
+ * lane leaves lanes without a chunk idle (2 of 8 at S = 96), spends a butterfly of log2 LR steps on every 64 / LR rows and
+ * has 32 rows in flight a wavefront (LR = 8).  Four chunks a lane leave one step (S <= 128) on 32 rows, 64 in flight.
+ * Measured with the entries' loads overlapped too (collect_candidates): the gathers of 1,000 queries of 3840 list and 8192
+ * table entries (S = 96) 108, 190 and 104 -> 79, 143 and 77 us on unchanged threads, of one query 23, 30, 20 -> 15, 23,
+ * 15 us; 10,000 queries of 4096 table entries over 1.5M rows 552 -> 528 us (45 G rows/s: the random-row ceiling).  The scales and the
+ * query's sketch come from LDS (the same 16 bytes for every lane of a chunk, once for kRows rows); sq holds (scale, -qs),
+ * a chunk every kChunkPitch.  All loads of kRows rows are issued before the first is used, unconditionally
+ * (past-the-end candidates read row 0, a chunk past S the row's first).
  */
-template <int LR, typename IdOf, typename Put>
+template <int LR, int NJ, typename IdOf, typename Put>
 __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const signed char* __restrict__ code, int S,
                                               int pitch, const float2* sq, Put const& put)
 {
-  constexpr int kRows = 4;        // candidates per group in flight
-  constexpr int GPW   = 64 / LR;  // groups per wavefront
+  constexpr int J     = LR < 4 ? LR : 4;  // chunks of a lane in the butterfly
+  constexpr int G     = LR / J;           // lanes per candidate
+  constexpr int kRows = 2;                // candidates per group in flight
+  constexpr int GPW   = 64 / G;           // groups per wavefront
+  static_assert(NJ >= 1 && NJ <= J && NJ > J / 2, "the chunks of a row: more than half of LR");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int sub = lane & (LR - 1), grp = lane / LR;
-  const int k = sub * 16;         // this lane's chunk (S <= 512 = 32 chunks: one chunk per lane)
-  const bool has = k < S;
-  float s16[16], q16[16];         // the chunk's scale and query sketch, held in registers
-#pragma unroll
-  for (int e = 0; e < 16; e++) {
-    const float2 v = has ? sq[k + e] : make_float2(0.f, 0.f);
-    s16[e]         = v.x;
-    q16[e]         = v.y;
-  }
-  const int per_wave = GPW * kRows;
-  // Loads are unconditional (past-the-end candidates read row 0, chunkless lanes chunk 0) so that every row of
-  // the group is requested before the first one is used.  A past-the-end candidate's id is row 0 whatever id_of
-  // returns for the clamped index n - 1: that entry belongs to another group, which may already have replaced
-  // what id_of reads there (the slot list kept in `cand` is overwritten by ids as candidates are scored), so its
-  // value is no row id.
+  const int sub = lane & (G - 1), grp = lane / G;
+  const bool has_last = sub + G * (NJ - 1) < S / 16;  // this lane's last chunk lies in the row
+  const int last      = has_last ? 16 * G * (NJ - 1) : 0;
+  const int per_wave  = GPW * kRows;
+  // A past-the-end candidate's id is row 0 whatever id_of returns for the clamped index n - 1: that entry belongs to
+  // another group, which may already have replaced what id_of reads there (the slot list kept in `cand` is overwritten
+  // by ids as candidates are scored), so its value is no row id.
   const int stride = nw * per_wave;
   auto id_at = [&](int j) {
     const int v = id_of(min(j, n - 1));
@@ -432,34 +465,68 @@ __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const si
       id[r] = id_at(wid * per_wave + r * GPW + grp);
   }
   for (int j0 = wid * per_wave; j0 < n; j0 += stride) {
-    int4 w[kRows];
+    int4_t w[kRows][NJ];
 #pragma unroll
-    for (int r = 0; r < kRows; r++)
-      w[r] = *reinterpret_cast<const int4*>(code + static_cast<int64_t>(id[r]) * pitch + (has ? k : 0));
+    for (int r = 0; r < kRows; r++) {
+      const signed char* row = code + static_cast<int64_t>(id[r]) * pitch + sub * 16;
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+        w[r][j] = *reinterpret_cast<const int4_t*>(j + 1 < NJ ? row + 16 * G * j : row - (has_last ? 0 : sub * 16) + last);
+    }
     int idn[kRows];  // the next rows' ids, read while these rows are in flight
 #pragma unroll
     for (int r = 0; r < kRows; r++)
       idn[r] = j0 + stride < n ? id_at(j0 + stride + r * GPW + grp) : 0;
-    float d[kRows];
+    float c[kRows][J];  // the chunks' sums
 #pragma unroll
-    for (int r = 0; r < kRows; r++) {
-      const signed char* bb = reinterpret_cast<const signed char*>(&w[r]);
-      float acc             = 0.f;
+    for (int j = 0; j < J; j++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        float u = fmaf(static_cast<float>(bb[e]), s16[e], -q16[e]);
-        acc     = fmaf(u, u, acc);
+      for (int r = 0; r < kRows; r++)
+        c[r][j] = 0.f;
+    // the coefficients in pieces of four coordinates, the next piece's LDS reads issued before a piece is used and kept
+    // there by scheduling barriers (all of them hoisted would take 32 registers a chunk); their address is unknown to
+    // the compiler in every pass, or they would be held in registers over the loop
+    int at = 0;
+    asm volatile("" : "+v"(at));
+    const float4_t* coef[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+      coef[j] = reinterpret_cast<const float4_t*>(sq + at + (j + 1 < NJ || has_last ? sub + G * j : 0) * kChunkPitch);
+    float4_t next[2] = {coef[0][0], coef[0][1]};  // (scale, -qs) of two coordinates each
+#pragma unroll
+    for (int p = 0; p < 4 * NJ; p++) {
+      const int j          = p / 4, word = p % 4;  // coordinates 4 word .. 4 word + 3 of chunk j
+      const float4_t sc[2] = {next[0], next[1]};
+      if (p + 1 < 4 * NJ) {
+        next[0] = coef[(p + 1) / 4][2 * ((p + 1) % 4)];
+        next[1] = coef[(p + 1) / 4][2 * ((p + 1) % 4) + 1];
       }
-      d[r] = acc;
+#pragma unroll
+      for (int r = 0; r < kRows; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float x = static_cast<float>(static_cast<signed char>(w[r][j][word] >> (8 * e)));
+          const float u = fmaf(x, sc[e / 2][2 * (e % 2)], sc[e / 2][2 * (e % 2) + 1]);
+          c[r][j]       = fmaf(u, u, c[r][j]);
+        }
+#pragma unroll
+      for (int r = 0; r < kRows; r++)  // a row's sums stay in this piece (they would sink to where they are stored,
+        asm volatile("" : "+v"(c[r][j]));  // with all coefficients held until there)
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int r = 0; r < kRows; r++) {
-      if (!has) d[r] = 0.f;
+    for (int r = 0; r < kRows; r++)
+      if (!has_last) c[r][NJ - 1] = 0.f;
 #pragma unroll
-      for (int o = LR >> 1; o; o >>= 1)
-        d[r] += __shfl_xor(d[r], o);
-      const int j = j0 + r * GPW + grp;
-      if (j < n && sub == 0) put(j, id[r], d[r]);
+    for (int r = 0; r < kRows; r++) {
+#pragma unroll
+      for (int o = J >> 1; o; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < o; j++)
+          c[r][j] += c[r][j + o];
+      const float d = group_sum<G>(c[r][0]);
+      const int j   = j0 + r * GPW + grp;
+      if (j < n && sub == 0) put(j, id[r], d);
     }
 #pragma unroll
     for (int r = 0; r < kRows; r++)
@@ -469,20 +536,35 @@ __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const si
 
 /** Per-query state of collect_candidates (LDS). */
 struct collect_state {
-  int cnt, nsp, ulen;
+  int cnt;
   int hts;       // the hash set's slots
   int known;     // candidates whose scores came from earlier rows (row gathers)
   int wsum[16];  // a prefix sum's per-wavefront totals
+  int wcnt[16], wlen[16];  // collect_candidates: a wavefront's non-empty segments, their one length (-1: several)
 };
 
 /**
- * The distinct ids of a query's segments (search_kernels.cuh:138-222).  Wavefront 0 compacts the
- * non-empty segments (entry pointer sp and exclusive prefix pre of the lengths) into LDS; the entries
- * are then split evenly over the workgroup, kUnroll per thread with their loads issued together (entry
- * i of a query whose non-empty segments all have one length len lies in segment i / len, otherwise a
- * binary search over the prefix finds it); an LDS open-addressing set ht (of up to W slots) drops
- * duplicates, and each new id gets the next number by one atomic per wavefront: add(slot, id, h) with
- * h its hash-set slot, for slot < cap.  Returns min(distinct count, cap) in every thread.
+ * Loads through a pointer that lies in LDS or was computed from one: the address space is stated, since a generic
+ * pointer becomes a flat load, which counts as an LDS operation too, and every wait for an LDS read then waits for the
+ * loads in flight (the four entry loads of a thread ran one after another).
+ */
+template <typename T>
+__device__ __forceinline__ T load_global(const T* p)
+{
+  return *reinterpret_cast<const __attribute__((address_space(1))) T*>(reinterpret_cast<uint64_t>(p));
+}
+
+/**
+ * The distinct ids of a query's segments (search_kernels.cuh:138-222).  The workgroup compacts the non-empty segments
+ * (entry pointer sp and exclusive prefix pre of the lengths) into LDS; the entries are then split evenly over it, four a
+ * thread at a time with the next four's loads in flight; an LDS open-addressing set ht (of up to W slots, 16-byte
+ * aligned) drops duplicates, and each new id gets the next number by one atomic per wavefront and four entries:
+ * add(slot, id, h) with h its hash-set slot, for slot < cap.  Returns min(distinct count, cap) in every thread.
+ *
+ * Where an entry lies: when all non-empty segments have one length len (a search's always do), a multiple of 4, and
+ * start at multiples of 16 bytes, a thread's four entries are one 16-byte load of segment i / (len / 4); otherwise entry
+ * i of the query lies in segment i / len, or with several lengths where a binary search over the prefix finds it.
+ * A thread's four first tries at the set are issued together, so that their latencies overlap.
  *
  * kRows = false: segment c = (first entry, length) in the lists of copy c (at list_ptr[c]).
  * kRows = true:  segment = (row, length) of the neighbor table [N, table_len]; -1 entries skipped.
@@ -494,111 +576,152 @@ __device__ int collect_candidates(const int2* __restrict__ seg, int nseg, const 
 {
   constexpr int kUnroll = 4;
   const int q = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
+  const unsigned long long below = (1ULL << lane) - 1ULL;
   if (tid == 0) cs.cnt = 0;
-  if (wid == 0) {
-    int carry = 0, at = 0, lmin = 0x7fffffff, lmax = 0;
-    for (int c0 = 0; c0 < nseg; c0 += 64) {
-      const int c = c0 + lane;
-      int2 sl     = c < nseg ? seg[static_cast<int64_t>(q) * nseg + c] : make_int2(0, 0);
-      if (sl.y < 0) sl.y = 0;
-      const bool keep               = sl.y > 0;
-      const unsigned long long mask = __ballot(keep);
-      const int o                   = at + __popcll(mask & ((1ULL << lane) - 1ULL));
-      int v                         = sl.y;
+  int ns = 0, total = 0, len = 0;  // non-empty segments, their entries, their one length (0: none yet, -1: several)
+  bool aligned = true;
+  for (int c0 = 0; c0 < nseg; c0 += blockDim.x) {  // uniform
+    const int c = c0 + tid;
+    int2 sl     = c < nseg ? seg[static_cast<int64_t>(q) * nseg + c] : make_int2(0, 0);
+    if (sl.y < 0) sl.y = 0;
+    const bool keep               = sl.y > 0;
+    const unsigned long long mask = __ballot(keep);
+    int v                         = sl.y;
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        int u = __shfl_up(v, d);
-        if (lane >= d) v += u;
-      }
-      if (keep) {
-        pre[o] = carry + v - sl.y;
-        if constexpr (kRows)
-          sp[o] = table + static_cast<int64_t>(sl.x) * table_len;
-        else
-          sp[o] = reinterpret_cast<const int*>(list_ptr[c]) + sl.x;
-        lmin = min(lmin, sl.y);
-        lmax = max(lmax, sl.y);
-      }
-      carry += __shfl(v, 63);
-      at += __popcll(mask);
+    for (int d = 1; d < 64; d <<= 1) {
+      int u = __shfl_up(v, d);
+      if (lane >= d) v += u;
     }
-#pragma unroll
-    for (int d = 32; d; d >>= 1) {
-      lmin = min(lmin, __shfl_xor(lmin, d));
-      lmax = max(lmax, __shfl_xor(lmax, d));
+    const int* p = nullptr;
+    if (keep) {
+      if constexpr (kRows)
+        p = table + static_cast<int64_t>(sl.x) * table_len;
+      else
+        p = reinterpret_cast<const int*>(list_ptr[c]) + sl.x;
     }
-    if (lane == 0) {
-      pre[at] = carry;
-      cs.nsp  = at;
-      cs.ulen = at > 0 && lmin == lmax ? lmax : 0;  // one length for every non-empty segment
+    const int l0   = mask != 0 ? __shfl(sl.y, __ffsll(static_cast<long long>(mask)) - 1) : 0;
+    const bool one = __ballot(keep && sl.y != l0) == 0;
+    const bool odd = __ballot(keep && (reinterpret_cast<uint64_t>(p) & 15) != 0) != 0;
+    if (lane == 63) {
+      cs.wsum[wid] = v;
+      cs.wcnt[wid] = __popcll(mask) | (odd ? 1 << 30 : 0);
+      cs.wlen[wid] = one ? l0 : -1;
     }
+    __syncthreads();
+    int cb = ns, vb = total;  // segments and entries before this wavefront's
+    for (int w = 0; w < nw; w++) {
+      const int wc = cs.wcnt[w] & ~(1 << 30), wv = cs.wsum[w], wl = cs.wlen[w];
+      cb += w < wid ? wc : 0;
+      vb += w < wid ? wv : 0;
+      ns += wc;
+      total += wv;
+      aligned = aligned && (cs.wcnt[w] >> 30) == 0;
+      if (wl != 0) len = len == 0 || len == wl ? wl : -1;
+    }
+    if (keep) {
+      const int o = cb + __popcll(mask & below);
+      pre[o]      = vb + v - sl.y;
+      sp[o]       = p;
+    }
+    if (c0 + static_cast<int>(blockDim.x) < nseg) __syncthreads();  // wsum, wcnt and wlen are rewritten
   }
-  __syncthreads();
-  const int ns = cs.nsp, len = cs.ulen;
-  const int total = pre[ns];
-  const int HT    = 1 << hash_log_dev(total, logW);
-  for (int i = tid; i < HT; i += blockDim.x)
-    ht[i] = -1;
+  const int HT = 1 << hash_log_dev(total, logW);
+  for (int i = tid; i < HT / 4; i += blockDim.x)
+    reinterpret_cast<int4_t*>(ht)[i] = int4_t{-1, -1, -1, -1};
   if (tid == 0) cs.hts = HT;
   __syncthreads();
-  const int step = blockDim.x;
+  // the four ids v (-1: none) into the set
+  auto insert = [&](int4_t v) {
+    unsigned h[kUnroll];
+    int prev[kUnroll];
+    bool fresh[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; u++) {
+      if (v[u] >= N) v[u] = -1;  // -1: padding of a table row (search_kernels.cuh:213)
+      h[u]    = (static_cast<unsigned>(v[u]) * kIdHash) & (HT - 1);
+      prev[u] = 0;
+      if (v[u] >= 0) prev[u] = atomicCAS(&ht[h[u]], -1, v[u]);
+    }
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < kUnroll; u++) {
+      if (v[u] >= 0 && prev[u] != -1 && prev[u] != v[u]) {
+        for (int p = 1; p < HT; p++) {
+          h[u]    = (h[u] + 1) & (HT - 1);
+          prev[u] = atomicCAS(&ht[h[u]], -1, v[u]);
+          if (prev[u] == -1 || prev[u] == v[u]) break;
+        }
+      }
+      fresh[u] = v[u] >= 0 && prev[u] == -1;
+      mine += __popcll(__ballot(fresh[u]));
+    }
+    if (mine != 0) {  // uniform over the wavefront
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&cs.cnt, mine);
+      at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+      for (int u = 0; u < kUnroll; u++) {
+        const unsigned long long mask = __ballot(fresh[u]);
+        const int slot                = at + __popcll(mask & below);
+        if (fresh[u] && slot < cap) add(slot, v[u], h[u]);
+        at += __popcll(mask);
+      }
+    }
+  };
   // i / len as (i + 1/2) * fl(1 / len), truncated: the product's relative error is at most 2^-23 (1 + 2^-24), under
   // the 1/(2 len) between (i + 1/2) / len and an integer when i + 1/2 < 2^22 (a search reads at most kMaxHash
   // entries per query); larger totals divide
-  const float inv_len = len > 0 ? 1.f / static_cast<float>(len) : 0.f;
   const bool by_recip = total < (1 << 22);
-  for (int i0 = 0; i0 < total; i0 += step * kUnroll) {
-    int v[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {  // kUnroll entries' loads issued together (past the end: the last)
-      const int i = min(i0 + u * step + tid, total - 1);
-      int sg;
+  auto quotient       = [&](int i, int l, float inv) {
+    return by_recip ? static_cast<int>((static_cast<float>(i) + 0.5f) * inv) : i / l;
+  };
+  const int step = blockDim.x;
+  if (len > 0 && (len & 3) == 0 && aligned) {
+    const int l4 = len >> 2, n4 = total >> 2;
+    const float inv = 1.f / static_cast<float>(l4);
+    auto load       = [&](int i) {  // past the end: the last
+      i            = min(i, n4 - 1);
+      const int sg = quotient(i, l4, inv);
+      return load_global(reinterpret_cast<const int4_t*>(sp[sg]) + (i - sg * l4));
+    };
+    int4_t next = load(tid);
+    for (int i0 = 0; i0 < n4; i0 += step) {  // uniform
+      const int4_t v = next;
+      if (i0 + step < n4) next = load(i0 + step + tid);
+      insert(i0 + tid < n4 ? v : int4_t{-1, -1, -1, -1});
+    }
+  } else if (total > 0) {
+    const float inv = len > 0 ? 1.f / static_cast<float>(len) : 0.f;
+    auto where      = [&](int i) {
+      int sg = 0;
       if (len > 0) {
-        sg = by_recip ? static_cast<int>((static_cast<float>(i) + 0.5f) * inv_len) : i / len;
+        sg = quotient(i, len, inv);
       } else {
-        int lo = 0, hi = ns - 1;
-        while (lo < hi) {
-          int mid = (lo + hi + 1) >> 1;
+        int hi = ns - 1;
+        while (sg < hi) {
+          const int mid = (sg + hi + 1) >> 1;
           if (pre[mid] <= i)
-            lo = mid;
+            sg = mid;
           else
             hi = mid - 1;
         }
-        sg = lo;
       }
-      v[u] = sp[sg][i - pre[sg]];
-    }
+      return sp[sg] + (i - pre[sg]);
+    };
+    for (int i0 = 0; i0 < total; i0 += step * kUnroll) {  // uniform
+      const int* p[kUnroll];
+      int4_t v;
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++)
-      if (i0 + u * step + tid >= total) v[u] = -1;
+      for (int u = 0; u < kUnroll; u++)
+        p[u] = where(min(i0 + u * step + tid, total - 1));
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      bool fresh = false;
-      unsigned h = 0;
-      if (v[u] >= 0 && v[u] < N) {  // -1: padding of a table row (search_kernels.cuh:213)
-        h = (static_cast<unsigned>(v[u]) * kIdHash) & (HT - 1);
-        for (int p = 0; p < HT; p++) {
-          int prev = atomicCAS(&ht[h], -1, v[u]);
-          if (prev == -1) {
-            fresh = true;
-            break;
-          }
-          if (prev == v[u]) break;
-          h = (h + 1) & (HT - 1);
-        }
-      }
-      const unsigned long long mask = __ballot(fresh);
-      if (mask != 0) {
-        const int leader = __ffsll(static_cast<long long>(mask)) - 1;
-        int at           = 0;
-        if (lane == leader) at = atomicAdd(&cs.cnt, __popcll(mask));
-        at = __shfl(at, leader);
-        if (fresh) {
-          const int slot = at + __popcll(mask & ((1ULL << lane) - 1ULL));
-          if (slot < cap) add(slot, v[u], h);
-        }
-      }
+      for (int u = 0; u < kUnroll; u++)  // the loads issued together
+        v[u] = load_global(p[u]);
+#pragma unroll
+      for (int u = 0; u < kUnroll; u++)
+        if (i0 + u * step + tid >= total) v[u] = -1;
+      insert(v);
     }
   }
   __syncthreads();
@@ -657,16 +780,16 @@ __device__ int collect_segments_whole(const int2* __restrict__ seg, int nseg, co
 {
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
   if (tid == 0) {
-    cs.cnt  = 0;
-    cs.ulen = 0;
+    cs.cnt     = 0;
+    cs.wsum[0] = 0;
   }
   __syncthreads();
   int part = 0;
   for (int c = tid; c < nseg; c += blockDim.x)
     part += max(seg[static_cast<int64_t>(q) * nseg + c].y, 0);
-  if (part > 0) atomicAdd(&cs.ulen, part);
+  if (part > 0) atomicAdd(&cs.wsum[0], part);
   __syncthreads();
-  const int HT = 1 << hash_log_dev(cs.ulen, logW);
+  const int HT = 1 << hash_log_dev(cs.wsum[0], logW);
   for (int i = tid; i < HT; i += blockDim.x)
     ht[i] = -1;
   if (tid == 0) cs.hts = HT;
@@ -984,9 +1107,8 @@ __device__ __forceinline__ int select_by_bins(const unsigned* __restrict__ kd, c
  * sketch_scores with LR = the reference's lanes per candidate for this S), written to the query's rows of
  * cand / dist and their count to nout.  The candidates are kept as hash-set slot numbers: 16-bit in LDS
  * (kLdsSlots), or, when they do not fit in LDS beside a large hash set, in the query's own row of cand,
- * where candidate j's slot is read and then overwritten by its id by the one lane group that scores it.  A list
- * gather runs on kGatherListThreads, a row gather on kGatherRowThreads: the row gather's larger hash set leaves room
- * for fewer workgroups per CU, so each gets more threads.
+ * where candidate j's slot is read and then overwritten by its id by the one lane group that scores it.  NT threads: see
+ * gather_impl.
  */
 constexpr int kKnown = static_cast<int>(0x80000000u);  // a hash-set entry whose id's score came from an earlier row
 
@@ -1112,25 +1234,25 @@ __device__ int take_known(earlier_entries const& ee, int const (&pid)[kKnownPre]
   return kept;
 }
 
-template <bool kRows, int LR, bool kLdsSlots, bool kBalanced>
-__global__ __launch_bounds__(kRows ? kGatherRowThreads : kGatherListThreads) void gather_kernel(
+template <bool kRows, int LR, int NJ, int NT, bool kLdsSlots, bool kBalanced>
+__global__ __launch_bounds__(NT) void gather_kernel(
   const int2* __restrict__ seg, int nseg, const long long* __restrict__ list_ptr,
   const int* __restrict__ table, int table_len, int64_t N, const signed char* __restrict__ code,
   const float* __restrict__ scale, const float* __restrict__ qs, int S, int pitch, int W, int logW, int cap,
   int* __restrict__ cand, float* __restrict__ dist, int* __restrict__ nout, earlier_rows er, int* __restrict__ nknown)
 {
   const int q = blockIdx.x;
-  extern __shared__ long long smq[];
-  const int** sp = reinterpret_cast<const int**>(smq);  // [nseg] first entry of every non-empty segment
-  float2* sq     = reinterpret_cast<float2*>(smq + nseg);  // [S] (scale, query sketch) per coordinate
-  int* pre       = reinterpret_cast<int*>(sq + S);  // [nseg + 1] exclusive prefix of the compacted lengths
-  int* ht        = pre + nseg + 1;                  // [W] hash set
-  auto* cl       = reinterpret_cast<unsigned short*>(ht + W);  // [cap] slots of the candidates (kLdsSlots)
+  extern __shared__ int4 smq[];
+  int* ht        = reinterpret_cast<int*>(smq);         // [W] hash set (16-byte aligned)
+  float2* sq     = reinterpret_cast<float2*>(ht + W);   // (scale, -query sketch), kChunkPitch a chunk (16-byte aligned)
+  const int** sp = reinterpret_cast<const int**>(sq + sketch_lds_words(S));  // [nseg] first entry of a segment
+  int* pre       = reinterpret_cast<int*>(sp + nseg);   // [nseg] exclusive prefix of the compacted lengths
+  auto* cl       = reinterpret_cast<unsigned short*>(pre + nseg);  // [cap] slots of the candidates (kLdsSlots)
   __shared__ collect_state cs;
   int* crow   = cand + static_cast<int64_t>(q) * W;
   float* drow = dist + static_cast<int64_t>(q) * W;
   for (int i = threadIdx.x; i < S; i += blockDim.x)
-    sq[i] = make_float2(scale[i], qs[static_cast<int64_t>(q) * S + i]);
+    sq[i / 16 * kChunkPitch + i % 16] = make_float2(scale[i], -qs[static_cast<int64_t>(q) * S + i]);
   auto keep_slot = [&](int slot, int, unsigned h) {
     if constexpr (kLdsSlots)
       cl[slot] = static_cast<unsigned short>(h);
@@ -1149,7 +1271,7 @@ __global__ __launch_bounds__(kRows ? kGatherRowThreads : kGatherListThreads) voi
       const earlier_entries ee(er, q);
 #pragma unroll
       for (int u = 0; u < kKnownPre; u++)
-        pok[u] = ee.load(threadIdx.x + u * kGatherRowThreads, pid[u], psc[u]);
+        pok[u] = ee.load(threadIdx.x + u * NT, pid[u], psc[u]);
     }
   }
   int n = 0;
@@ -1160,10 +1282,10 @@ __global__ __launch_bounds__(kRows ? kGatherRowThreads : kGatherListThreads) voi
   int nu = n;  // the candidates scored here
   if constexpr (kRows && kLdsSlots) {
     if (reuse && cs.cnt <= cap)  // uniform (read after the collection's last barrier)
-      nu = take_known<kGatherRowThreads>(earlier_entries(er, q), pid, psc, pok, N, n, ht, cs.hts, cl, crow, drow, cs);
+      nu = take_known<NT>(earlier_entries(er, q), pid, psc, pok, N, n, ht, cs.hts, cl, crow, drow, cs);
   }
   if (nknown != nullptr && threadIdx.x == 0) nknown[q] = n - nu;
-  sketch_scores<LR>(
+  sketch_scores<LR, NJ>(
     nu,
     [&](int j) {
       if constexpr (kLdsSlots)
@@ -2102,7 +2224,7 @@ auto gather_cap(int W, int nseg, int max_len) -> int
 
 auto gather_smem(int W, int S, int nseg, int max_len, bool lds_slots) -> size_t
 {
-  return static_cast<size_t>(nseg) * sizeof(long long) + static_cast<size_t>(W + 2 * S + nseg + 1) * sizeof(int) +
+  return static_cast<size_t>(nseg) * sizeof(long long) + static_cast<size_t>(W + 2 * sketch_lds_words(S) + nseg) * sizeof(int) +
          (lds_slots ? static_cast<size_t>(gather_cap(W, nseg, max_len)) * sizeof(unsigned short) : 0);
 }
 
@@ -2134,28 +2256,43 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
   int Lr = 1;  // the reference's lanes per candidate: the next power of two >= S / 16, at most 32
   while (Lr < S / 16 && Lr < 32)
     Lr <<= 1;
-  auto go = [&](auto rows_tag, auto lr_tag) {
+  // 512 threads a query; 256 for few entries, whose small hash sets leave room for more workgroups.  Measured, 256 / 512
+  // threads: 800 list entries a query 129 / 162 us and 1024 table entries 111 / 179 us (10,000 queries of 128 codes);
+  // 1440 list entries 280 / 279 us; 6400 list entries 74 / 57 us (1,000 queries), 3200 79 / 69 us.  1024 threads leave
+  // one workgroup a CU: 280 -> 506 us.
+  const bool wide = static_cast<int64_t>(nseg) * max_len > kGatherFew || !lds_slots || !kBalanced;
+  const int G  = std::max(1, Lr / 4);         // lanes per candidate and
+  const int nj = (S / 16 + G - 1) / G;        // chunks a lane: sketch_scores
+  auto go = [&](auto rows_tag, auto lr_tag, auto nj_tag) {
     constexpr bool kRowsTag = decltype(rows_tag)::value;
     constexpr int LR        = decltype(lr_tag)::value;
+    constexpr int NJ        = decltype(nj_tag)::value;
     auto launch             = [&](auto kernel) {
       allow_lds(reinterpret_cast<const void*>(kernel), smem);
-      kernel<<<m, kRowsTag ? kGatherRowThreads : kGatherListThreads, smem, s>>>(
-        seg, nseg, list_ptr, table, table_len, n, code, scale, qs, S, pitch, W, logW, cap, cand, dist, nout, er,
-        nknown);
+      kernel<<<m, wide ? 512 : 256, smem, s>>>(seg, nseg, list_ptr, table, table_len, n, code, scale, qs, S, pitch, W,
+                                               logW, cap, cand, dist, nout, er, nknown);
     };
-    if (lds_slots)
-      launch(&gather_kernel<kRowsTag, LR, true, kBalanced>);
+    if (!lds_slots)
+      launch(&gather_kernel<kRowsTag, LR, NJ, 512, false, kBalanced>);
+    else if (wide)
+      launch(&gather_kernel<kRowsTag, LR, NJ, 512, true, kBalanced>);
+    else if constexpr (kBalanced)
+      launch(&gather_kernel<kRowsTag, LR, NJ, 256, true, kBalanced>);
+  };
+  auto by_nj = [&](auto rows_tag, auto lr_tag) {
+    if (nj <= 3)
+      go(rows_tag, lr_tag, std::integral_constant<int, 3>{});
     else
-      launch(&gather_kernel<kRowsTag, LR, false, kBalanced>);
+      go(rows_tag, lr_tag, std::integral_constant<int, 4>{});
   };
   auto by_lr = [&](auto rows_tag) {
     switch (Lr) {
-      case 1: go(rows_tag, std::integral_constant<int, 1>{}); break;
-      case 2: go(rows_tag, std::integral_constant<int, 2>{}); break;
-      case 4: go(rows_tag, std::integral_constant<int, 4>{}); break;
-      case 8: go(rows_tag, std::integral_constant<int, 8>{}); break;
-      case 16: go(rows_tag, std::integral_constant<int, 16>{}); break;
-      default: go(rows_tag, std::integral_constant<int, 32>{}); break;
+      case 1: go(rows_tag, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
+      case 2: go(rows_tag, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}); break;
+      case 4: by_nj(rows_tag, std::integral_constant<int, 4>{}); break;
+      case 8: by_nj(rows_tag, std::integral_constant<int, 8>{}); break;
+      case 16: by_nj(rows_tag, std::integral_constant<int, 16>{}); break;
+      default: by_nj(rows_tag, std::integral_constant<int, 32>{}); break;
     }
   };
   if (rows)

@@ -18,8 +18,7 @@ constexpr int kMaxKeepSort    = 1024;   // kept + reranked keys sorted together
 constexpr int kMaxSketchKO    = 1024;   // kept entries of the sketch merge
 constexpr int kPickHash       = 8192;   // hash set of the expanded start points
 constexpr int kMaxExpanded    = 6144;   // start points expanded by earlier waves
-constexpr int kGatherListThreads = 256;  // gathers of cell lists (first round): small hash sets, many per CU
-constexpr int kGatherRowThreads  = 512;  // gathers of neighbor-table rows (waves)
+constexpr int kGatherFew      = 1024;   // entries a query up to which a gather takes 256 threads (gather_impl)
 constexpr int kKeepThreads    = 256;
 
 /** log2 of the hash set of a query reading `total` entries: ceil(log2(1.5 total)) in [11, log_cap]. */

@@ -535,6 +535,40 @@ def test_row_layouts_match_oracle(L, D, S):
         dd = dev(dist)
 
 
+# How a gather reads a query's entries and splits a sketch row over lanes (S / 16 chunks: 3 or 4 a lane, the last partly
+# past the row at S = 80 and 272): segments of one length, a multiple of 4 and 16-byte aligned (16-byte loads), of one
+# other length, of several lengths, starting off alignment; more segments than threads (300 of 256, 700 of 512, the
+# latter with the slot list in global memory); up to 1024 entries a query (256 threads) and more (512).
+@pytest.mark.parametrize("S,table_len,nst,lens", [(128, 16, 24, "one"), (80, 16, 24, "one"), (272, 16, 65, "one"),
+                                                  (112, 15, 24, "one"), (96, 16, 24, "several"), (64, 6, 24, "one"),
+                                                  (48, 3, 300, "one"), (32, 16, 700, "one"), (16, 16, 64, "short")])
+def test_gather_entry_and_lane_splits(L, S, table_len, nst, lens):
+    import octex_amd
+
+    D = max(S, 32)
+    X, Q = clustered(n=1200, m=12, d=D, clusters=6, seed=S + nst)
+    index, _ = octex_amd.build_in_memory(X, copies=3, blocks=2, pca_dims=32, list_len=8, table_len=table_len,
+                                         log_buckets=8, sketch_width=S, member_lists=True, reverse_edges=False, seed=3)
+    rix = O.Index(index)
+    rdix = dict(lists=dev(rix.lists), table=dev(rix.table), sketch=dev(rix.sketch), scale=dev(rix.scale))
+    g = np.random.default_rng(S + table_len + nst)
+    m = len(Q)
+    length = {"one": np.full((m, nst), table_len), "several": g.integers(0, table_len + 1, (m, nst)),
+              "short": np.full((m, nst), 8)}[lens]
+    seg2 = np.stack([g.integers(0, rix.n, (m, nst)), length], -1).astype(np.int32)
+    seg2[:, -3:] = 0
+    seg2[0] = 0
+    qs = g.standard_normal((m, S)).astype(np.float32)
+    cand, dist, nout = gather_gpu(L, rix, rdix, dev(seg2), qs, rows=1, W=1 << 15 if nst == 700 else 4096)
+    check_gather(rix, seg2, qs, cand, dist, nout, rows=True)
+    # lists: full ones, and parts of them that start one entry in
+    for first, count in ((0, 8), (1, 4), (0, 5)):
+        rows = g.integers(0, rix.lists.shape[1] // 8, (m, rix.copies)) * 8
+        segl = np.stack([rows + first, np.full((m, rix.copies), count)], -1).astype(np.int32)
+        cand, dist, nout = gather_gpu(L, rix, rdix, dev(segl), qs, rows=0)
+        check_gather(rix, segl, qs, cand, dist, nout, rows=False)
+
+
 # ---------------------------------------------------------------- the rerank's history of selected ids
 
 
