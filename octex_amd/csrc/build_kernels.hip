@@ -22,6 +22,9 @@ namespace {
 
 constexpr int kMaxW = 64;  // 8 * blocks
 
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
 /** A[i, :] = x[i * step, :] - mean (fp64), for the scatter matrix of the PCA sample. */
 __global__ void pca_sample_kernel(const __half* __restrict__ x, int64_t ns, int64_t step, int d,
                                   const float* __restrict__ mean, double* __restrict__ A)
@@ -65,33 +68,45 @@ __global__ __launch_bounds__(256) void scatter_kernel(const double* __restrict__
   if (a0 + ty < d && b0 + tx < d) G[static_cast<int64_t>(a0 + ty) * d + b0 + tx] = acc;
 }
 
-/** y [n, w] = (x - mean) @ U + shift (fp32): one thread per row, U [d, w] in LDS. */
-__global__ __launch_bounds__(256) void project_rows_kernel(const __half* __restrict__ x, int64_t n, int d,
-                                                           const float* __restrict__ mean,
-                                                           const float* __restrict__ U,
-                                                           const float* __restrict__ shift, int w,
-                                                           float* __restrict__ y)
+/**
+ * y [n, W] = (x - mean) @ U + shift (fp32), each output one sequential fma chain over d.  A thread holds its row's W
+ * sums in registers; U, the mean and the shift are the same for all threads, so they come by scalar loads and feed the
+ * fmas as scalar operands.  A row is read 8 values at a time (VEC: d a multiple of 8), else 2 (d is even).
+ * Bound by the fmas (n d W; 150k x 128 -> 32: 37.5k cycles of the chip).  Measured there 950 -> 42 us: with a runtime W
+ * the sums had lived in scratch memory.
+ */
+template <int W, bool VEC>
+__global__ __launch_bounds__(64) void project_rows_kernel(const __half* __restrict__ x, int64_t n, int d,
+                                                          const float* __restrict__ mean, const float* __restrict__ U,
+                                                          const float* __restrict__ shift, float* __restrict__ y)
 {
-  extern __shared__ float su[];
-  float* sm = su + d * w;
-  for (int t = threadIdx.x; t < d * w; t += blockDim.x)
-    su[t] = U[t];
-  for (int t = threadIdx.x; t < d; t += blockDim.x)
-    sm[t] = mean[t];
-  __syncthreads();
-  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float acc[kMaxW];
-  for (int s = 0; s < w; s++)
+  constexpr int kStep = VEC ? 8 : 2;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  const __half* r = x + (i < n ? i : 0) * d;  // past the end: row 0, nothing stored
+  float acc[W];
+#pragma unroll
+  for (int s = 0; s < W; s++)
     acc[s] = 0.f;
-  const __half* r = x + i * d;
-  for (int k = 0; k < d; k++) {
-    float v = __half2float(r[k]) - sm[k];
-    for (int s = 0; s < w; s++)
-      acc[s] = fmaf(v, su[k * w + s], acc[s]);
+  for (int k = 0; k < d; k += kStep) {
+    __half h[kStep];
+    if constexpr (VEC)
+      *reinterpret_cast<uint4*>(h) = *reinterpret_cast<const uint4*>(r + k);
+    else
+      *reinterpret_cast<unsigned*>(h) = *reinterpret_cast<const unsigned*>(r + k);
+#pragma unroll
+    for (int e = 0; e < kStep; e++) {
+      const float v = __half2float(h[e]) - mean[k + e];
+#pragma unroll
+      for (int s = 0; s < W; s++)
+        acc[s] = fmaf(v, U[(k + e) * W + s], acc[s]);
+    }
   }
-  for (int s = 0; s < w; s++)
-    y[i * w + s] = acc[s] + shift[s];
+  if (i >= n) return;
+  float* o = y + i * W;
+#pragma unroll
+  for (int s = 0; s < W; s += 4)
+    *reinterpret_cast<float4_t*>(o + s) =
+      float4_t{acc[s] + shift[s], acc[s + 1] + shift[s + 1], acc[s + 2] + shift[s + 2], acc[s + 3] + shift[s + 3]};
 }
 
 /** keys[i] = cell id of y[i] / f (division, as build_cells.cuh:69-71), idx[i] = i. */
@@ -365,9 +380,6 @@ __global__ void float_to_half_kernel(const float* __restrict__ x, int64_t total,
 }
 
 // ------------------------------------------------------------------ exact k nearest neighbors
-
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kKnnQ    = 64;   // query rows per workgroup
 constexpr int kKnnRows = 128;  // database rows per step: 4 waves x 32
@@ -891,11 +903,27 @@ void project_rows(const __half* x, int64_t n, int d, const float* mean, const fl
                   float* y, hipStream_t s)
 {
   OCTEX_EXPECTS(w <= kMaxW, "octex: blocks must be at most 8");
-  const size_t smem = static_cast<size_t>(d * w + d) * sizeof(float);
+  const size_t smem = static_cast<size_t>(d * w + d) * sizeof(float);  // the largest projection taken
   OCTEX_EXPECTS(smem <= 160 * 1024, "octex: dimension x 8 blocks too large for the projection kernel");
-  OCTEX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&project_rows_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem)));
-  project_rows_kernel<<<grid_for(n, 256), 256, smem, s>>>(x, n, d, mean, U, shift, w, y);
+  if (n == 0) return;
+  const unsigned g = grid_for(n, 64);
+  auto go          = [&](auto w_tag) {
+    constexpr int W = decltype(w_tag)::value;
+    if (d % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0)
+      project_rows_kernel<W, true><<<g, 64, 0, s>>>(x, n, d, mean, U, shift, y);
+    else
+      project_rows_kernel<W, false><<<g, 64, 0, s>>>(x, n, d, mean, U, shift, y);
+  };
+  switch (w) {
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 24: go(std::integral_constant<int, 24>{}); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    case 40: go(std::integral_constant<int, 40>{}); break;
+    case 48: go(std::integral_constant<int, 48>{}); break;
+    case 64: go(std::integral_constant<int, 64>{}); break;
+    default: fail("octex: blocks must be 1-6 or 8");
+  }
   OCTEX_HIP(hipGetLastError());
 }
 
