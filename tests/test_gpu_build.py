@@ -200,6 +200,26 @@ def test_exact_table_matches_oracle(octex, tmp_path, n, d, reverse):
     assert np.array_equal(tg, tc)
 
 
+@pytest.mark.parametrize("n,blocks", [(900, 1), (1500, 3), (70000, 4), (3000, 8)])
+def test_kmeans_centers_give_the_same_ivf_lists(octex, n, blocks):
+    """Every list probed, IVF lists hold the exact l nearest rows whatever the centers are, if every row lies in the
+    list of one center: rows lost or doubled by the assignment (16 rows a workgroup, 64 from 65,536 rows) would show."""
+    X = clustered(n=n, m=1, d=64, clusters=9, seed=n)[0].astype(np.float16)
+    kw = dict(copies=2, blocks=blocks, list_len=16, log_buckets=10, table_len=0, min_cell=3, seed=2)
+    ivf, _ = octex.build_in_memory(X, list_probes=1 << 20, **kw)
+    exact, _ = octex.build_in_memory(X, exact_lists=True, **kw)
+    nlist = max(64, int(4 * np.sqrt(n)))
+    for c in range(2):
+        a, b = ivf.array("lists", np.int32, copy=c), exact.array("lists", np.int32, copy=c)
+        assert a.shape == b.shape
+        if nlist <= 128:  # every list is probed
+            assert (a != b).mean() < 1e-3  # near ties of the two distance forms
+        else:
+            assert (a == b).mean() > 0.5 and (a < n).all()
+        rows = a.reshape(-1, 16)[a.reshape(-1, 16).min(1) >= 0]
+        assert all(len(set(r)) == 16 for r in rows[:500])
+
+
 def test_exact_table_real_valued(octex, data, tmp_path):
     """On real-valued rows the forward table holds the exact k nearest (fp64) up to near ties of the
     fp32 expanded distance |x|^2 + |y|^2 - 2 x.y, nearest first; no self, no duplicates."""
