@@ -382,9 +382,12 @@ __global__ void float_to_half_kernel(const float* __restrict__ x, int64_t total,
 // ------------------------------------------------------------------ exact k nearest neighbors
 
 constexpr int kKnnQ    = 64;   // query rows per workgroup
-constexpr int kKnnRows = 128;  // database rows per step: 4 waves x 32
-constexpr int kKnnCap  = 256;  // LDS keys per query row: the K kept (K <= 128) and one step's appends
-constexpr int kKnnChunk = 8;   // k steps whose fragments are loaded together
+constexpr int kKnnWaves = 8;   // wavefronts of a workgroup, 32 database rows of a step each
+constexpr int kKnnRows = 32 * kKnnWaves;
+constexpr int kKnnMaxK = 128;  // rows kept per query row
+constexpr int kKnnCap  = 256;  // LDS keys per query row: the K kept and new ones
+constexpr int kKnnHold  = 8;   // k steps up to which the queries' fragments are held in registers
+constexpr int kKnnChunk = 4;   // k steps whose fragments are loaded together otherwise
 
 __device__ __forceinline__ float knn_f(__half v) { return __half2float(v); }
 __device__ __forceinline__ float knn_f(float v) { return v; }
@@ -483,36 +486,73 @@ struct knn_op<float> {
   }
 };
 
+/** The K-th smallest (1 <= K <= 256) of the four 32-bit values of every lane, by bisection from the top bit: the largest T
+ * with fewer than K values below it.  `valid` marks the values that count. */
+__device__ __forceinline__ unsigned kth_smallest(unsigned const (&v)[4], bool const (&valid)[4], int K)
+{
+  unsigned T = 0;
+  for (int bit = 31; bit >= 0; bit--) {
+    const unsigned probe = T | (1u << bit);
+    int below            = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      below += __popcll(__ballot(valid[j] && v[j] < probe));
+    if (below < K) T = probe;
+  }
+  return T;
+}
+
 /**
- * Every query row's LDS keys (ordered distance << 32 | row) sorted ascending by a bitonic network over
- * all kKnnQ x kKnnCap slots (unused slots padded with ~0), the first K kept, the threshold set to the
- * K-th distance.  Called by the whole workgroup.
+ * The K smallest of every query row's LDS keys (ordered distance << 32 | row) moved to their front, in any order, and the
+ * threshold set to the largest distance kept (+inf for fewer than K keys).  A wavefront takes a query at a time, four keys
+ * a lane: the K-th distance by bisection on ballots, then the rows among equal distances.  Called by the whole workgroup.
+ * A bitonic sort of all
+ * kKnnQ x kKnnCap slots took about 30 us: 185 against 107 us for 15,000 rows of 32 against 565, K = 16.
  */
 __device__ void knn_compact(unsigned long long* key, int* cnt, float* tau, int K)
 {
   __syncthreads();
-  for (int t = threadIdx.x; t < kKnnQ * kKnnCap; t += blockDim.x)
-    if ((t % kKnnCap) >= cnt[t / kKnnCap]) key[t] = ~0ULL;
-  for (int size = 2; size <= kKnnCap; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      __syncthreads();
-      for (int t = threadIdx.x; t < kKnnQ * kKnnCap / 2; t += blockDim.x) {
-        const int q = t / (kKnnCap / 2), h = t % (kKnnCap / 2);
-        const int lo = ((h & ~(stride - 1)) << 1) | (h & (stride - 1)), hi = lo | stride;
-        const bool up = (lo & size) == 0;
-        unsigned long long* s = key + q * kKnnCap;
-        const unsigned long long x = s[lo], y = s[hi];
-        if ((x > y) == up) {
-          s[lo] = y;
-          s[hi] = x;
-        }
-      }
+  const int lane = threadIdx.x & 63;
+  for (int q = threadIdx.x >> 6; q < kKnnQ; q += blockDim.x >> 6) {
+    unsigned long long* k = key + q * kKnnCap;
+    const int c           = min(cnt[q], kKnnCap);
+    if (c < K) {  // uniform over the wavefront
+      if (lane == 0) cnt[q] = c;
+      continue;
     }
-  __syncthreads();
-  if (threadIdx.x < kKnnQ) {
-    const int q = threadIdx.x, c = min(cnt[q], K);
-    cnt[q]      = c;
-    tau[q]      = c >= K ? knn_unord(static_cast<unsigned>(key[q * kKnnCap + K - 1] >> 32)) : INFINITY;
+    unsigned hi[4], lo[4];
+    bool valid[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      valid[j]                   = lane + 64 * j < c;
+      const unsigned long long e = k[lane + 64 * j];
+      hi[j]                      = static_cast<unsigned>(e >> 32);
+      lo[j]                      = static_cast<unsigned>(e);
+    }
+    const unsigned T = kth_smallest(hi, valid, K);
+    bool tie[4];
+    int below = 0, ties = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      below += __popcll(__ballot(valid[j] && hi[j] < T));
+      tie[j] = valid[j] && hi[j] == T;
+      ties += __popcll(__ballot(tie[j]));
+    }
+    unsigned row = ~0u;  // equal distances are kept up to this row
+    if (below + ties > K) row = kth_smallest(lo, tie, K - below);
+    int at = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {  // every key was read above
+      const bool keep               = valid[j] && (hi[j] < T || (tie[j] && lo[j] <= row));
+      const unsigned long long mask = __ballot(keep);
+      if (keep)
+        k[at + __popcll(mask & ((1ULL << lane) - 1ULL))] = (static_cast<unsigned long long>(hi[j]) << 32) | lo[j];
+      at += __popcll(mask);
+    }
+    if (lane == 0) {
+      cnt[q] = at;
+      tau[q] = knn_unord(T);
+    }
   }
   __syncthreads();
 }
@@ -520,18 +560,24 @@ __device__ void knn_compact(unsigned long long* key, int* cnt, float* tau, int K
 /**
  * The K nearest database rows X [n, d] of each query row Q [m, d] by squared L2 distance
  * |q|^2 + |x|^2 - 2 q.x (fp32; the dot products by MFMA, knn_op: fp16 products are exact in fp32 and
- * accumulated in fp32), ties by row.  A workgroup owns 64 query rows and scans every database row,
- * 128 per step: wave w computes rows [32 w, 32 w + 32) of the step against the 64 queries as 4 x 2
- * MFMA tiles (lane l holds rows 4 (l / 16) + r of a 16-row tile for query l % 16), the fragments of 8 k steps
- * loaded together before their MFMAs.  A distance at or
- * below its query's threshold is appended to the query's LDS keys; when a query holds more than
- * kKnnCap - kKnnRows keys after a step, knn_compact keeps the K smallest and lowers the thresholds, so
- * a step's appends always fit.  out_d / out_i [m, K], sorted; -1 / +inf past the n rows.
+ * accumulated in fp32), ties by row.  A workgroup owns 64 query rows and scans every database row, kKnnRows per step:
+ * wave w computes rows [32 w, 32 w + 32) of the step against the 64 queries as 4 x 2 MFMA tiles (lane l holds rows
+ * 4 (l / 16) + r of a 16-row tile for query l % 16).  With NK (d is NK whole k steps, at most
+ * kKnnHold) the queries' fragments stay in registers for the whole scan, and a step's row fragments are loaded during the
+ * step before; otherwise (NK = 0) both are loaded per kKnnChunk k steps, together before their MFMAs.
+ * A distance at or below its query's threshold is appended to the query's LDS keys.  When one finds them full, or a
+ * query holds more than kKnnCap - kKnnMaxK keys after a step, knn_compact keeps the K smallest and lowers the
+ * thresholds, and what found no room is tried again.  out_d / out_i [m, K], sorted; -1 / +inf past the n rows.
+ *
+ * The keys fill the LDS, so one workgroup runs per CU; its eight wavefronts (two a SIMD) hide the loads.  Measured with
+ * four wavefronts that loaded the queries anew in every step and sorted to compact, then now: 150k x 128 fp16 rows,
+ * K = 65: 111 -> 38 ms; 15,000 fp32 rows against 565 of 32, K = 16: 368 -> 107 us.
  */
-template <typename T, bool FULL>
-__global__ __launch_bounds__(256) void knn_kernel(const T* __restrict__ Q, const float* __restrict__ qn, int64_t m,
-                                                  const T* __restrict__ X, const float* __restrict__ xn, int64_t n,
-                                                  int d, int K, float* __restrict__ out_d, int* __restrict__ out_i)
+template <typename T, bool FULL, int NK>
+__global__ __launch_bounds__(64 * kKnnWaves) void knn_kernel(const T* __restrict__ Q, const float* __restrict__ qn,
+                                                             int64_t m, const T* __restrict__ X,
+                                                             const float* __restrict__ xn, int64_t n, int d, int K,
+                                                             float* __restrict__ out_d, int* __restrict__ out_i)
 {
   using op = knn_op<T>;
   __shared__ unsigned long long key[kKnnQ * kKnnCap];
@@ -545,10 +591,43 @@ __global__ __launch_bounds__(256) void knn_kernel(const T* __restrict__ Q, const
     tau[tid] = INFINITY;
   }
   float qq[4];
+  const T* qrow[4];  // this lane's query rows (row 0 past the end) and validity
+  bool qok[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int64_t q = q0 + i * 16 + (lane & 15);
-    qq[i]           = q < m ? qn[q] : 0.f;
+    qok[i]          = q < m;
+    qq[i]           = qok[i] ? qn[q] : 0.f;
+    qrow[i]         = Q + (qok[i] ? q : 0) * d;
+  }
+  constexpr bool HOLD = NK > 0;
+  constexpr int kC    = HOLD ? NK : kKnnChunk;
+  typename op::frag a[kC][2], b[kC][4];
+  auto load_q = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < kC; j++) {
+      if (!HOLD && c0 + op::kStep * j >= d) break;  // uniform
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        b[j][i] = op::template load<FULL>(qrow[i], qok[i], d, c0 + op::kStep * j, lane);
+    }
+  };
+  auto load_x = [&](int64_t r0, int c0) {  // of the step at r0: row 0 past the end
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int64_t r = r0 + wid * 32 + t * 16 + (lane & 15);
+      const bool ok   = r < n;
+      const T* row    = X + (ok ? r : 0) * d;
+#pragma unroll
+      for (int j = 0; j < kC; j++) {
+        if (!HOLD && c0 + op::kStep * j >= d) break;
+        a[j][t] = op::template load<FULL>(row, ok, d, c0 + op::kStep * j, lane);
+      }
+    }
+  };
+  if constexpr (HOLD) {
+    load_q(0);
+    load_x(0, 0);
   }
   __syncthreads();
   for (int64_t r0 = 0; r0 < n; r0 += kKnnRows) {
@@ -559,87 +638,101 @@ __global__ __launch_bounds__(256) void knn_kernel(const T* __restrict__ Q, const
 #pragma unroll
       for (int t = 0; t < 2; t++)
         acc[i][t] = float4_t{0.f, 0.f, 0.f, 0.f};
-    // this step's rows and the workgroup's queries: row pointers (row 0 past the end) and validity, the same
-    // for every k step
-    const T* xrow[2];
-    const T* qrow[4];
-    bool xok[2], qok[4];
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int64_t r = rw + t * 16 + (lane & 15);
-      xok[t]          = r < n;
-      xrow[t]         = X + (xok[t] ? r : 0) * d;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int64_t r = q0 + i * 16 + (lane & 15);
-      qok[i]          = r < m;
-      qrow[i]         = Q + (qok[i] ? r : 0) * d;
-    }
-    // k in chunks of kKnnChunk steps: the chunk's fragment loads (unconditional, see knn_h4) are all in flight
-    // before its MFMAs, so a step of rows waits for memory once per chunk (once for d <= 128 fp16, <= 32 fp32)
-    for (int c0 = 0; c0 < d; c0 += op::kStep * kKnnChunk) {
-      typename op::frag a[kKnnChunk][2], b[kKnnChunk][4];
-#pragma unroll
-      for (int j = 0; j < kKnnChunk; j++) {
-        if (c0 + op::kStep * j >= d) break;  // uniform
-        const int k = c0 + op::kStep * j;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-          a[j][t] = op::template load<FULL>(xrow[t], xok[t], d, k, lane);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          b[j][i] = op::template load<FULL>(qrow[i], qok[i], d, k, lane);
-      }
-#pragma unroll
-      for (int j = 0; j < kKnnChunk; j++) {
-        if (c0 + op::kStep * j >= d) break;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int t = 0; t < 2; t++)
-            acc[i][t] = op::mma(a[j][t], b[j][i], acc[i][t]);
-      }
-    }
     float xr[2][4];
 #pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int64_t row = rw + t * 16 + kq + r;
-        const float v     = xn[row < n ? row : 0];  // unconditional load, then a select
-        xr[t][r]          = row < n ? v : 0.f;
+        xr[t][r]          = xn[row < n ? row : 0];  // unconditional load; rows past the end are not taken
+      }
+    for (int c0 = 0; c0 < d; c0 += op::kStep * kC) {
+      if constexpr (!HOLD) {
+        load_q(c0);
+        load_x(r0, c0);
       }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int ql   = i * 16 + (lane & 15);
-      const float th = tau[ql];
+      for (int j = 0; j < kC; j++) {
+        if (!HOLD && c0 + op::kStep * j >= d) break;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+            acc[i][t] = op::mma(a[j][t], b[j][i], acc[i][t]);
+      }
+      if constexpr (HOLD) break;
+    }
+    if constexpr (HOLD) {
+      if (r0 + kKnnRows < n) load_x(r0 + kKnnRows, 0);
+    }
+    // the distances in place; NaN, which is below no threshold, for rows past the end and once appended
+    const float none = __uint_as_float(0x7fc00000u);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          const int64_t row = rw + t * 16 + kq + r;
-          const float dd    = fmaf(-2.f, acc[i][t][r], qq[i] + xr[t][r]);
-          if (row < n && dd <= th) {
-            const int p           = atomicAdd(&cnt[ql], 1);
-            key[ql * kKnnCap + p] = (static_cast<unsigned long long>(knn_ord(dd)) << 32) |
-                                    static_cast<unsigned>(row);
-          }
+          const float dd = fmaf(-2.f, acc[i][t][r], qq[i] + xr[t][r]);
+          acc[i][t][r]   = rw + t * 16 + kq + r < n ? dd : none;
         }
+    for (;;) {  // uniform: until every distance at or below its threshold is in
+      bool left = false;
+      // the keys are made where they are stored: made before this loop, they would take 64 registers
+      int row0 = static_cast<int>(rw) + kq;
+      asm volatile("" : "+v"(row0));
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int ql   = i * 16 + (lane & 15);
+        const float th = tau[ql];
+        float least    = acc[i][0][0];
+#pragma unroll
+        for (int e = 1; e < 8; e++)
+          least = __builtin_fminf(least, acc[i][e >> 2][e & 3]);
+        if (!(least <= th)) continue;  // most steps: none of a lane's eight
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float dd = acc[i][t][r];
+            if (dd <= th) {
+              const int p = atomicAdd(&cnt[ql], 1);
+              if (p < kKnnCap) {
+                key[ql * kKnnCap + p] =
+                  (static_cast<unsigned long long>(knn_ord(dd)) << 32) | static_cast<unsigned>(row0 + t * 16 + r);
+                acc[i][t][r] = none;
+              } else {
+                left = true;
+              }
+            }
+          }
+      }
+      __syncthreads();  // every append of the round is in
+      const int full = tid < kKnnQ && cnt[tid] > kKnnCap - kKnnMaxK;
+      if (!__syncthreads_or(full)) break;  // none full: nothing was left either
+      const int again = __syncthreads_or(left);
+      knn_compact(key, cnt, tau, K);
+      if (!again) break;
     }
-    __syncthreads();  // every append of the step is in
-    const int full = tid < kKnnQ && cnt[tid] > kKnnCap - kKnnRows;
-    if (__syncthreads_or(full)) knn_compact(key, cnt, tau, K);
   }
   knn_compact(key, cnt, tau, K);
-  for (int t = tid; t < kKnnQ * K; t += blockDim.x) {
-    const int ql = t / K, j = t % K;
+  // the kept keys in order: a wavefront takes a query, a key's place is the number of smaller ones
+  for (int ql = wid; ql < kKnnQ; ql += kKnnWaves) {
     const int64_t q = q0 + ql;
-    if (q >= m) continue;
-    const bool ok                = j < cnt[ql];
-    const unsigned long long e   = key[ql * kKnnCap + j];
-    out_i[q * K + j]             = ok ? static_cast<int>(e & 0xffffffffULL) : -1;
-    out_d[q * K + j]             = ok ? knn_unord(static_cast<unsigned>(e >> 32)) : INFINITY;
+    if (q >= m) break;
+    const unsigned long long* k = key + ql * kKnnCap;
+    const int c                 = min(cnt[ql], K);
+    for (int j = lane; j < K; j += 64) {
+      const unsigned long long e = k[j];
+      int place                  = j;  // past the kept keys: the row's end
+      if (j < c) {
+        place = 0;
+        for (int o = 0; o < c; o++)
+          place += k[o] < e ? 1 : 0;
+      }
+      out_i[q * K + place] = j < c ? static_cast<int>(e & 0xffffffffULL) : -1;
+      out_d[q * K + place] = j < c ? knn_unord(static_cast<unsigned>(e >> 32)) : INFINITY;
+    }
   }
 }
 
@@ -1120,16 +1213,32 @@ template <typename T>
 void knn_rows(const T* Q, const float* qn, int64_t m, const T* X, const float* xn, int64_t n, int d, int K,
               float* out_d, int* out_i, hipStream_t s)
 {
-  OCTEX_EXPECTS(K >= 1 && K <= kKnnCap - kKnnRows, "octex: exact neighbors: at most %d per row",
-                kKnnCap - kKnnRows);
+  OCTEX_EXPECTS(K >= 1 && K <= kKnnMaxK, "octex: exact neighbors: at most %d per row", kKnnMaxK);
   OCTEX_EXPECTS(n < (int64_t{1} << 31) && d >= 1, "octex: exact neighbors: at most 2^31 - 1 rows");
   if (m == 0) return;
   const int64_t blocks = (m + kKnnQ - 1) / kKnnQ;
   OCTEX_EXPECTS(blocks < (int64_t{1} << 31), "octex: exact neighbors: too many query rows");
-  if (d % knn_op<T>::kFull == 0)
-    knn_kernel<T, true><<<static_cast<unsigned>(blocks), 256, 0, s>>>(Q, qn, m, X, xn, n, d, K, out_d, out_i);
-  else
-    knn_kernel<T, false><<<static_cast<unsigned>(blocks), 256, 0, s>>>(Q, qn, m, X, xn, n, d, K, out_d, out_i);
+  auto go = [&](auto kernel) {
+    kernel<<<static_cast<unsigned>(blocks), 64 * kKnnWaves, 0, s>>>(Q, qn, m, X, xn, n, d, K, out_d, out_i);
+  };
+  using op           = knn_op<T>;
+  const int nk = d % op::kFull == 0 && d <= op::kStep * kKnnHold ? d / op::kStep : 0;
+  static_assert(op::kStep == op::kFull, "whole k steps");
+  switch (nk) {
+    case 1: go(&knn_kernel<T, true, 1>); break;
+    case 2: go(&knn_kernel<T, true, 2>); break;
+    case 3: go(&knn_kernel<T, true, 3>); break;
+    case 4: go(&knn_kernel<T, true, 4>); break;
+    case 5: go(&knn_kernel<T, true, 5>); break;
+    case 6: go(&knn_kernel<T, true, 6>); break;
+    case 7: go(&knn_kernel<T, true, 7>); break;
+    case 8: go(&knn_kernel<T, true, 8>); break;
+    default:
+      if (d % op::kFull == 0)
+        go(&knn_kernel<T, true, 0>);
+      else
+        go(&knn_kernel<T, false, 0>);
+  }
   OCTEX_HIP(hipGetLastError());
 }
 template void knn_rows<__half>(const __half*, const float*, int64_t, const __half*, const float*, int64_t, int, int,

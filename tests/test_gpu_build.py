@@ -200,6 +200,20 @@ def test_exact_table_matches_oracle(octex, tmp_path, n, d, reverse):
     assert np.array_equal(tg, tc)
 
 
+# The k-NN kernel's row widths: 3, 7 and 8 k steps of 16 (held fragments), 9 and 13 (not held), a partial step; rows of 0
+# and 1, of which hundreds lie at one distance (more ties at the K-th than its key lists hold), and 300 equal rows
+@pytest.mark.parametrize("n,d,top", [(700, 48, 8), (700, 112, 8), (600, 128, 8), (600, 144, 8), (400, 208, 8),
+                                     (600, 100, 8), (900, 34, 2), (300, 32, 1)])
+def test_exact_table_widths_and_ties(octex, tmp_path, n, d, top):
+    g = np.random.default_rng(n + d + top)
+    X = g.integers(0, top, size=(n, d)).astype(np.float32)
+    kw = dict(copies=2, blocks=1, pca_dims=8, list_len=8, table_len=40, log_buckets=8, member_lists=True,
+              reverse_edges=False, seed=1)
+    octex.build(X, tmp_path / "gpu", **kw)
+    O.build(X, str(tmp_path / "cpu"), **kw)
+    assert np.array_equal(_table(tmp_path / "gpu"), _table(tmp_path / "cpu"))
+
+
 @pytest.mark.parametrize("n,blocks", [(900, 1), (1500, 3), (70000, 4), (3000, 8)])
 def test_kmeans_centers_give_the_same_ivf_lists(octex, n, blocks):
     """Every list probed, IVF lists hold the exact l nearest rows whatever the centers are, if every row lies in the
