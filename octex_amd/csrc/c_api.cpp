@@ -431,7 +431,7 @@ extern "C" cuvsError_t octexIndexCopyPlanBuffer(cuvsOctexIndex_t index, const ch
     if (size != nullptr) *size = static_cast<int64_t>(sz);
     if (dst != nullptr && bytes > 0 && src != nullptr) {
       OCTEX_HIP(hipSetDevice(ix.device));
-      OCTEX_HIP(hipStreamSynchronize(ix.stream));
+      ix.drain();
       OCTEX_HIP(hipMemcpy(dst, src, std::min<size_t>(sz, static_cast<size_t>(bytes)), hipMemcpyDefault));
     }
   });
@@ -536,7 +536,7 @@ extern "C" cuvsError_t octexIndexPlaceOnHost(cuvsOctexIndex_t index, int32_t vec
     auto& ix = as_index(*index)->impl();
     std::lock_guard<std::mutex> run(ix.stream_mu);
     OCTEX_HIP(hipSetDevice(ix.device));
-    OCTEX_HIP(hipStreamSynchronize(ix.stream));
+    ix.drain();
     {
       std::lock_guard<std::mutex> lock(ix.mu);
       ix.plans.clear();  // cached plans and their graphs hold the arrays' device addresses

@@ -102,10 +102,14 @@ struct index_impl {
 
   std::mutex mu;  // the plan cache
   std::map<std::string, std::shared_ptr<plan>> plans;
-  // Held by whoever works on `stream`: plan creation (its graph capture), a search's batches, the release of
-  // an evicted plan (whose destructor waits for the stream), introspection and placement changes.  Work of
-  // another thread reaching the stream during a capture would be captured into, or invalidate, that graph.
+  // Held by whoever works on `stream` or with the plans' buffers: plan creation (its graph capture), the enqueueing of a
+  // search's batches (on the caller's stream), the release of an evicted plan (whose destructor waits), introspection and
+  // placement changes.  Work of another thread reaching the stream during a capture would be captured into, or
+  // invalidate, that graph.
   std::mutex stream_mu;
+  hipEvent_t searched = nullptr;  // recorded behind every search on its caller's stream; every search waits for it first
+  /** Waits for the index's stream and its last search (stream_mu held, or no search running). */
+  void drain();
 
   index_impl() = default;
   index_impl(index_impl const&) = delete;

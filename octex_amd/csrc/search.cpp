@@ -30,16 +30,22 @@ index_impl::~index_impl()
     (void)hipStreamSynchronize(stream);
     (void)hipStreamDestroy(stream);
   }
+  if (searched != nullptr) (void)hipEventDestroy(searched);
+}
+
+void index_impl::drain()
+{
+  OCTEX_HIP(hipStreamSynchronize(stream));
+  if (searched != nullptr) OCTEX_HIP(hipEventSynchronize(searched));
 }
 
 plan::~plan()
 {
-  // an evicted plan can be released by a search whose batch is still running on the index's stream: its
-  // graph and buffers go only after that work
+  // an evicted plan can be released while its last batch is still running: its graph and buffers go only after the
+  // index's stream and the last search (which ran after every earlier one)
   if (stream != nullptr) (void)hipStreamSynchronize(stream);
+  if (searched != nullptr) (void)hipEventSynchronize(searched);
   if (graph != nullptr) (void)hipGraphExecDestroy(graph);
-  if (ev_in != nullptr) (void)hipEventDestroy(ev_in);
-  if (ev_out != nullptr) (void)hipEventDestroy(ev_out);
 }
 
 auto make_shape(index_impl const& ix, search_params const& sp, int m, int k) -> plan_shape
@@ -287,12 +293,11 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
 auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>
 {
   auto pl    = std::make_shared<plan>();
-  pl->stream = ix.stream;
-  pl->shape  = make_shape(ix, sp, m, k);
+  pl->stream   = ix.stream;
+  pl->searched = ix.searched;
+  pl->shape    = make_shape(ix, sp, m, k);
   pl->block  = dbuf(carve_buffers(ix, pl->shape, nullptr, nullptr));
   carve_buffers(ix, pl->shape, pl->block.ptr, &pl->buf);
-  OCTEX_HIP(hipEventCreateWithFlags(&pl->ev_in, hipEventDisableTiming));
-  OCTEX_HIP(hipEventCreateWithFlags(&pl->ev_out, hipEventDisableTiming));
   // one eager run on zeroed buffers (code objects loaded, LDS limits set), then the capture of the whole batch.
   // Only the index's own stream is drained first: the index arrays were complete when its load or build returned,
   // and other streams (another index's searches) are not waited for
@@ -371,27 +376,42 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   OCTEX_HIP(hipSetDevice(ix.device));
   const int m = static_cast<int>(std::min<int64_t>(std::max(sp.batch, 1), nq));
   std::unique_lock<std::mutex> run(ix.stream_mu);
+  if (ix.searched == nullptr)
+    OCTEX_HIP(hipEventCreateWithFlags(&ix.searched, hipEventDisableTiming | hipEventDisableSystemFence));
   auto pl = get_plan(ix, sp, m, static_cast<int>(k));  // released before `run` on every path
   auto const& b    = pl->buf;
   const int64_t D  = ix.dim;
-  hipStream_t s    = ix.stream;
   hipStream_t call = raft::resource::get_cuda_stream(res);
-  OCTEX_HIP(hipEventRecord(pl->ev_in, call));
-  OCTEX_HIP(hipStreamWaitEvent(s, pl->ev_in, 0));
-  for (int64_t b0 = 0; b0 < nq; b0 += m) {
-    const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
-    if (!resident) {
-      OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, s));
-      if (n < m) launch_pad_rows(b.qbuf, n, m, static_cast<int>(D), s);
+  // the batches run on the caller's stream itself, after the previous search of the index (its plan buffers may be the
+  // same), which may have run on another stream.  A hop to the index's stream and back, two events and two waits, took
+  // 38 us of a search of one query
+  OCTEX_HIP(hipStreamWaitEvent(call, ix.searched, 0));
+  auto mark = [&] {  // the event the next search, and whoever frees or reads the buffers, waits for
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(call, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
+      OCTEX_HIP(hipEventRecord(ix.searched, call));
+  };
+  try {
+    for (int64_t b0 = 0; b0 < nq; b0 += m) {
+      const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
+      if (!resident) {
+        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, call));
+        if (n < m) launch_pad_rows(b.qbuf, n, m, static_cast<int>(D), call);
+      }
+      run_batch(ix, *pl, call);
+      if (!resident) {
+        OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, call));
+        OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, call));
+      }
     }
-    run_batch(ix, *pl, s);
-    if (!resident) {
-      OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, s));
-      OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, s));
+  } catch (...) {
+    try {
+      mark();
+    } catch (...) {
     }
+    throw;
   }
-  OCTEX_HIP(hipEventRecord(pl->ev_out, s));
-  OCTEX_HIP(hipStreamWaitEvent(call, pl->ev_out, 0));
+  mark();
   pl.reset();  // an evicted plan goes here, with the stream lock held
   run.unlock();
   if (host_out) OCTEX_HIP(hipStreamSynchronize(call));
@@ -409,6 +429,7 @@ void profile_batch(index_impl& ix, plan& pl, int reps, std::vector<std::string>&
   hipStream_t s = ix.stream;
   auto const& sh = pl.shape;
   auto const& b  = pl.buf;
+  OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));  // the plan's last search
   const int C = ix.copies, m = sh.m, st = sh.sp.starts;
   auto steps    = batch_stages(ix, sh, b, s);
   std::vector<hipEvent_t> ev(steps.size() + 1);

@@ -81,8 +81,8 @@ struct plan {
   dbuf block;
   batch_buffers buf;
   hipGraphExec_t graph = nullptr;
-  hipEvent_t ev_in = nullptr, ev_out = nullptr;
-  hipStream_t stream = nullptr;  // the index's stream, where every batch of the plan runs
+  hipStream_t stream = nullptr;   // the index's stream, where the plan's first run and capture were
+  hipEvent_t searched = nullptr;  // the index's event after its last search
   plan() = default;
   plan(plan const&) = delete;
   ~plan();

@@ -218,6 +218,26 @@ def test_search_on_a_side_stream(octex, small_index):
     torch.cuda.synchronize()
 
 
+def test_searches_alternating_between_streams(octex, small_index):
+    """Searches enqueued on several streams in turn, without waiting, share one plan's buffers (and replace the plan,
+    with another parameter set in between): each waits for the one before, whatever its stream."""
+    index = octex.load(small_index["path"])
+    Q = torch.from_numpy(small_index["Q"]).cuda()
+    parts = [Q[:200].contiguous(), Q[200:400].contiguous(), Q[100:300].contiguous()]
+    sets = [dict(k=10, **PARAMS), dict(k=5, read=8, starts=32, waves=1)]
+    want = [[index.search(x, **p) for x in parts] for p in sets]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.default_stream()]
+    got = []
+    for r in range(24):
+        j = 1 if r % 8 == 7 else 0
+        with torch.cuda.stream(streams[r % 3]):
+            got.append((j, (r // 3) % 3, index.search(parts[(r // 3) % 3], **sets[j])))
+    torch.cuda.synchronize()
+    for j, i, (D, I) in got:
+        assert torch.equal(I, want[j][i][1]) and torch.equal(D, want[j][i][0])
+
+
 def test_sketch_rank_matches_oracle(octex, small_index):
     index = octex.load(small_index["path"])
     oix = O.Index(small_index["path"])
