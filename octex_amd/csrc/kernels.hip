@@ -1557,6 +1557,7 @@ __host__ __device__ constexpr auto keys_per_thread(int keys, int threads) -> int
 
 constexpr int kRerankThreads = 128;         // rerank_keep_kernel's workgroup: one query
 constexpr int64_t kWideRerank = int64_t{1} << 15;  // R D from which a query takes 256 threads
+constexpr int kFewRerank = 2048;                   // queries up to which each takes twice the threads (launch_rerank_keep)
 constexpr int kHistWindow    = 256;  // the most recent history entries a round skips (earlier ones are reranked again)
 
 /** Slots of the set of a round's history window (hoff entries before it): a power of two at least twice the window,
@@ -2399,8 +2400,12 @@ void launch_rerank_keep(const int* cand, const float* dist, const int* nin, int 
                 "octex: the selected-id history must hold this round's offset and ids");
   // 128 threads a query (16 queries in flight per CU): measured at 100M rows with the history skip, the waves'
   // launches 0.155 / 0.125 ms on 256 threads, 0.141 / 0.096 ms on 128.  Rounds of many long rows (R D >= 2^15: 512
-  // rows of 960 at gist1m) take 256, twice the rows in flight
-  const int nt      = static_cast<int64_t>(R) * D >= kWideRerank ? 256 : kRerankThreads;
+  // rows of 960 at gist1m) take 256, twice the rows in flight.  Twice that while all queries still run at once (8
+  // workgroups of 256 threads, 4 of 512 a CU): a query's chain is then all that counts.  128 / 256 / 512 threads, three
+  // rounds: 16 queries 22.2, 23.0, 22.9 / 17.5, 19.6, 18.5 / 17.9, 21.3, 19.6 us; 1,000 (R 128, D 128) 27.9, 28.0, 26.0 /
+  // 22.5, 24.7, 22.4 / 29.6, 31.7, 27.6 us; 1,000 of R D = 512 x 384 on 256 / 512: 94, 82, 79 / 92, 76, 73 us
+  const bool wide = static_cast<int64_t>(R) * D >= kWideRerank;
+  const int nt    = (wide ? 256 : kRerankThreads) << (m <= (wide ? kFewRerank / 2 : kFewRerank) ? 1 : 0);
   const int hslots  = !fresh && hoff > 0 ? hist_slots(hoff) : 0;
   const size_t smem = rerank_lds_bytes(R, KO, D, nt, hslots);
   const int c       = keys_per_thread(KO + R, nt);
@@ -2412,15 +2417,22 @@ void launch_rerank_keep(const int* cand, const float* dist, const int* nin, int 
                                  nskip);
     };
     auto by_c = [&](auto nt_tag) {
-      constexpr int NT = decltype(nt_tag)::value;
+      constexpr int NT   = decltype(nt_tag)::value;
+      constexpr int kMost = kMaxKeepSort / NT;  // keys a thread at most
       switch (c) {
         case 1: go(&rerank_keep_kernel<LX, NT, 1>); break;
         case 2: go(&rerank_keep_kernel<LX, NT, 2>); break;
-        case 4: go(&rerank_keep_kernel<LX, NT, 4>); break;
-        default: go(&rerank_keep_kernel<LX, NT, 8>); break;
+        case 4:
+          if constexpr (kMost >= 4) go(&rerank_keep_kernel<LX, NT, 4>);
+          break;
+        default:
+          if constexpr (kMost >= 8) go(&rerank_keep_kernel<LX, NT, 8>);
+          break;
       }
     };
-    if (nt == 256)
+    if (nt == 512)
+      by_c(std::integral_constant<int, 512>{});
+    else if (nt == 256)
       by_c(std::integral_constant<int, 256>{});
     else
       by_c(std::integral_constant<int, kRerankThreads>{});

@@ -569,6 +569,28 @@ def test_gather_entry_and_lane_splits(L, S, table_len, nst, lens):
         check_gather(rix, segl, qs, cand, dist, nout, rows=False)
 
 
+@pytest.mark.parametrize("R,KO", [(24, 40), (512, 64)])
+def test_rerank_keep_thread_counts_agree(L, ix, dix, small_index, R, KO):
+    """A launch's queries choose its threads a query (128, 256 or 512; R D >= 2^15 takes twice as many): 20 queries alone,
+    and repeated to 1,100 and 2,200, give the same kept lists in a fresh and in a merging round."""
+    g = np.random.default_rng(R)
+    m, W = 20, 4096
+    cand, dist, nin = random_candidates(g, m, W, 3000, ix.n)
+    Q = small_index["Q"][:m]
+    out = []
+    for rep in (1, 55, 110):
+        n = m * rep
+        dc, dd, dn, dQ = (dev(np.tile(a, (rep,) + (1,) * (a.ndim - 1))) for a in (cand, dist, nin, Q))
+        dsi = torch.full((n, KO), -1, dtype=torch.int64, device="cuda")
+        dsd = torch.full((n, KO), float("inf"), device="cuda")
+        for fresh, d in ((1, dd), (0, dd.flip(1).contiguous())):
+            L.call("octexStageRerankKeep", P(dc), P(d), P(dn), i32(n), i32(W), P(dix["vectors"]), i32(ix.dim), P(dQ),
+                   i32(R), i32(KO), P(dsi), P(dsd), i32(fresh), None)
+        out.append((host(dsi).reshape(rep, m, KO), host(dsd).reshape(rep, m, KO)))
+    for si, sd in out[1:]:
+        assert (si == out[0][0]).all() and (sd == out[0][1]).all()
+
+
 # ---------------------------------------------------------------- the rerank's history of selected ids
 
 
