@@ -591,6 +591,13 @@ def test_rerank_keep_thread_counts_agree(L, ix, dix, small_index, R, KO):
         assert (si == out[0][0]).all() and (sd == out[0][1]).all()
 
 
+@pytest.mark.parametrize("m,K,N", [(70, 8, 264), (64, 72, 40), (129, 192, 512)])
+def test_projection_chunk_edges(L, m, K, N):
+    """The staged projection's edges: less than a chunk of 64 columns, one and a part, whole chunks; outputs and queries
+    past a tile."""
+    test_projection_within_one_ulp(L, m, K, N)
+
+
 # ---------------------------------------------------------------- the rerank's history of selected ids
 
 
