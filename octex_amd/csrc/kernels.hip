@@ -27,24 +27,6 @@ constexpr uint64_t kEmpty  = ~0ULL;
 
 // ------------------------------------------------------------------ query preparation
 
-__global__ void center_kernel(const float* __restrict__ q, const float* __restrict__ mu,
-                              int64_t total, int D, float* __restrict__ qc, __half* __restrict__ qh)
-{
-  int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  float v = q[t] - mu[t % D];
-  qc[t]   = v;
-  qh[t]   = __float2half(v);
-}
-
-__global__ void pad_rows_kernel(float* __restrict__ q, int from, int m, int D)
-{
-  int64_t t     = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  int64_t total = static_cast<int64_t>(m - from) * D;
-  if (t >= total) return;
-  q[static_cast<int64_t>(from) * D + t] = q[t % D];
-}
-
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef int int4_t __attribute__((ext_vector_type(4)));
@@ -278,34 +260,78 @@ __global__ __launch_bounds__(256) void project_staged_kernel(const __half* __res
 }
 
 /**
- * qs [m, S] = qc [m, D] @ basis [D, S] with one sequential fma chain over d per output (fp32; the
- * reference uses a TF32 GEMM here).  A workgroup takes 16 queries (their rows staged in LDS) by 64
- * sketch coordinates; a thread keeps 4 queries' chains for one coordinate, so every basis load feeds
- * four fmas.
+ * The preparation of a batch in one pass over its queries: rows of q [n, D] (rows n .. m - 1 of the batch take row 0),
+ * copied to qbuf, centred (qc = q - mu) and rounded (qh), and the sketch query qs [m, S] = qc @ basis [D, S], one
+ * sequential fma chain over d per output (fp32; the reference uses a TF32 GEMM here).  Null outputs are left out; a null
+ * mu centres nothing; qbuf may be q.
+ * A workgroup takes 4 QPT queries (their centred rows staged in LDS) by 64 sketch coordinates; a thread keeps QPT
+ * queries' chains for one coordinate, the next kU basis values loading under the fmas of these.  The first column of
+ * workgroups writes the rows.  QPT = 4 reads the basis a quarter as often; 1 keeps the chip busy for few queries, where
+ * the chain's loads are what counts.  Measured as one kernel against centring, sketching and the copy of the queries:
+ * 1,000 queries of 384 (S = 128) 21 us against 6 + 48; 10,000 of 96 19 against 7 + 17 (8 values in flight; 16: 28).
  */
-__global__ __launch_bounds__(256) void sketch_query_kernel(const float* __restrict__ qc,
-                                                           const float* __restrict__ basis, int m, int D,
-                                                           int S, float* __restrict__ qs)
+template <int QPT>
+__global__ __launch_bounds__(256) void prepare_kernel(const float* q, int n, int m, int D, const float* __restrict__ mu,
+                                                      const float* __restrict__ basis, int S, float* qbuf,
+                                                      float* __restrict__ qc, __half* __restrict__ qh,
+                                                      float* __restrict__ qs)
 {
-  extern __shared__ float qrows[];  // [16, D]
-  const int q0 = blockIdx.y * 16, s = blockIdx.x * 64 + (threadIdx.x & 63), ty = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < 16 * D; i += blockDim.x) {
-    const int q = q0 + i / D;
-    qrows[i]     = q < m ? qc[static_cast<int64_t>(q) * D + i % D] : 0.f;
+  constexpr int kRows = 4 * QPT, kU = QPT == 1 ? 32 : 8;  // basis values in flight a thread
+  extern __shared__ float qrows[];  // [kRows, D]
+  const int q0 = blockIdx.y * kRows, col = blockIdx.x * 64 + (threadIdx.x & 63), ty = threadIdx.x >> 6;
+  const bool sketched = qs != nullptr && col < S;
+  float next[kU];
+  auto load = [&](int d0) {
+#pragma unroll
+    for (int j = 0; j < kU; j++)
+      next[j] = basis[static_cast<int64_t>(min(d0 + j, D - 1)) * S + col];
+  };
+  if (sketched) load(0);
+  for (int i = threadIdx.x; i < kRows * D; i += blockDim.x) {
+    const int r = i / D, d = i - r * D, row = q0 + r;
+    float v = 0.f;
+    if (row < m) {
+      const float x = q[static_cast<int64_t>(row < n ? row : 0) * D + d];
+      v             = mu != nullptr ? x - mu[d] : x;
+      if (blockIdx.x == 0) {
+        const int64_t o = static_cast<int64_t>(row) * D + d;
+        if (qbuf != nullptr && (qbuf != q || row >= n)) qbuf[o] = x;
+        if (qc != nullptr) qc[o] = v;
+        if (qh != nullptr) qh[o] = __float2half(v);
+      }
+    }
+    if (qs != nullptr) qrows[i] = v;
   }
   __syncthreads();
-  if (s >= S) return;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int d = 0; d < D; d++) {
-    const float b = basis[static_cast<int64_t>(d) * S + s];
+  if (!sketched) return;
+  float acc[QPT];
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      acc[r] = fmaf(qrows[(4 * ty + r) * D + d], b, acc[r]);
+  for (int r = 0; r < QPT; r++)
+    acc[r] = 0.f;
+  const float* mine = qrows + QPT * ty * D;
+  int d0 = 0;
+  for (; d0 + kU <= D; d0 += kU) {  // uniform
+    float b[kU];
+#pragma unroll
+    for (int j = 0; j < kU; j++)
+      b[j] = next[j];
+    if (d0 + kU < D) load(d0 + kU);
+#pragma unroll
+    for (int j = 0; j < kU; j++)
+#pragma unroll
+      for (int r = 0; r < QPT; r++)
+        acc[r] = fmaf(mine[r * D + d0 + j], b[j], acc[r]);
   }
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int q = q0 + 4 * ty + r;
-    if (q < m) qs[static_cast<int64_t>(q) * S + s] = acc[r];
+  for (int j = 0; j < kU; j++)  // fewer than kU are left
+    if (d0 + j < D)
+#pragma unroll
+      for (int r = 0; r < QPT; r++)
+        acc[r] = fmaf(mine[r * D + d0 + j], next[j], acc[r]);
+#pragma unroll
+  for (int r = 0; r < QPT; r++) {
+    const int row = q0 + QPT * ty + r;
+    if (row < m) qs[static_cast<int64_t>(row) * S + col] = acc[r];
   }
 }
 
@@ -1574,14 +1600,15 @@ __host__ __device__ constexpr auto merge_bytes(int keys) -> size_t
 /**
  * The kept list merged with new keys (search_kernels.cuh:379-415): the keys of the kept list (pb, pd: KO entries,
  * ignored when `fresh`, -1 entries empty) and the ns new (sdv[i], sid[i]) pairs, sorted together in registers,
- * and the first KO distinct keys written back to (pb, pd), padded with (-1, +inf).  Thread t loads elements
+ * and the first KOout distinct keys given to put(place, id, distance), padded with (-1, +inf).  put may write over
+ * (pb, pd).  Thread t loads elements
  * C t .. C t + C - 1 of the concatenation (kept first), so equal keys end next to each other after the sort; a
  * key is kept when it differs from its predecessor, and its place is the number of kept keys before it (a
  * workgroup prefix sum).  ns <= C blockDim - KO.  Every thread of the workgroup calls it.
  */
-template <int C>
-__device__ void merge_keep(long long* pb, float* pd, int KO, bool fresh, const int* sid, const float* sdv, int ns,
-                           long long* ob, float* od, int KOout, merge_view sh)
+template <int C, typename Put>
+__device__ void merge_keep(const long long* pb, const float* pd, int KO, bool fresh, const int* sid, const float* sdv,
+                           int ns, int KOout, merge_view sh, Put const& put)
 {
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   uint64_t k[C];
@@ -1615,16 +1642,13 @@ __device__ void merge_keep(long long* pb, float* pd, int KO, bool fresh, const i
   int at    = block_exclusive_sum(mine, sh.wsum, &total);
 #pragma unroll
   for (int j = 0; j < C; j++) {
-    if (keep[j] && at < KOout) {
-      ob[at] = static_cast<long long>(static_cast<unsigned>(k[j] & 0xffffffffULL));
-      od[at] = __uint_as_float(static_cast<unsigned>(k[j] >> 32));
-    }
+    if (keep[j] && at < KOout)
+      put(at, static_cast<long long>(static_cast<unsigned>(k[j] & 0xffffffffULL)),
+          __uint_as_float(static_cast<unsigned>(k[j] >> 32)));
     at += keep[j] ? 1 : 0;
   }
-  for (int o = min(total, KOout) + t; o < KOout; o += blockDim.x) {
-    ob[o] = -1;
-    od[o] = INFINITY;
-  }
+  for (int o = min(total, KOout) + t; o < KOout; o += blockDim.x)
+    put(o, -1LL, INFINITY);
 }
 
 /**
@@ -1782,8 +1806,12 @@ rerank_keep_kernel(
   if (nskip != nullptr && threadIdx.x == 0) nskip[q] = ns - nr;
   exact_distances<LX>(rr, nr, vectors, D, sq, sd);
   // exact_distances ended with a barrier: the region is free for the merge
-  merge_keep<C>(bi + static_cast<int64_t>(q) * KO, bd + static_cast<int64_t>(q) * KO, KO, fresh, rr, sd, nr,
-                bi + static_cast<int64_t>(q) * KO, bd + static_cast<int64_t>(q) * KO, KO, mv);
+  long long* pb = bi + static_cast<int64_t>(q) * KO;
+  float* pd     = bd + static_cast<int64_t>(q) * KO;
+  merge_keep<C>(pb, pd, KO, fresh, rr, sd, nr, KO, mv, [&](int at, long long id, float d) {
+    pb[at] = id;
+    pd[at] = d;
+  });
 }
 
 /** The KO sketch-nearest candidates merged into the kept list by sketch distance (:471-508). */
@@ -1807,7 +1835,10 @@ __global__ __launch_bounds__(512) void sketch_keep_kernel(const int* __restrict_
   float* pd     = sd + static_cast<int64_t>(q) * KO;
   with_keys_per_thread(KO + ns, blockDim.x, [&](auto c) {
     constexpr int C = decltype(c)::value;
-    merge_keep<C>(pb, pd, KO, fresh, sid, sdv, ns, pb, pd, KO, view(u.merge));
+    merge_keep<C>(pb, pd, KO, fresh, sid, sdv, ns, KO, view(u.merge), [&](int at, long long id, float d) {
+      pb[at] = id;
+      pd[at] = d;
+    });
   });
 }
 
@@ -1920,7 +1951,7 @@ __global__ __launch_bounds__(256) void pick_starts_kernel(const long long* __res
 template <int LX>
 __global__ __launch_bounds__(kKeepThreads) void final_rerank_kernel(
   const long long* __restrict__ si, int KO, int R, const __half* __restrict__ vectors, int D,
-  const float* __restrict__ Q, int k, long long* __restrict__ bi, float* __restrict__ bd)
+  const float* __restrict__ Q, int k, long long* __restrict__ bi, float* __restrict__ bd, result_rows out)
 {
   const int q = blockIdx.x;
   extern __shared__ float sq[];
@@ -1951,8 +1982,15 @@ __global__ __launch_bounds__(kKeepThreads) void final_rerank_kernel(
   exact_distances<LX>(sid, ns, vectors, D, sq, sd);
   with_keys_per_thread(ns, blockDim.x, [&](auto c) {
     constexpr int C = decltype(c)::value < 2 ? decltype(c)::value : 2;
-    merge_keep<C>(nullptr, nullptr, 0, true, sid, sd, ns, bi + static_cast<int64_t>(q) * k,
-                  bd + static_cast<int64_t>(q) * k, k, view(m2));
+    merge_keep<C>(nullptr, nullptr, 0, true, sid, sd, ns, k, view(m2), [&](int place, long long id, float d) {
+      const int64_t o = static_cast<int64_t>(q) * k + place;
+      bi[o]           = id;
+      bd[o]           = d;
+      if (q < out.n) {
+        out.ids[o]  = id;
+        out.dist[o] = d;
+      }
+    });
   });
 }
 
@@ -2160,13 +2198,19 @@ __global__ __launch_bounds__(64) void take_starts_kernel(const long long* __rest
 }
 
 __global__ void take_k_kernel(const long long* __restrict__ si, const float* __restrict__ sd, int KO,
-                              int k, int m, long long* __restrict__ bi, float* __restrict__ bd)
+                              int k, int m, long long* __restrict__ bi, float* __restrict__ bd, result_rows out)
 {
   int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= static_cast<int64_t>(m) * k) return;
   int64_t q = t / k, j = t % k;
-  bi[t]     = si[q * KO + j];
-  bd[t]     = sd[q * KO + j];
+  const long long id = si[q * KO + j];
+  const float d      = sd[q * KO + j];
+  bi[t]              = id;
+  bd[t]              = d;
+  if (q < out.n) {
+    out.ids[t]  = id;
+    out.dist[t] = d;
+  }
 }
 
 /** out[r] = the `words` 32-bit words of src at word offset off[r] (one workgroup per range). */
@@ -2205,20 +2249,26 @@ void with_lx(int D, F&& f)
 }  // namespace
 
 
-void launch_center(const float* q, const float* mu, int64_t m, int D, float* qc, __half* qh,
-                   hipStream_t s)
+void launch_prepare(const float* q, int n, int m, int D, const float* mu, const float* basis, int S, float* qbuf,
+                    float* qc, __half* qh, float* qs, hipStream_t s)
 {
-  const int64_t total = m * D;
-  if (total == 0) return;
-  center_kernel<<<grid_for(total, 256), 256, 0, s>>>(q, mu, total, D, qc, qh);
-  OCTEX_HIP(hipGetLastError());
-}
-
-void launch_pad_rows(float* q, int from, int m, int D, hipStream_t s)
-{
-  const int64_t total = static_cast<int64_t>(m - from) * D;
-  if (total <= 0) return;
-  pad_rows_kernel<<<grid_for(total, 256), 256, 0, s>>>(q, from, m, D);
+  if (m == 0 || D == 0) return;
+  OCTEX_EXPECTS(n >= 1 && n <= m, "octex: a batch holds at least one query");
+  OCTEX_EXPECTS(qs == nullptr || (D >= 1 && 16 * static_cast<int64_t>(D) * sizeof(float) <= 64 * 1024),
+                "octex: the sketch query stages 16 query rows of at most 4096 values in LDS");
+  // one query a thread up to 2,048 queries (512 workgroups of 4), else four
+  const bool few    = m <= 2048;
+  const int rows    = few ? 4 : 16;
+  const size_t smem = qs != nullptr ? static_cast<size_t>(rows) * D * sizeof(float) : 0;
+  dim3 grid(static_cast<unsigned>(qs != nullptr ? (S + 63) / 64 : 1), static_cast<unsigned>((m + rows - 1) / rows));
+  auto go = [&](auto kernel) {
+    allow_lds(reinterpret_cast<const void*>(kernel), smem);
+    kernel<<<grid, 256, smem, s>>>(q, n, m, D, mu, basis, S, qbuf, qc, qh, qs);
+  };
+  if (few)
+    go(&prepare_kernel<1>);
+  else
+    go(&prepare_kernel<4>);
   OCTEX_HIP(hipGetLastError());
 }
 
@@ -2233,17 +2283,6 @@ void launch_project(const __half* qh, const __half* ucatT, const __half* shift, 
     project_staged_kernel<<<grid, 256, 0, s>>>(qh, ucatT, shift, m, K, N, Y);
   else
     project_kernel<<<grid, 256, 0, s>>>(qh, ucatT, shift, m, K, N, Y);
-  OCTEX_HIP(hipGetLastError());
-}
-
-void launch_sketch_query(const float* qc, const float* basis, int m, int D, int S, float* qs,
-                         hipStream_t s)
-{
-  if (static_cast<int64_t>(m) * S == 0) return;
-  OCTEX_EXPECTS(D >= 1 && 16 * static_cast<int64_t>(D) * sizeof(float) <= 64 * 1024,
-                "octex: the sketch query stages 16 query rows of at most 4096 values in LDS");
-  dim3 grid(static_cast<unsigned>((S + 63) / 64), static_cast<unsigned>((m + 15) / 16));
-  sketch_query_kernel<<<grid, 256, 16 * D * sizeof(float), s>>>(qc, basis, m, D, S, qs);
   OCTEX_HIP(hipGetLastError());
 }
 
@@ -2558,24 +2597,24 @@ void launch_pick_starts(const long long* si, int m, int KO, long long* done, int
 }
 
 void launch_final_rerank(const long long* si, int m, int KO, int R, const __half* vectors, int D,
-                         const float* Q, int k, long long* bi, float* bd, hipStream_t s)
+                         const float* Q, int k, long long* bi, float* bd, result_rows out, hipStream_t s)
 {
   if (m == 0) return;
   OCTEX_EXPECTS(R >= k && R <= kMaxRerank && R <= KO,
                 "octex: final_rerank 0 (sketch order) or k <= final_rerank <= 512");
   with_lx(D, [&](auto lx) {
     final_rerank_kernel<decltype(lx)::value>
-      <<<m, kKeepThreads, D * sizeof(float), s>>>(si, KO, R, vectors, D, Q, k, bi, bd);
+      <<<m, kKeepThreads, D * sizeof(float), s>>>(si, KO, R, vectors, D, Q, k, bi, bd, out);
   });
   OCTEX_HIP(hipGetLastError());
 }
 
 void launch_take_k(const long long* si, const float* sd, int m, int KO, int k, long long* bi,
-                   float* bd, hipStream_t s)
+                   float* bd, result_rows out, hipStream_t s)
 {
   const int64_t total = static_cast<int64_t>(m) * k;
   if (total == 0) return;
-  take_k_kernel<<<grid_for(total, 256), 256, 0, s>>>(si, sd, KO, k, m, bi, bd);
+  take_k_kernel<<<grid_for(total, 256), 256, 0, s>>>(si, sd, KO, k, m, bi, bd, out);
   OCTEX_HIP(hipGetLastError());
 }
 

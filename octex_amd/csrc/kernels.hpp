@@ -32,15 +32,15 @@ inline auto hash_log_host(int total, int log_cap) -> int
   return e < kMinLogHash ? kMinLogHash : (e > log_cap ? log_cap : e);
 }
 
-void launch_center(const float* q, const float* mu, int64_t m, int D, float* qc, __half* qh,
-                   hipStream_t s);
-void launch_pad_rows(float* q, int from, int m, int D, hipStream_t s);
+/**
+ * The rows of a batch's queries q [n, D] (rows n .. m - 1 take row 0): copied to qbuf (may be q), qc = q - mu, qh =
+ * fp16(qc), and qs [m, S] = qc @ basis [D, S] (fp32, sequential fma over d).  Null outputs are left out; mu may be null.
+ */
+void launch_prepare(const float* q, int n, int m, int D, const float* mu, const float* basis, int S, float* qbuf,
+                    float* qc, __half* qh, float* qs, hipStream_t s);
 /** Y [m, N] = qh [m, K] @ ucatT [N, K]^T + shift [N] (fp16 MFMA, fp32 accumulate, fp16 out). */
 void launch_project(const __half* qh, const __half* ucatT, const __half* shift, int m, int K, int N,
                     __half* Y, hipStream_t s);
-/** qs [m, S] = qc [m, D] @ basis [D, S] (fp32, sequential fma over d). */
-void launch_sketch_query(const float* qc, const float* basis, int m, int D, int S, float* qs,
-                         hipStream_t s);
 /** E8^b points and hashes of y [n, 8b] * inv_f (the E8 decode of the probe, for tests). */
 void launch_e8(const float* y, int64_t n, int b, float inv_f, float* p, long long* h, hipStream_t s);
 /**
@@ -134,12 +134,18 @@ void launch_sketch_keep(const int* cand, const float* dist, const int* nin, int 
                         long long* si, float* sd, bool fresh, hipStream_t s);
 void launch_pick_starts(const long long* si, int m, int KO, long long* done, int E, int off, int S,
                         int rowlen, int2* seg2, hipStream_t s);
+/** Where a batch's first n results go besides bi / bd: the caller's rows ids / dist [n, k] (n 0: nowhere). */
+struct result_rows {
+  long long* ids = nullptr;
+  float* dist    = nullptr;
+  int n          = 0;
+};
 void launch_final_rerank(const long long* si, int m, int KO, int R, const __half* vectors, int D,
-                         const float* Q, int k, long long* bi, float* bd, hipStream_t s);
+                         const float* Q, int k, long long* bi, float* bd, result_rows out, hipStream_t s);
 /** out [n, words] = the 32-bit words src[off[r], off[r] + words) of every range r (offsets on the device). */
 void launch_copy_ranges(const uint32_t* src, const int64_t* off, int64_t n, int words, uint32_t* out,
                         hipStream_t s);
 void launch_take_k(const long long* si, const float* sd, int m, int KO, int k, long long* bi,
-                   float* bd, hipStream_t s);
+                   float* bd, result_rows out, hipStream_t s);
 
 }  // namespace cuvs::neighbors::octex::detail

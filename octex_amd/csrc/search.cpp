@@ -186,24 +186,27 @@ struct stage {
 };
 
 /**
- * The launches of one batch in order (search.cu:294-518): the first round over all copies with the
- * best KO kept in si / sd, then the waves over the neighbor table, then the best k into bi / bd.  The
+ * The launches of one batch in order (search.cu:294-518): the preparation, the first round over all copies with the
+ * best KO kept in si / sd, then the waves over the neighbor table, then the best k into bi / bd.  The first launch alone
+ * reads the caller's queries and the last alone writes its results (io), so a plan's graph holds those between.  The
  * reference's ablation switches pick other kernels with the same results: balanced_gather = false reads
  * every segment whole by one wavefront (gather_warp_kernel, search_kernels.cuh:687-792), fused_merge =
  * false keeps and picks start points through sorts in global memory (search.cu:213-291).
  */
-auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, hipStream_t s)
-  -> std::vector<stage>
+auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, batch_io const& io,
+                  hipStream_t s) -> std::vector<stage>
 {
   const int D = static_cast<int>(ix.dim), S = ix.sketch_width, C = ix.copies, m = sh.m;
   const bool balanced = sh.sp.balanced_gather, fused = sh.sp.fused_merge, sketch_rank = sh.sp.sketch_rank;
   std::vector<stage> out;
   auto add = [&](const char* n, std::function<void()> f) { out.push_back({n, std::move(f)}); };
-  add("center", [&ix, b, s, m, D] { launch_center(b.qbuf, ix.mean.as<float>(), m, D, b.qc, b.qh, s); });
+  add("prepare", [&ix, b, io, s, m, D, S] {
+    launch_prepare(io.queries != nullptr ? io.queries : b.qbuf, io.n > 0 ? io.n : m, m, D, ix.mean.as<float>(),
+                   ix.basis.as<float>(), S, b.qbuf, b.qc, b.qh, b.qs, s);
+  });
   add("project", [&ix, b, s, m, D, C] {
     launch_project(b.qh, ix.ucatT.as<__half>(), ix.shift.as<__half>(), m, D, C * 8 * ix.blocks, b.Y, s);
   });
-  add("sketch_query", [&ix, b, s, m, D, S] { launch_sketch_query(b.qc, ix.basis.as<float>(), m, D, S, b.qs, s); });
   add("probe", [&ix, b, sh, s, m, C] {
     launch_probe(b.Y, m, C, ix.levels(), ix.blocks, ix.inv_f.as<float>(), ix.offsets.as<int>(),
                  ix.lines.as<bucket_line>(), ix.T1, ix.keys.as<long long>(), ix.mmax, ix.base.as<int>(), ix.list_len,
@@ -281,12 +284,13 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
     keep(sketch_rank ? "sketch_keep_wave" : "rerank_keep_wave", b.cand2[r], b.dist2[r], b.n2[r], sh.W2, sh.R2,
          sh.pool2, wv + 1);
   }
+  const result_rows rows{reinterpret_cast<long long*>(io.neighbors), io.distances, io.neighbors != nullptr ? io.n : 0};
   if (sketch_rank && sh.FR > 0)
-    add("final_rerank", [&ix, b, sh, s, m, D] {
-      launch_final_rerank(b.si, m, sh.KO, sh.FR, ix.vecs(), D, b.qbuf, sh.k, b.bi, b.bd, s);
+    add("final_rerank", [&ix, b, sh, rows, s, m, D] {
+      launch_final_rerank(b.si, m, sh.KO, sh.FR, ix.vecs(), D, b.qbuf, sh.k, b.bi, b.bd, rows, s);
     });
   else
-    add("take_k", [b, sh, s, m] { launch_take_k(b.si, b.sd, m, sh.KO, sh.k, b.bi, b.bd, s); });
+    add("take_k", [b, sh, rows, s, m] { launch_take_k(b.si, b.sd, m, sh.KO, sh.k, b.bi, b.bd, rows, s); });
   return out;
 }
 
@@ -304,13 +308,15 @@ auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sh
   hipStream_t s = ix.stream;
   OCTEX_HIP(hipStreamSynchronize(s));
   OCTEX_HIP(hipMemsetAsync(pl->block.ptr, 0, pl->block.size, s));
-  launch_batch(ix, pl->shape, pl->buf, s);
+  launch_batch(ix, pl->shape, pl->buf, batch_io{}, s);
   OCTEX_HIP(hipStreamSynchronize(s));
   if (sp.use_graph) {
     hipGraph_t graph = nullptr;
     OCTEX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     try {
-      launch_batch(ix, pl->shape, pl->buf, s);
+      auto stages = batch_stages(ix, pl->shape, pl->buf, batch_io{}, s);
+      for (size_t i = 1; i + 1 < stages.size(); i++)
+        stages[i].launch();
     } catch (...) {
       hipGraph_t g2 = nullptr;
       (void)hipStreamEndCapture(s, &g2);
@@ -326,9 +332,9 @@ auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sh
 
 }  // namespace
 
-void launch_batch(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, hipStream_t s)
+void launch_batch(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, batch_io const& io, hipStream_t s)
 {
-  for (auto& st : batch_stages(ix, sh, b, s))
+  for (auto& st : batch_stages(ix, sh, b, io, s))
     st.launch();
 }
 
@@ -354,14 +360,32 @@ auto get_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sha
   return pl;
 }
 
-void run_batch(index_impl const& ix, plan const& pl, hipStream_t s)
+void run_batch(index_impl const& ix, plan const& pl, batch_io const& io, hipStream_t s)
 {
-  if (pl.graph != nullptr) {
-    OCTEX_HIP(hipGraphLaunch(pl.graph, s));
-  } else {
-    launch_batch(ix, pl.shape, pl.buf, s);
+  if (pl.graph == nullptr) {
+    launch_batch(ix, pl.shape, pl.buf, io, s);
+    return;
   }
+  auto stages = batch_stages(ix, pl.shape, pl.buf, io, s);
+  stages.front().launch();
+  OCTEX_HIP(hipGraphLaunch(pl.graph, s));
+  stages.back().launch();
 }
+
+namespace {
+
+/** p lies in the memory of `device`, where the index's kernels read and write it in place. */
+auto on_device(const void* p, int device) -> bool
+{
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();  // not memory that the runtime knows
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
+}  // namespace
 
 void search_impl(raft::resources const& res, search_params const& sp, index const& idx, const float* queries,
                  int64_t nq, int64_t qdim, int64_t* neighbors, float* distances, int64_t k, bool host_out,
@@ -385,7 +409,16 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   // the batches run on the caller's stream itself, after the previous search of the index (its plan buffers may be the
   // same), which may have run on another stream.  A hop to the index's stream and back, two events and two waits, took
   // 38 us of a search of one query
+  if (call != nullptr) {
+    int at = ix.device;
+    OCTEX_HIP(hipStreamGetDevice(call, &at));
+    OCTEX_EXPECTS(at == ix.device, "octex: the search's stream is on device %d, the index on device %d", at, ix.device);
+  }
   OCTEX_HIP(hipStreamWaitEvent(call, ix.searched, 0));
+  // queries and results in the GPU's own memory are read and written in place by the batch's first and last kernel;
+  // others are copied (each copy and its gap about 10 us of a small search)
+  const bool in_place  = !resident && !host_out && on_device(queries, ix.device);
+  const bool out_place = !resident && !host_out && on_device(neighbors, ix.device) && on_device(distances, ix.device);
   auto mark = [&] {  // the event the next search, and whoever frees or reads the buffers, waits for
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(call, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
@@ -394,12 +427,17 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   try {
     for (int64_t b0 = 0; b0 < nq; b0 += m) {
       const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
-      if (!resident) {
-        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, call));
-        if (n < m) launch_pad_rows(b.qbuf, n, m, static_cast<int>(D), call);
+      batch_io io;
+      io.n = n;
+      if (in_place) io.queries = queries + b0 * D;
+      if (out_place) {
+        io.neighbors = neighbors + b0 * k;
+        io.distances = distances + b0 * k;
       }
-      run_batch(ix, *pl, call);
-      if (!resident) {
+      if (!resident && !in_place)
+        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, call));
+      run_batch(ix, *pl, io, call);
+      if (!resident && !out_place) {
         OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, call));
         OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, call));
       }
@@ -431,7 +469,7 @@ void profile_batch(index_impl& ix, plan& pl, int reps, std::vector<std::string>&
   auto const& b  = pl.buf;
   OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));  // the plan's last search
   const int C = ix.copies, m = sh.m, st = sh.sp.starts;
-  auto steps    = batch_stages(ix, sh, b, s);
+  auto steps    = batch_stages(ix, sh, b, batch_io{}, s);
   std::vector<hipEvent_t> ev(steps.size() + 1);
   for (auto& e : ev)
     OCTEX_HIP(hipEventCreate(&e));

@@ -90,10 +90,18 @@ struct plan {
 
 auto plan_key(search_params const& sp, int m, int k) -> std::string;
 auto get_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>;
-/** One batch of the plan on stream s (graph replay, or direct launches without a graph). */
-void run_batch(index_impl const& ix, plan const& pl, hipStream_t s);
+/** Where a batch's n queries come from and its results go: device memory of the index's GPU that the batch's first and
+ * last kernel read and write in place.  Null queries: the plan's qbuf; null results: only bi / bd. */
+struct batch_io {
+  const float* queries = nullptr;
+  int64_t* neighbors   = nullptr;
+  float* distances     = nullptr;
+  int n                = 0;  // 0: the whole batch
+};
+/** One batch of the plan on stream s (its first kernel, the graph's replay and its last kernel; or direct launches). */
+void run_batch(index_impl const& ix, plan const& pl, batch_io const& io, hipStream_t s);
 /** The launches of one batch over the buffers b on stream s, in order (direct launches, no graph). */
-void launch_batch(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, hipStream_t s);
+void launch_batch(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, batch_io const& io, hipStream_t s);
 /** Work counters of one profiled batch (summed over its m queries; per wave for the waves). */
 struct profile_counters {
   int64_t seg_hits = 0, entries1 = 0, distinct1 = 0, reranked1 = 0;

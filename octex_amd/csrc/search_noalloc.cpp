@@ -71,11 +71,12 @@ void search_no_alloc(search_params const& sp, index const& idx, const float* que
     const int64_t D = ix.dim;
     for (int64_t b0 = 0; b0 < nq; b0 += m) {
       const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
-      OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDeviceToDevice, s));
-      if (n < m) launch_pad_rows(b.qbuf, n, m, static_cast<int>(D), s);
-      launch_batch(ix, sh, b, s);
-      OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDeviceToDevice, s));
-      OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDeviceToDevice, s));
+      batch_io io;  // device pointers: read and written in place
+      io.queries   = queries + b0 * D;
+      io.neighbors = neighbors + b0 * k;
+      io.distances = distances + b0 * k;
+      io.n         = n;
+      launch_batch(ix, sh, b, io, s);
     }
   } catch (...) {
     (void)hipSetDevice(cur);

@@ -44,7 +44,9 @@ extern "C" cuvsError_t octexStageCenter(const float* q, const float* mu, int64_t
 {
   return run(stream, [&](hipStream_t s) {
     need(q, "q"), need(mu, "mu"), need(qc, "qc"), need(qh, "qh");
-    launch_center(q, mu, m, D, qc, static_cast<__half*>(qh), s);
+    OCTEX_EXPECTS(m >= 0 && m < (int64_t{1} << 31), "octex: at most 2^31 - 1 queries");
+    launch_prepare(q, static_cast<int>(m), static_cast<int>(m), D, mu, nullptr, 0, nullptr, qc,
+                   static_cast<__half*>(qh), nullptr, s);
   });
 }
 
@@ -64,7 +66,7 @@ extern "C" cuvsError_t octexStageSketchQuery(const float* qc, const float* basis
 {
   return run(stream, [&](hipStream_t s) {
     need(qc, "qc"), need(basis, "basis"), need(qs, "qs");
-    launch_sketch_query(qc, basis, m, D, S, qs, s);
+    launch_prepare(qc, m, m, D, nullptr, basis, S, nullptr, nullptr, nullptr, qs, s);
   });
 }
 
@@ -233,7 +235,7 @@ extern "C" cuvsError_t octexStageFinalRerank(const int64_t* si, int32_t m, int32
   return run(stream, [&](hipStream_t s) {
     need(si, "si"), need(vectors, "vectors"), need(Q, "Q"), need(bi, "bi"), need(bd, "bd");
     launch_final_rerank(reinterpret_cast<const long long*>(si), m, KO, R, static_cast<const __half*>(vectors),
-                        D, Q, k, reinterpret_cast<long long*>(bi), bd, s);
+                        D, Q, k, reinterpret_cast<long long*>(bi), bd, result_rows{}, s);
   });
 }
 
@@ -244,6 +246,6 @@ extern "C" cuvsError_t octexStageTakeK(const int64_t* si, const float* sd, int32
     need(si, "si"), need(sd, "sd"), need(bi, "bi"), need(bd, "bd");
     OCTEX_EXPECTS(k <= KO, "octex: k <= KO");
     launch_take_k(reinterpret_cast<const long long*>(si), sd, m, KO, k, reinterpret_cast<long long*>(bi), bd,
-                  s);
+                  result_rows{}, s);
   });
 }

@@ -106,6 +106,32 @@ def test_batch_split_and_padding(octex, small_index):
     assert np.array_equal(I1, I2) and np.array_equal(D1, D2)
 
 
+@pytest.mark.parametrize("batch,use_graph", [(37, True), (1000, True), (37, False)])
+@pytest.mark.parametrize("sketch_rank", [False, True])
+def test_results_written_in_place(octex, small_index, batch, use_graph, sketch_rank):
+    """Device queries are read and their results written in place by a batch's first and last kernel, the last batch's
+    only as far as it has queries: rows of larger tensors, through the C ABI, with nothing around them touched."""
+    import ctypes as ct
+
+    from octex_amd import _lib
+    from octex_amd.index import search_params
+
+    index = octex.load(small_index["path"])
+    Q = small_index["Q"][:100]
+    p = dict(PARAMS, batch=batch, use_graph=use_graph, sketch_rank=sketch_rank, final_rerank=32)
+    D1, I1 = index.search(Q, k=10, **p)
+    m = len(Q)
+    q = torch.full((m + 2, Q.shape[1]), float("nan"), device="cuda")
+    q[1:-1] = torch.from_numpy(Q).cuda()
+    I = torch.full((m + 2, 10), -9, dtype=torch.int64, device="cuda")
+    D = torch.full((m + 2, 10), -9.0, device="cuda")
+    res, sp = _lib.Resources(stream=0), search_params(**p)
+    t = [_lib.Dl(x[1:-1]) for x in (q, I, D)]
+    _lib.call("cuvsOctexSearch", res.h, ct.byref(sp), index._handle, *(x.ptr for x in t))
+    assert np.array_equal(I[1:-1].cpu().numpy(), I1) and np.array_equal(D[1:-1].cpu().numpy(), D1)
+    assert (I[[0, -1]] == -9).all() and (D[[0, -1]] == -9).all()
+
+
 def test_graph_equals_direct_launches(octex, small_index):
     index = octex.load(small_index["path"])
     Q = small_index["Q"]

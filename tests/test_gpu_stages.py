@@ -598,6 +598,19 @@ def test_projection_chunk_edges(L, m, K, N):
     test_projection_within_one_ulp(L, m, K, N)
 
 
+@pytest.mark.parametrize("m,D,S", [(1, 2, 16), (5, 34, 48), (70, 384, 128), (2049, 40, 96), (2100, 96, 64)])
+def test_sketch_query_shapes(L, m, D, S):
+    """The preparation's sketch on one query a thread (up to 2,048 queries) and four: whole and partial groups of basis
+    values (32 and 8), within half an ulp plus the fp32 chain's bound D 2^-24 sum |terms| of the fp64 product."""
+    g = np.random.default_rng(m + D + S)
+    qc, basis = g.standard_normal((m, D)).astype(np.float32), g.standard_normal((D, S)).astype(np.float32)
+    dq, db = dev(qc), dev(basis)
+    qs = torch.full((m, S), 7.0, device="cuda")
+    L.call("octexStageSketchQuery", P(dq), P(db), i32(m), i32(D), i32(S), P(qs), None)
+    a, b = qc.astype(np.float64), basis.astype(np.float64)
+    assert (np.abs(host(qs) - a @ b) <= (D + 1) * 2.0**-24 * (np.abs(a) @ np.abs(b))).all()
+
+
 # ---------------------------------------------------------------- the rerank's history of selected ids
 
 
