@@ -227,6 +227,26 @@ def test_probe_level_and_bucket_shapes(L, tmp_path, blocks, spacings, log_bucket
     assert hit.mean() > 0.3 and (len(spacings) == 1 or len(np.unique(levels[hit])) > 1)  # hits at several levels
 
 
+@pytest.mark.parametrize("blocks,spacings", [(2, [1.5, 2.0, 2.5, 3.2, 4.0, 5.0, 6.5]), (4, [2.5]), (5, [4.0, 8.0]),
+                                             (1, [1.0 + 0.5 * j for j in range(11)])])
+@pytest.mark.parametrize("stage", PROBES)
+def test_probe_few_and_many_items(L, tmp_path, blocks, spacings, stage):
+    """The probe of few items (a lane a level) and of more than 65,536 (a lane an item) against the oracle: one level, two,
+    up to a group's eight, and more."""
+    X, _ = clustered(n=1500, m=10, d=48, clusters=8, seed=12)
+    path = str(tmp_path / "probe")
+    O.build(X, path, copies=6, blocks=blocks, pca_dims=48, spacings=spacings, list_len=8, table_len=0, log_buckets=5,
+            min_cell=2, member_lists=True, seed=4)
+    pix = O.Index(path)
+    pdix = dict(inv_f=dev(pix.inv_f), offsets=dev(pix.offsets), keys=dev(pix.keys), base=dev(pix.base))
+    Y = queries_Y(pix, X[:200], extra_random=57)
+    ref = O.probe(pix, Y, read=pix.list_len)
+    assert np.array_equal(host(run_probe(L, pix, pdix, Y, pix.list_len, stage)), ref)
+    rep = 65536 // (len(Y) * 6) + 1
+    seg = host(run_probe(L, pix, pdix, np.tile(Y, (rep, 1)), pix.list_len, stage))
+    assert np.array_equal(seg, np.tile(ref, (rep, 1, 1)))
+
+
 def gather_gpu(L, ix, dix, seg, qs, rows, W=4096):
     m, nseg = seg.shape[0], seg.shape[1]
     cand = torch.full((m, W), -5, dtype=torch.int32, device="cuda")
