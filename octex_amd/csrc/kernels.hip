@@ -1571,6 +1571,94 @@ __device__ __forceinline__ void exact_distances(const int* sid, int ns, const __
 
 // ------------------------------------------------------------------ kept-list merges (search_kernels.cuh:345-508)
 
+/**
+ * A set of ids in LDS, in nb buckets of four slots (nb a power of two): an id lives in its home bucket (a
+ * multiplicative hash) or, when that is full, in the next buckets.  A lookup reads a whole bucket with one 16-byte
+ * load.  The set is sized per launch to at least twice the ids it takes (at most kPickHash slots).
+ */
+struct id_buckets {
+  static constexpr int kSlots = 4;
+  int4* b;
+  int nb;
+
+  [[nodiscard]] __device__ unsigned home(long long v) const
+  {
+    return ((static_cast<unsigned>(v) * kIdHash) >> 7) & static_cast<unsigned>(nb - 1);
+  }
+  __device__ void clear() const
+  {
+    for (int i = threadIdx.x; i < nb; i += blockDim.x)
+      b[i] = make_int4(-1, -1, -1, -1);
+  }
+  __device__ void insert(int v) const
+  {
+    for (unsigned h = home(v), p = 0; p < static_cast<unsigned>(nb); p++, h = (h + 1) & (nb - 1)) {
+      int* slot = reinterpret_cast<int*>(&b[h]);
+      for (int j = 0; j < kSlots; j++) {
+        const int prev = atomicCAS(&slot[j], -1, v);
+        if (prev == -1 || prev == v) return;
+      }
+    }
+  }
+  [[nodiscard]] __device__ bool contains(int v) const
+  {
+    for (unsigned h = home(v), p = 0; p < static_cast<unsigned>(nb); p++, h = (h + 1) & (nb - 1)) {
+      const int4 w = b[h];
+      if (w.x == v || w.y == v || w.z == v || w.w == v) return true;
+      if (w.w == -1) return false;  // a bucket with a free slot ends the run
+    }
+    return false;
+  }
+};
+
+/** Buckets of pick_starts_kernel's set for `off` expanded ids: at least 2 off slots, at most kPickHash. */
+__host__ __device__ constexpr auto pick_buckets(int off) -> int
+{
+  int nb = 4;
+  while (nb * id_buckets::kSlots < 2 * off && nb * id_buckets::kSlots < kPickHash)
+    nb <<= 1;
+  return nb;
+}
+
+/** Buckets of the LDS set of expanded ids beside a kept-list kernel's own LDS. */
+__host__ __device__ constexpr auto next_set_buckets(next_starts const& next) -> int
+{
+  return next.seg2 != nullptr && next.off > 0 ? pick_buckets(next.off) : 0;
+}
+
+/**
+ * The ids that earlier waves expanded (at most kMaxFusedSeen of them, next.off), for a kept-list kernel that also takes the
+ * next wave's start points: each thread's ids are loaded as the kernel starts, the LDS set is cleared, and after a barrier
+ * filled; NT threads.
+ */
+template <int NT>
+struct seen_ids {
+  static constexpr int kPer = (kMaxFusedSeen + NT - 1) / NT;
+  int v[kPer];
+  id_buckets set{};
+
+  __device__ void start(next_starts const& next, int4* lds)
+  {
+    if (next.seg2 == nullptr || next.off == 0) return;  // uniform
+    set                   = {lds, pick_buckets(next.off)};
+    const long long* done = next.done + static_cast<int64_t>(blockIdx.x) * next.E;
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+      const int i       = static_cast<int>(threadIdx.x) + e * NT;
+      const long long d = done[i < next.off ? i : 0];
+      v[e]              = i < next.off ? static_cast<int>(d) : -1;
+    }
+    set.clear();
+  }
+  __device__ void fill(next_starts const& next) const
+  {
+    if (next.seg2 == nullptr || next.off == 0) return;
+#pragma unroll
+    for (int e = 0; e < kPer; e++)
+      if (v[e] >= 0) set.insert(v[e]);
+  }
+};
+
 /** A (distance, id) pair as one 64-bit key ordered by (distance bits, id): distances are non-negative. */
 __device__ __forceinline__ uint64_t dist_key(float d, long long id)
 {
@@ -1672,7 +1760,8 @@ __host__ __device__ constexpr auto merge_bytes(int keys) -> size_t
  */
 template <int C, typename Put>
 __device__ void merge_keep(const long long* pb, const float* pd, int KO, bool fresh, const int* sid, const float* sdv,
-                           int ns, int KOout, merge_view sh, Put const& put)
+                           int ns, int KOout, merge_view sh, Put const& put, next_starts const& next = {},
+                           id_buckets seen = {})
 {
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   uint64_t k[C];
@@ -1702,8 +1791,9 @@ __device__ void merge_keep(const long long* pb, const float* pd, int KO, bool fr
     keep[j] = k[j] != kEmpty && k[j] != (j == 0 ? prev : k[j - 1]);
     mine += keep[j] ? 1 : 0;
   }
-  int total = 0;
-  int at    = block_exclusive_sum(mine, sh.wsum, &total);
+  int total       = 0;
+  const int first = block_exclusive_sum(mine, sh.wsum, &total);
+  int at          = first;
 #pragma unroll
   for (int j = 0; j < C; j++) {
     if (keep[j] && at < KOout)
@@ -1713,6 +1803,32 @@ __device__ void merge_keep(const long long* pb, const float* pd, int KO, bool fr
   }
   for (int o = min(total, KOout) + t; o < KOout; o += blockDim.x)
     put(o, -1LL, INFINITY);
+  if (next.seg2 == nullptr) return;
+  // the next wave's start points, as pick_starts_kernel takes them: the first next.S kept entries that are not in `seen`
+  long long* done = next.done + static_cast<int64_t>(blockIdx.x) * next.E + next.off;
+  int2* seg2      = next.seg2 + static_cast<int64_t>(blockIdx.x) * next.S;
+  bool take[C];
+  int place = first, taken = 0;
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    take[j] = keep[j] && place < KOout && (next.off == 0 || !seen.contains(static_cast<int>(k[j] & 0xffffffffULL)));
+    place += keep[j] ? 1 : 0;
+    taken += take[j] ? 1 : 0;
+  }
+  int o = block_exclusive_sum(taken, sh.wsum, &total);
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    if (take[j] && o < next.S) {
+      const int id = static_cast<int>(k[j] & 0xffffffffULL);
+      done[o]      = id;
+      seg2[o]      = make_int2(id, next.rowlen);
+    }
+    o += take[j] ? 1 : 0;
+  }
+  for (int i = min(total, next.S) + t; i < next.S; i += blockDim.x) {
+    done[i] = -1;
+    seg2[i] = make_int2(0, 0);
+  }
 }
 
 /**
@@ -1796,7 +1912,13 @@ __device__ __forceinline__ int hist_slot(int* hs, int slots, int v, bool insert)
  * becomes the KO smallest distinct keys of every key merged so far, so an id an earlier round reranked has its exact key
  * either in the kept list already (merging it again changes nothing) or above all KO kept keys (it cannot enter):
  * dropping it leaves the merge's result unchanged.  It is neither read nor merged; nskip [m] (when not null) gets the
- * count.  The window's ids are loaded as the kernel starts and their set (hslots slots, at least twice the window)
+ * count.
+ *
+ * With next.seg2 the next wave's start points are taken from the merged list (next_starts), with k > 0 (the batch's last
+ * round) its first k go to ki / kd and `out`: launches of their own took 4 to 20 us each, here at most 10 (measured, 16
+ * queries at the defaults 117 -> 111 us, 10,000 at the deep point 1649 -> 1634).  sketch_keep_kernel does not: its 512
+ * threads lost more (227 -> 264 us a wave of 10,000) than the launches cost.
+  The window's ids are loaded as the kernel starts and their set (hslots slots, at least twice the window)
  * cleared, so neither waits after the selection.
  */
 // Eight waves a SIMD: the selection's 64-bit tie bounds took the kernel to about 100 SGPRs, which allow seven (the
@@ -1808,13 +1930,16 @@ rerank_keep_kernel(
   const int* __restrict__ cand, const float* __restrict__ dist, const int* __restrict__ nin, int W,
   const __half* __restrict__ vectors, int D, const float* __restrict__ Q, int R, int KO,
   long long* __restrict__ bi, float* __restrict__ bd, bool fresh, int* __restrict__ hist, int H, int hoff, bool hstore,
-  int hslots, int* __restrict__ nskip)
+  int hslots, int* __restrict__ nskip, next_starts next, result_rows out, long long* __restrict__ ki,
+  float* __restrict__ kd, int k)
 {
   const int q = blockIdx.x;
-  extern __shared__ uint64_t rk_lds[];
+  extern __shared__ int4 rk_lds[];
   __shared__ int nfresh;  // selected ids no earlier round reranked
   const size_t region = rerank_region_bytes(R, KO, NT);
-  auto* base          = reinterpret_cast<unsigned char*>(rk_lds);
+  seen_ids<NT> seen;
+  seen.start(next, rk_lds);
+  auto* base = reinterpret_cast<unsigned char*>(rk_lds + next_set_buckets(next));
   auto& sel           = *reinterpret_cast<bin_select_lds*>(base);
   const int keys      = keys_per_thread(KO + R, NT) * NT;
   merge_view mv{reinterpret_cast<uint64_t*>(base), reinterpret_cast<int*>(base + static_cast<size_t>(keys) * 8 + 16 * 8),
@@ -1849,6 +1974,7 @@ rerank_keep_kernel(
   if (hstore)
     for (int t = threadIdx.x; t < R; t += NT)
       hrow[hoff + t] = t < ns ? sid[t] : -1;
+  seen.fill(next);
   int nr        = ns;  // the selected ids reranked here
   const int* rr = sid;
   if (filter) {
@@ -1872,10 +1998,22 @@ rerank_keep_kernel(
   // exact_distances ended with a barrier: the region is free for the merge
   long long* pb = bi + static_cast<int64_t>(q) * KO;
   float* pd     = bd + static_cast<int64_t>(q) * KO;
-  merge_keep<C>(pb, pd, KO, fresh, rr, sd, nr, KO, mv, [&](int at, long long id, float d) {
-    pb[at] = id;
-    pd[at] = d;
-  });
+  merge_keep<C>(
+    pb, pd, KO, fresh, rr, sd, nr, KO, mv,
+    [&](int at, long long id, float d) {
+      pb[at] = id;
+      pd[at] = d;
+      if (at < k) {  // the batch's last round: the best k are its results
+        const int64_t o = static_cast<int64_t>(q) * k + at;
+        ki[o]           = id;
+        kd[o]           = d;
+        if (q < out.n) {
+          out.ids[o]  = id;
+          out.dist[o] = d;
+        }
+      }
+    },
+    next, seen.set);
 }
 
 /** The KO sketch-nearest candidates merged into the kept list by sketch distance (:471-508). */
@@ -1904,55 +2042,6 @@ __global__ __launch_bounds__(512) void sketch_keep_kernel(const int* __restrict_
       pd[at] = d;
     });
   });
-}
-
-/**
- * A set of ids in LDS, in nb buckets of four slots (nb a power of two): an id lives in its home bucket (a
- * multiplicative hash) or, when that is full, in the next buckets.  A lookup reads a whole bucket with one 16-byte
- * load.  The set is sized per launch to at least twice the ids it takes (at most kPickHash slots).
- */
-struct id_buckets {
-  static constexpr int kSlots = 4;
-  int4* b;
-  int nb;
-
-  [[nodiscard]] __device__ unsigned home(long long v) const
-  {
-    return ((static_cast<unsigned>(v) * kIdHash) >> 7) & static_cast<unsigned>(nb - 1);
-  }
-  __device__ void clear() const
-  {
-    for (int i = threadIdx.x; i < nb; i += blockDim.x)
-      b[i] = make_int4(-1, -1, -1, -1);
-  }
-  __device__ void insert(int v) const
-  {
-    for (unsigned h = home(v), p = 0; p < static_cast<unsigned>(nb); p++, h = (h + 1) & (nb - 1)) {
-      int* slot = reinterpret_cast<int*>(&b[h]);
-      for (int j = 0; j < kSlots; j++) {
-        const int prev = atomicCAS(&slot[j], -1, v);
-        if (prev == -1 || prev == v) return;
-      }
-    }
-  }
-  [[nodiscard]] __device__ bool contains(int v) const
-  {
-    for (unsigned h = home(v), p = 0; p < static_cast<unsigned>(nb); p++, h = (h + 1) & (nb - 1)) {
-      const int4 w = b[h];
-      if (w.x == v || w.y == v || w.z == v || w.w == v) return true;
-      if (w.w == -1) return false;  // a bucket with a free slot ends the run
-    }
-    return false;
-  }
-};
-
-/** Buckets of pick_starts_kernel's set for `off` expanded ids: at least 2 off slots, at most kPickHash. */
-__host__ __device__ constexpr auto pick_buckets(int off) -> int
-{
-  int nb = 4;
-  while (nb * id_buckets::kSlots < 2 * off && nb * id_buckets::kSlots < kPickHash)
-    nb <<= 1;
-  return nb;
 }
 
 /**
@@ -2607,9 +2696,21 @@ void launch_unfused_pick(const long long* si, int m, int KO, long long* done, in
   OCTEX_HIP(hipGetLastError());
 }
 
+namespace {
+
+void check_next_starts(next_starts const& next, int KO)
+{
+  OCTEX_EXPECTS(next.seg2 == nullptr || (next.done != nullptr && next.S >= 1 && next.S <= KO && next.off >= 0 &&
+                                         next.off <= kMaxFusedSeen && next.off + next.S <= next.E),
+                "octex: a kept-list kernel takes start points after at most %d expanded ids", kMaxFusedSeen);
+}
+
+}  // namespace
+
 void launch_rerank_keep(const int* cand, const float* dist, const int* nin, int m, int W, const __half* vectors, int D,
                         const float* Q, int R, int KO, long long* si, float* sd, bool fresh, int* hist, int H, int hoff,
-                        bool hstore, int* nskip, hipStream_t s)
+                        bool hstore, int* nskip, next_starts const& next, long long* ki, float* kd, int k,
+                        result_rows out, hipStream_t s)
 {
   if (m == 0) return;
   OCTEX_EXPECTS(R >= 1 && R <= kMaxRerank && KO + R <= kMaxKeepSort && KO >= 1,
@@ -2626,14 +2727,16 @@ void launch_rerank_keep(const int* cand, const float* dist, const int* nin, int 
   const bool wide = static_cast<int64_t>(R) * D >= kWideRerank;
   const int nt    = (wide ? 256 : kRerankThreads) << (m <= (wide ? kFewRerank / 2 : kFewRerank) ? 1 : 0);
   const int hslots  = !fresh && hoff > 0 ? hist_slots(hoff) : 0;
-  const size_t smem = rerank_lds_bytes(R, KO, D, nt, hslots);
+  check_next_starts(next, KO);
+  OCTEX_EXPECTS(k >= 0 && k <= KO && (k == 0 || (ki != nullptr && kd != nullptr)), "octex: k <= max(starts, k) results");
+  const size_t smem = static_cast<size_t>(next_set_buckets(next)) * sizeof(int4) + rerank_lds_bytes(R, KO, D, nt, hslots);
   const int c       = keys_per_thread(KO + R, nt);
   with_lx(D, [&](auto lx) {
     constexpr int LX = decltype(lx)::value;
     auto go          = [&](auto kernel) {
       allow_lds(reinterpret_cast<const void*>(kernel), smem);
       kernel<<<m, nt, smem, s>>>(cand, dist, nin, W, vectors, D, Q, R, KO, si, sd, fresh, hist, H, hoff, hstore, hslots,
-                                 nskip);
+                                 nskip, next, out, ki, kd, k);
     };
     auto by_c = [&](auto nt_tag) {
       constexpr int NT   = decltype(nt_tag)::value;

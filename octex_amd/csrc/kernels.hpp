@@ -119,6 +119,21 @@ void launch_unfused_keep(const int* cand, const float* dist, const int* nin, int
  * dsort [m, Ep], kept entries marked fresh by binary search, the first S fresh taken. */
 void launch_unfused_pick(const long long* si, int m, int KO, long long* done, int E, int off, int S, int rowlen,
                          uint64_t* dsort, int Ep, unsigned char* fresh, int2* seg2, hipStream_t s);
+/** Where a batch's first n results go besides bi / bd: the caller's rows ids / dist [n, k] (n 0: nowhere). */
+struct result_rows {
+  long long* ids = nullptr;
+  float* dist    = nullptr;
+  int n          = 0;
+};
+/** Expanded ids up to which the exact rerank takes the next wave's start points itself: its LDS set of them is small. */
+constexpr int kMaxFusedSeen = 256;
+/** The start points of the next wave taken from a merged kept list, as launch_pick_starts takes them: the first S kept
+ * ids not in done[q, 0 .. off), to done[q, off .. off + S) and seg2 [m, S] (id, rowlen).  seg2 null: none. */
+struct next_starts {
+  long long* done = nullptr;  // [m, E]
+  int2* seg2      = nullptr;
+  int E = 0, off = 0, S = 0, rowlen = 0;
+};
 /**
  * Exact rerank of each query's R sketch-nearest candidates (of its nin [m] in cand / dist [m, W]) merged into its kept
  * list si / sd [m, KO] (search_kernels.cuh:421-467).
@@ -126,20 +141,16 @@ void launch_unfused_pick(const long long* si, int m, int KO, long long* done, in
  * with hstore this round's go to hist[q, hoff .. hoff + R).  Unless fresh, the ids of hist[q, 0 .. hoff) are those the
  * earlier rounds reranked into this kept list; those of its last 256 entries, selected again, are neither read nor
  * merged (the kept list of the KO smallest keys comes out the same), and nskip [m] (when not null) gets their count.
+ * next: the next wave's start points.  k > 0: the first k kept also to ki / kd [m, k] and `out`.
  */
 void launch_rerank_keep(const int* cand, const float* dist, const int* nin, int m, int W, const __half* vectors, int D,
                         const float* Q, int R, int KO, long long* si, float* sd, bool fresh, int* hist, int H, int hoff,
-                        bool hstore, int* nskip, hipStream_t s);
+                        bool hstore, int* nskip, next_starts const& next, long long* ki, float* kd, int k,
+                        result_rows out, hipStream_t s);
 void launch_sketch_keep(const int* cand, const float* dist, const int* nin, int m, int W, int KO,
                         long long* si, float* sd, bool fresh, hipStream_t s);
 void launch_pick_starts(const long long* si, int m, int KO, long long* done, int E, int off, int S,
                         int rowlen, int2* seg2, hipStream_t s);
-/** Where a batch's first n results go besides bi / bd: the caller's rows ids / dist [n, k] (n 0: nowhere). */
-struct result_rows {
-  long long* ids = nullptr;
-  float* dist    = nullptr;
-  int n          = 0;
-};
 void launch_final_rerank(const long long* si, int m, int KO, int R, const __half* vectors, int D,
                          const float* Q, int k, long long* bi, float* bd, result_rows out, hipStream_t s);
 /** out [n, words] = the 32-bit words src[off[r], off[r] + words) of every range r (offsets on the device). */

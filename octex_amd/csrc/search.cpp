@@ -179,7 +179,8 @@ auto named_buffer(index_impl const& ix, plan_shape const& sh, batch_buffers cons
 
 namespace {
 
-/** One stage of a batch: its name (as profiled) and its launch. */
+/** One stage of a batch: its name (as profiled) and its launch; none where the kernel of the stage before does its work
+ * too (profiled at no time). */
 struct stage {
   std::string name;
   std::function<void()> launch;
@@ -222,6 +223,11 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
         ix.table_len, ix.n, ix.code(), ix.sketch_pitch, ix.scale.as<float>(), b.qs, S, W, logW, cand, dist, n, s);
     });
   };
+  const result_rows rows{reinterpret_cast<long long*>(io.neighbors), io.distances, io.neighbors != nullptr ? io.n : 0};
+  // wave wv's start points come from the exact rerank of round wv, while earlier waves expanded few ids (its LDS set)
+  auto fused_pick = [&](int wv) {
+    return fused && !sketch_rank && wv < sh.sp.waves && wv * sh.sp.starts <= kMaxFusedSeen;
+  };
   // the kept list merged with a round's candidates: fused (one kernel) or through global-memory sorts.  The fused
   // rerank of round r (0 the first) keeps its selected ids at hist[:, off(r) ..) for the later rounds, which skip them:
   // off(0) = 0, off(r) = rerank + (r - 1) wave_rerank
@@ -230,6 +236,10 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
     const bool fresh = round == 0;
     const int hoff   = round == 0 ? 0 : sh.R1 + (round - 1) * sh.R2;
     const bool store = sh.H > 0 && round < sh.sp.waves;
+    // the next wave's start points (round r's merge is before wave r), and in the last round the results
+    next_starts next;
+    if (fused_pick(round)) next = {b.done, b.seg2, sh.sp.starts * sh.sp.waves, round * sh.sp.starts, sh.sp.starts, ix.table_len};
+    const bool last = round == sh.sp.waves;
     const std::string nm = base_name + unfused;
     const char* name     = nm.c_str();
     if (fused && sketch_rank)
@@ -237,9 +247,10 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
         launch_sketch_keep(cand, dist, n, m, W, sh.KO, b.si, b.sd, fresh, s);
       });
     else if (fused)
-      add(name, [&ix, b, sh, s, m, D, cand, dist, n, W, R, fresh, hoff, store] {
+      add(name, [&ix, b, sh, rows, s, m, D, cand, dist, n, W, R, fresh, hoff, store, next, last] {
         launch_rerank_keep(cand, dist, n, m, W, ix.vecs(), D, b.qbuf, R, sh.KO, b.si, b.sd, fresh,
-                           sh.H > 0 ? b.hist : nullptr, sh.H, sh.H > 0 ? hoff : 0, store, fresh ? nullptr : b.nskip, s);
+                           sh.H > 0 ? b.hist : nullptr, sh.H, sh.H > 0 ? hoff : 0, store, fresh ? nullptr : b.nskip,
+                           next, b.bi, b.bd, last ? sh.k : 0, last ? rows : result_rows{}, s);
       });
     else
       add(name, [&ix, b, sh, s, m, D, cand, dist, n, W, R, pool, fresh, sketch_rank] {
@@ -251,7 +262,10 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
   keep(sketch_rank ? "sketch_keep" : "rerank_keep", b.cand, b.dist, b.nin, sh.W, sh.R1, sh.pool1, 0);
   const int st = sh.sp.starts, nw = sh.sp.waves;
   for (int wv = 0; wv < nw; wv++) {
-    add(("pick_starts" + unfused).c_str(), [&ix, b, sh, s, m, st, nw, wv, fused] {
+    if (fused_pick(wv))
+      add("pick_starts", nullptr);
+    else
+      add(("pick_starts" + unfused).c_str(), [&ix, b, sh, s, m, st, nw, wv, fused] {
       if (fused)
         launch_pick_starts(b.si, m, sh.KO, b.done, st * nw, wv * st, st, ix.table_len, b.seg2, s);
       else
@@ -284,14 +298,24 @@ auto batch_stages(index_impl const& ix, plan_shape const& sh, batch_buffers cons
     keep(sketch_rank ? "sketch_keep_wave" : "rerank_keep_wave", b.cand2[r], b.dist2[r], b.n2[r], sh.W2, sh.R2,
          sh.pool2, wv + 1);
   }
-  const result_rows rows{reinterpret_cast<long long*>(io.neighbors), io.distances, io.neighbors != nullptr ? io.n : 0};
   if (sketch_rank && sh.FR > 0)
     add("final_rerank", [&ix, b, sh, rows, s, m, D] {
       launch_final_rerank(b.si, m, sh.KO, sh.FR, ix.vecs(), D, b.qbuf, sh.k, b.bi, b.bd, rows, s);
     });
-  else
+  else if (sketch_rank || !fused)
     add("take_k", [b, sh, rows, s, m] { launch_take_k(b.si, b.sd, m, sh.KO, sh.k, b.bi, b.bd, rows, s); });
+  else
+    add("take_k", nullptr);
   return out;
+}
+
+/** The launches of a batch, in order. */
+auto batch_launches(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, batch_io const& io, hipStream_t s)
+  -> std::vector<stage>
+{
+  auto all = batch_stages(ix, sh, b, io, s);
+  all.erase(std::remove_if(all.begin(), all.end(), [](stage const& st) { return !st.launch; }), all.end());
+  return all;
 }
 
 auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>
@@ -314,7 +338,7 @@ auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sh
     hipGraph_t graph = nullptr;
     OCTEX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     try {
-      auto stages = batch_stages(ix, pl->shape, pl->buf, batch_io{}, s);
+      auto stages = batch_launches(ix, pl->shape, pl->buf, batch_io{}, s);
       for (size_t i = 1; i + 1 < stages.size(); i++)
         stages[i].launch();
     } catch (...) {
@@ -334,7 +358,7 @@ auto make_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sh
 
 void launch_batch(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, batch_io const& io, hipStream_t s)
 {
-  for (auto& st : batch_stages(ix, sh, b, io, s))
+  for (auto& st : batch_launches(ix, sh, b, io, s))
     st.launch();
 }
 
@@ -366,7 +390,7 @@ void run_batch(index_impl const& ix, plan const& pl, batch_io const& io, hipStre
     launch_batch(ix, pl.shape, pl.buf, io, s);
     return;
   }
-  auto stages = batch_stages(ix, pl.shape, pl.buf, io, s);
+  auto stages = batch_launches(ix, pl.shape, pl.buf, io, s);
   stages.front().launch();
   OCTEX_HIP(hipGraphLaunch(pl.graph, s));
   stages.back().launch();
@@ -484,6 +508,7 @@ void profile_batch(index_impl& ix, plan& pl, int reps, std::vector<std::string>&
     const bool last = r + 1 == reps;
     int wv = -1;
     for (size_t i = 0; i < steps.size(); i++) {
+      if (!steps[i].launch) continue;
       OCTEX_HIP(hipEventRecord(ev[i], s));
       steps[i].launch();
       OCTEX_HIP(hipEventRecord(ev[i + 1], s));
@@ -515,12 +540,11 @@ void profile_batch(index_impl& ix, plan& pl, int reps, std::vector<std::string>&
           cnt.distinct1 += v;
           cnt.reranked1 += std::min(v, sh.sp.sketch_rank ? sh.KO : sh.R1);
         }
-      } else if (nm == "pick_starts") {
+      } else if (nm == "gather_rows") {
         wv++;
         OCTEX_HIP(hipMemcpy(segh.data(), b.seg2, sizeof(int2) * m * st, hipMemcpyDeviceToHost));
         for (int64_t j = 0; j < int64_t{m} * st; j++)
           cnt.starts2[wv] += segh[j].y > 0;
-      } else if (nm == "gather_rows") {
         const int slot = wv % sh.ring;
         OCTEX_HIP(hipMemcpy(n2.data(), b.n2[slot], sizeof(int) * m, hipMemcpyDeviceToHost));
         OCTEX_HIP(hipMemcpy(nk.data(), b.nknown, sizeof(int) * m, hipMemcpyDeviceToHost));

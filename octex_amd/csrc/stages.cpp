@@ -195,7 +195,8 @@ extern "C" cuvsError_t octexStageRerankKeepHistory(const int32_t* cand, const fl
     need(cand, "cand"), need(dist, "dist"), need(nin, "nin"), need(vectors, "vectors"), need(Q, "Q");
     need(si, "si"), need(sd, "sd");
     launch_rerank_keep(cand, dist, nin, m, W, static_cast<const __half*>(vectors), D, Q, R, KO,
-                       reinterpret_cast<long long*>(si), sd, fresh != 0, hist, H, hoff, hstore != 0, nskip, s);
+                       reinterpret_cast<long long*>(si), sd, fresh != 0, hist, H, hoff, hstore != 0, nskip, next_starts{},
+                       nullptr, nullptr, 0, result_rows{}, s);
   });
 }
 

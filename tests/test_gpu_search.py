@@ -244,6 +244,25 @@ def test_search_on_a_side_stream(octex, small_index):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("starts,waves,k", [(128, 4, 10), (100, 3, 100), (16, 6, 1), (256, 2, 20), (20, 1, 50)])
+@pytest.mark.parametrize("sketch_rank", [False, True])
+def test_start_points_of_the_kept_list_kernels(octex, small_index, starts, waves, k, sketch_rank):
+    """Start points taken by the kept-list kernels (up to 256 ids expanded before) and by their own kernel (more: four
+    waves of 128), and the results taken from the last kept list: as the oracle's, and as the sorts in global memory."""
+    index = octex.load(small_index["path"])
+    oix = O.Index(small_index["path"])
+    Q = small_index["Q"][:90]
+    p = dict(read=16, starts=starts, waves=waves, rerank=96, wave_rerank=64, sketch_rank=sketch_rank,
+             final_rerank=max(k, 32))
+    if sketch_rank and p["final_rerank"] > max(starts, k):
+        p["final_rerank"] = k
+    D, I = index.search(Q, k=k, **p)
+    Do, Io, _, _, _ = oracle_given_gpu_projections(index, oix, Q, k, **p)
+    assert_same_results(D, I, Do, Io)
+    Du, Iu = index.search(Q, k=k, fused_merge=False, **p)
+    assert_same_results(D, I, Du, Iu)
+
+
 def test_searches_alternating_between_streams(octex, small_index):
     """Searches enqueued on several streams in turn, without waiting, share one plan's buffers (and replace the plan,
     with another parameter set in between): each waits for the one before, whatever its stream."""
