@@ -189,13 +189,7 @@ void make_projections(std::vector<float> const& vectors, std::vector<double> con
   }
 }
 
-/** The rule of a merged table row (build_table.cuh:157-164): its first kf forward entries, up to kr
- * reverse entries (lowest rank first, then lowest id), then its other forward entries; duplicates,
- * -1 and the row itself dropped; the first kout kept, in that priority order. */
-struct reverse_rule {
-  int kin, kf, ks, kr, kout;
-};
-
+/** The merged rows on the host, where the GPU lacks the memory (merge_on_device): the rows of a 100M-row index beside it. */
 void merge_reverse(std::vector<int32_t> const& fwd, int64_t n, reverse_rule const& rr, std::vector<int32_t>& table,
                    const float* fdist = nullptr)
 {
@@ -478,6 +472,32 @@ void set_table(index_impl& ix, std::vector<int32_t> const& rows, int k)
   ix.table_len = k;
 }
 
+/** set_table with the rows already on the device. */
+void set_device_table(index_impl& ix, dbuf&& rows, int k)
+{
+  std::lock_guard<std::mutex> run(ix.stream_mu);
+  {
+    std::lock_guard<std::mutex> lock(ix.mu);
+    ix.plans.clear();
+  }
+  ix.bytes += static_cast<int64_t>(rows.size) - static_cast<int64_t>(ix.table.size);
+  ix.table     = dbuf();
+  ix.table     = std::move(rows);
+  ix.table_len = k;
+}
+
+/** The forward rows and their merge stay on the GPU while they take at most half of its free memory (OCTEX_MERGE_HOST=1:
+ * they do not; the same rows).  Measured for 250k
+ * rows of 96 forward entries: a search pass and its merge 20 ms, with the merge on 16 host threads 125 ms. */
+auto merge_on_device(int64_t n, reverse_rule const& rr) -> bool
+{
+  const char* host = std::getenv("OCTEX_MERGE_HOST");
+  if (host != nullptr && std::atoi(host) != 0) return false;
+  size_t fr = 0, tot = 0;
+  OCTEX_HIP(hipMemGetInfo(&fr, &tot));
+  return merge_reverse_bytes(n, rr) + static_cast<size_t>(n) * (8 * rr.kin + 4 * rr.kout) <= fr / 2;
+}
+
 void drop_table(index_impl& ix)
 {
   std::lock_guard<std::mutex> run(ix.stream_mu);
@@ -496,7 +516,7 @@ void drop_table(index_impl& ix)
  * clamped at zero (drop_self_kernel, :60-74), then reverse edges merged by the half rule (kf = ks =
  * kr = k / 2) with the kept entries ordered nearest first (merge_rows_kernel, :166-252).
  */
-void exact_table(index_impl& ix, int k, bool reverse_edges, std::vector<int32_t>& table)
+void exact_table(index_impl& ix, int k, bool reverse_edges, std::vector<int32_t>& table, dbuf& dtable)
 {
   const int64_t n = ix.n, d = ix.dim;
   OCTEX_EXPECTS(k >= 1 && k < n, "octex: table_len must be in [1, n)");
@@ -508,15 +528,25 @@ void exact_table(index_impl& ix, int k, bool reverse_edges, std::vector<int32_t>
   row_norms(xd, n, static_cast<int>(d), norms.as<float>(), s);
   const int64_t chunk = std::min<int64_t>(n, int64_t{1} << 18);
   dbuf od(static_cast<size_t>(chunk) * K * sizeof(float)), oi(static_cast<size_t>(chunk) * K * sizeof(int32_t));
-  std::vector<float> hd(static_cast<size_t>(chunk) * K);
-  std::vector<int32_t> hi(static_cast<size_t>(chunk) * K);
-  std::vector<int32_t> fid(static_cast<size_t>(n) * k);
-  std::vector<float> fdist(static_cast<size_t>(n) * k);
+  const int h = std::max(1, k / 2);
+  const reverse_rule rr{k, h, h, h, k};
+  const bool on_device = reverse_edges && merge_on_device(n, rr);
+  dbuf dfid(on_device ? static_cast<size_t>(n) * k * sizeof(int32_t) : 0);
+  dbuf dfdist(on_device ? static_cast<size_t>(n) * k * sizeof(float) : 0);
+  std::vector<float> hd(on_device ? 0 : static_cast<size_t>(chunk) * K);
+  std::vector<int32_t> hi(on_device ? 0 : static_cast<size_t>(chunk) * K);
+  std::vector<int32_t> fid(on_device ? 0 : static_cast<size_t>(n) * k);
+  std::vector<float> fdist(on_device ? 0 : static_cast<size_t>(n) * k);
   const auto t0 = std::chrono::steady_clock::now();
   for (int64_t r0 = 0; r0 < n; r0 += chunk) {
     const int64_t m = std::min(chunk, n - r0);
     knn_rows(xd + r0 * d, norms.as<float>() + r0, m, xd, norms.as<float>(), n, static_cast<int>(d), K, od.as<float>(),
              oi.as<int32_t>(), s);
+    if (on_device) {
+      drop_self(oi.as<int32_t>(), od.as<float>(), r0, m, K, k, dfid.as<int32_t>() + r0 * k, dfdist.as<float>() + r0 * k,
+                s);
+      continue;
+    }
     OCTEX_HIP(hipMemcpyAsync(hd.data(), od.ptr, static_cast<size_t>(m) * K * sizeof(float), hipMemcpyDeviceToHost, s));
     OCTEX_HIP(hipMemcpyAsync(hi.data(), oi.ptr, static_cast<size_t>(m) * K * sizeof(int32_t), hipMemcpyDeviceToHost,
                              s));
@@ -541,9 +571,11 @@ void exact_table(index_impl& ix, int k, bool reverse_edges, std::vector<int32_t>
     build_log("exact table: %lld of %lld rows, %.1f s\n", static_cast<long long>(r0 + m), static_cast<long long>(n),
               seconds_since(t0));
   }
-  if (reverse_edges) {
-    const int h = std::max(1, k / 2);
-    merge_reverse(fid, n, reverse_rule{k, h, h, h, k}, table, fdist.data());
+  if (on_device) {
+    dtable = dbuf(static_cast<size_t>(n) * k * sizeof(int32_t));
+    merge_reverse_device(dfid.as<int32_t>(), dfdist.as<float>(), n, rr, dtable.as<int32_t>(), s);
+  } else if (reverse_edges) {
+    merge_reverse(fid, n, rr, table, fdist.data());
   } else {
     table = std::move(fid);
   }
@@ -555,7 +587,7 @@ void exact_table(index_impl& ix, int k, bool reverse_edges, std::vector<int32_t>
  * reverse edges merged by the rule kf = k/4 forward first, then up to k - kf reverse entries.
  */
 void searched_table(index_impl& ix, index const& idx, int k, bool reverse_edges, int passes, bool sketch_order,
-                    std::vector<int32_t>& table)
+                    std::vector<int32_t>& table, dbuf& dtable)
 {
   const int64_t n = ix.n, d = ix.dim;
   const int kin = k + k / 2, kq = kin + 1;
@@ -574,22 +606,28 @@ void searched_table(index_impl& ix, index const& idx, int k, bool reverse_edges,
   sp.batch        = 10000;
   sp.sketch_rank  = true;
   sp.final_rerank = sketch_order ? 0 : std::max(64, kin + 1);
-  std::vector<int32_t> fwd(static_cast<size_t>(n) * kin);
+  const bool on_device = reverse_edges && merge_on_device(n, rr);
+  dbuf dfwd(on_device ? static_cast<size_t>(n) * kin * sizeof(int32_t) : 0);
+  std::vector<int32_t> fwd(on_device ? 0 : static_cast<size_t>(n) * kin);
   const int64_t chunk = std::min<int64_t>(n, int64_t{1} << 20);
   dbuf qf(static_cast<size_t>(chunk) * d * sizeof(float));
   dbuf nb(static_cast<size_t>(chunk) * kq * sizeof(int64_t)), nd(static_cast<size_t>(chunk) * kq * sizeof(float));
-  std::vector<int64_t> hnb(static_cast<size_t>(chunk) * kq);
+  std::vector<int64_t> hnb(on_device ? 0 : static_cast<size_t>(chunk) * kq);
   raft::resources res;
   res.set_stream(ix.stream);
   for (size_t v = 0; v < plan.size(); v++) {
     auto t0 = std::chrono::steady_clock::now();
-    if (plan[v].waves > 0) set_table(ix, table, k);
+    if (plan[v].waves > 0) on_device ? set_device_table(ix, std::move(dtable), k) : set_table(ix, table, k);
     sp.starts = plan[v].starts;
     sp.waves  = plan[v].waves;
     for (int64_t r0 = 0; r0 < n; r0 += chunk) {
       const int64_t m = std::min(chunk, n - r0);
       half_to_float(ix.vecs() + r0 * d, m * d, qf.as<float>(), ix.stream);
       search_impl(res, sp, idx, qf.as<float>(), m, d, nb.as<int64_t>(), nd.as<float>(), kq, false, false);
+      if (on_device) {
+        drop_self(nb.as<int64_t>(), r0, m, kq, kin, dfwd.as<int32_t>() + r0 * kin, ix.stream);
+        continue;
+      }
       OCTEX_HIP(hipStreamSynchronize(ix.stream));
       OCTEX_HIP(hipMemcpy(hnb.data(), nb.ptr, sizeof(int64_t) * m * kq, hipMemcpyDeviceToHost));
       parallel_for(m, [&](int64_t i0, int64_t i1) {  // drop the vector itself, keep the first kin
@@ -609,8 +647,12 @@ void searched_table(index_impl& ix, index const& idx, int k, bool reverse_edges,
         build_log("table pass %zu: %lld of %lld rows, %.1f s\n", v + 1, static_cast<long long>(r0 + m),
                   static_cast<long long>(n), seconds_since(t0));
     }
+    if (on_device) OCTEX_HIP(hipStreamSynchronize(ix.stream));
     if (plan[v].waves > 0) drop_table(ix);
-    if (reverse_edges) {
+    if (on_device) {
+      dtable = dbuf(static_cast<size_t>(n) * k * sizeof(int32_t));
+      merge_reverse_device(dfwd.as<int32_t>(), nullptr, n, rr, dtable.as<int32_t>(), ix.stream);
+    } else if (reverse_edges) {
       build_log("table pass %zu: searched in %.1f s, merging reverse edges\n", v + 1, seconds_since(t0));
       merge_reverse(fwd, n, rr, table);
     } else {
@@ -942,13 +984,14 @@ auto build_in_memory(index_params const& params, dataset_view const& x, build_re
   // neighbor table: exact up to exact_table_max rows (build.cu:354-360), else searched by this library's search
   if (k > 0) {
     std::vector<int32_t> table;
+    dbuf dtable;  // or the rows on the device
     if (n <= params.exact_table_max) {
-      exact_table(ix, k, params.reverse_edges, table);
+      exact_table(ix, k, params.reverse_edges, table, dtable);
     } else {
       index idx(impl);
-      searched_table(ix, idx, k, params.reverse_edges, params.table_passes, params.table_sketch_order, table);
+      searched_table(ix, idx, k, params.reverse_edges, params.table_passes, params.table_sketch_order, table, dtable);
     }
-    set_table(ix, table, k);
+    dtable.ptr != nullptr ? set_device_table(ix, std::move(dtable), k) : set_table(ix, table, k);
     phase("table");
   }
   OCTEX_HIP(hipSetDevice(cur));
@@ -1145,13 +1188,14 @@ auto resume_table(index_params const& params, dataset_view const& x, std::string
   const int k = params.table_len;
   if (k > 0) {
     std::vector<int32_t> table;
+    dbuf dtable;  // or the rows on the device
     if (x.n <= params.exact_table_max) {
-      exact_table(ix, k, params.reverse_edges, table);
+      exact_table(ix, k, params.reverse_edges, table, dtable);
     } else {
       index idx(impl);
-      searched_table(ix, idx, k, params.reverse_edges, params.table_passes, params.table_sketch_order, table);
+      searched_table(ix, idx, k, params.reverse_edges, params.table_passes, params.table_sketch_order, table, dtable);
     }
-    set_table(ix, table, k);
+    dtable.ptr != nullptr ? set_device_table(ix, std::move(dtable), k) : set_table(ix, table, k);
   }
   rec.phases.emplace_back("table", seconds_since(t0));
   build_log("table: %.2f s\n", rec.phases.back().second);

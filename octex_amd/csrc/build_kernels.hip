@@ -1128,6 +1128,138 @@ __global__ void merge_lists_kernel(const float* __restrict__ bd, const int* __re
   }
 }
 
+// ------------------------------------------------------------------ neighbor table rows (build_table.cuh:60-74, 166-252)
+
+/** drop_self: a wavefront a row, the kept entries placed by ballots. */
+template <typename T>
+__global__ __launch_bounds__(256) void drop_self_kernel(const T* __restrict__ ids, const float* __restrict__ dist, int64_t r0,
+                                                        int64_t m, int K, int k, int* __restrict__ out,
+                                                        float* __restrict__ out_d)
+{
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int lane  = threadIdx.x & 63;
+  if (i >= m) return;
+  int at = 0;
+  for (int j0 = 0; j0 < K; j0 += 64) {  // uniform over the wavefront
+    const int j                   = j0 + lane;
+    const T v                     = j < K ? ids[i * K + j] : T{-1};
+    const bool keep               = j < K && v != static_cast<T>(r0 + i);
+    const unsigned long long mask = __ballot(keep);
+    const int o                   = at + __popcll(mask & ((1ULL << lane) - 1ULL));
+    if (keep && o < k) {
+      out[i * k + o] = v < 0 ? -1 : static_cast<int>(v);
+      if (out_d != nullptr) {
+        const float dv   = dist[i * K + j];
+        out_d[i * k + o] = v < 0 ? INFINITY : (dv > 0.f ? dv : 0.f);
+      }
+    }
+    at += __popcll(mask);
+  }
+  for (int o = min(at, k) + lane; o < k; o += 64) {
+    out[i * k + o] = -1;
+    if (out_d != nullptr) out_d[i * k + o] = INFINITY;
+  }
+}
+
+/** The reverse entries: entry r of row v naming u as key u 2^8 + r (n 2^8 for none) with value v. */
+__global__ __launch_bounds__(256) void reverse_keys_kernel(const int* __restrict__ fwd, int64_t n, int kin, int ks,
+                                                           unsigned long long* __restrict__ key, int* __restrict__ val)
+{
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (t >= n * ks) return;
+  const int64_t v = t / ks;
+  const int r     = static_cast<int>(t - v * ks);
+  const int u     = fwd[v * kin + r];
+  key[t]          = u >= 0 && u != v ? (static_cast<unsigned long long>(u) << 8) | static_cast<unsigned>(r)
+                                     : static_cast<unsigned long long>(n) << 8;
+  val[t]          = static_cast<int>(v);
+}
+
+/**
+ * The merged row of u = blockIdx.x by one wavefront: the row's candidates in the rule's order in LDS (at most kin + kr),
+ * an entry dropped when an earlier one holds its id (all pairs, the earlier ids by broadcast reads: 144 candidates of a
+ * table of 64 take 3 x 144 steps), the rest numbered by ballots.  (key, val): the sorted reverse entries, total of them;
+ * the row's are found by binary search.
+ */
+__global__ __launch_bounds__(64) void merge_rows_kernel(const int* __restrict__ fwd, const float* __restrict__ fdist,
+                                                        const unsigned long long* __restrict__ key,
+                                                        const int* __restrict__ val, int64_t total, reverse_rule rr,
+                                                        int* __restrict__ table)
+{
+  extern __shared__ int rows_lds[];
+  const int cap = rr.kin + rr.kr;
+  int* id       = rows_lds;                                  // [cap]
+  float* dist   = reinterpret_cast<float*>(id + cap);        // [cap], with fdist
+  auto* kept    = reinterpret_cast<unsigned long long*>(dist + cap);  // [kout], with fdist (2 cap words before it)
+  const int64_t u = blockIdx.x;
+  const int lane  = threadIdx.x;
+  int64_t lo = 0, hi = total;  // lanes 0 and 1: the first entry of rows u and u + 1
+  const unsigned long long want = static_cast<unsigned long long>(u + (lane & 1)) << 8;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (key[mid] < want)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  const int64_t e0 = __shfl(lo, 0);
+  const int nrev   = static_cast<int>(min(static_cast<int64_t>(rr.kr), static_cast<int64_t>(__shfl(lo, 1)) - e0));
+  const int nc     = rr.kin + nrev;
+  for (int c = lane; c < nc; c += 64) {
+    int v   = -1;
+    float d = 0.f;
+    if (c >= rr.kf && c < rr.kf + nrev) {
+      const int64_t e = e0 + (c - rr.kf);
+      v               = val[e];
+      if (fdist != nullptr) d = fdist[static_cast<int64_t>(v) * rr.kin + static_cast<int>(key[e] & 255)];
+    } else {
+      const int t = c < rr.kf ? c : c - nrev;
+      v           = fwd[u * rr.kin + t];
+      if (fdist != nullptr) d = fdist[u * rr.kin + t];
+    }
+    id[c] = v < 0 || v == u ? -1 : v;
+    if (fdist != nullptr) dist[c] = d > 0.f ? d : 0.f;
+  }
+  __syncthreads();
+  int* row = table + u * rr.kout;
+  int at   = 0;
+  for (int c0 = 0; c0 < nc && at < rr.kout; c0 += 64) {  // uniform
+    const int c = c0 + lane;
+    const int v = c < nc ? id[c] : -1;
+    bool keep   = v >= 0;
+    for (int j = 0; j < min(nc, c0 + 64); j++)  // uniform trips
+      if (j < c && id[j] == v) keep = false;
+    const unsigned long long mask = __ballot(keep);
+    const int o                   = at + __popcll(mask & ((1ULL << lane) - 1ULL));
+    if (keep && o < rr.kout) {
+      if (fdist != nullptr)
+        kept[o] = (static_cast<unsigned long long>(__float_as_uint(dist[c])) << 32) | static_cast<unsigned>(v);
+      else
+        row[o] = v;
+    }
+    at += __popcll(mask);
+  }
+  const int nk = min(at, rr.kout);
+  for (int o = nk + lane; o < rr.kout; o += 64)
+    row[o] = -1;
+  if (fdist == nullptr) return;
+  __syncthreads();
+  for (int o = lane; o < nk; o += 64) {  // nearest first, ties by id: an entry's place is the number of smaller ones
+    const unsigned long long e = kept[o];
+    int place                  = 0;
+    for (int j = 0; j < nk; j++)
+      place += kept[j] < e ? 1 : 0;
+    row[place] = static_cast<int>(e & 0xffffffffULL);
+  }
+}
+
+/** LDS bytes of merge_rows_kernel. */
+auto merge_rows_lds(reverse_rule const& rr) -> size_t
+{
+  const size_t cap = static_cast<size_t>(rr.kin + rr.kr);
+  return 2 * cap * sizeof(int) + static_cast<size_t>(rr.kout) * sizeof(unsigned long long);
+}
+
 template <typename T>
 void ensure(dbuf& b, int64_t count)
 {
@@ -1149,6 +1281,47 @@ void with_tmp(dbuf& tmp, F&& call)
 }  // namespace
 
 // ================================================================== host side
+
+auto merge_reverse_bytes(int64_t n, reverse_rule const& rr) -> size_t
+{
+  return static_cast<size_t>(n) * rr.ks * 36;  // keys and rows, sorted and unsorted, and as much again for the sort
+}
+
+void merge_reverse_device(const int* fwd, const float* fdist, int64_t n, reverse_rule const& rr, int* table, hipStream_t s)
+{
+  OCTEX_EXPECTS(rr.ks >= 1 && rr.ks <= 256 && rr.ks <= rr.kin && rr.kf <= rr.kin && rr.kr >= 0 && rr.kout >= 1,
+                "octex: the reverse-edge merge takes forward rows of at most 256 entries");
+  OCTEX_EXPECTS(merge_rows_lds(rr) <= 64 * 1024 && n < (int64_t{1} << 31), "octex: reverse-edge rows too long");
+  const int64_t total = n * rr.ks;
+  dbuf key(static_cast<size_t>(total) * 8), skey(static_cast<size_t>(total) * 8), val(static_cast<size_t>(total) * 4),
+    sval(static_cast<size_t>(total) * 4), tmp;
+  reverse_keys_kernel<<<grid_for(total, 256), 256, 0, s>>>(fwd, n, rr.kin, rr.ks, key.as<unsigned long long>(),
+                                                          val.as<int>());
+  with_tmp(tmp, [&](void* p, size_t& b) {
+    return rocprim::radix_sort_pairs(p, b, key.as<unsigned long long>(), skey.as<unsigned long long>(), val.as<int>(),
+                                     sval.as<int>(), static_cast<size_t>(total), 0, 8 + log2_ceil(n + 1), s);
+  });
+  merge_rows_kernel<<<static_cast<unsigned>(n), 64, merge_rows_lds(rr), s>>>(fwd, fdist, skey.as<unsigned long long>(),
+                                                                            sval.as<int>(), total, rr, table);
+  OCTEX_HIP(hipGetLastError());
+  OCTEX_HIP(hipStreamSynchronize(s));
+}
+
+void drop_self(const int64_t* ids, int64_t r0, int64_t m, int K, int k, int* out, hipStream_t s)
+{
+  if (m == 0) return;
+  drop_self_kernel<long long><<<grid_for(m, 4), 256, 0, s>>>(reinterpret_cast<const long long*>(ids), nullptr, r0, m, K, k,
+                                                            out, nullptr);
+  OCTEX_HIP(hipGetLastError());
+}
+
+void drop_self(const int* ids, const float* dist, int64_t r0, int64_t m, int K, int k, int* out, float* out_d,
+               hipStream_t s)
+{
+  if (m == 0) return;
+  drop_self_kernel<int><<<grid_for(m, 4), 256, 0, s>>>(ids, dist, r0, m, K, k, out, out_d);
+  OCTEX_HIP(hipGetLastError());
+}
 
 void pca_scatter(const __half* x, int64_t n, int d, int64_t step, int64_t ns, const float* mean, double* G,
                  hipStream_t s)

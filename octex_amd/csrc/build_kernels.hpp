@@ -49,6 +49,23 @@ struct row_source {
 void make_sketch(row_source& x, int64_t n, int d, const float* mean, const float* basis, int S, int pitch,
                  std::vector<float>& scale, signed char* codes, hipStream_t s);
 
+/** The rule of a merged table row (build_table.cuh:157-164): its first kf forward entries, up to kr reverse entries
+ * (lowest rank first, then lowest id), then its other forward entries; duplicates, -1 and the row itself dropped; the
+ * first kout kept, in that priority order.  A reverse entry is an entry of a row's first ks forward ones. */
+struct reverse_rule {
+  int kin, kf, ks, kr, kout;
+};
+/** Device bytes of merge_reverse_device over n rows, beside its inputs and its table. */
+auto merge_reverse_bytes(int64_t n, reverse_rule const& rr) -> size_t;
+/** The table rows [n, kout] of the forward rows fwd [n, kin] with their reverse edges by the rule, -1 padded; with fdist
+ * [n, kin] (the forward distances) a row's kept entries nearest first, ties by id (build_table.cuh:240-251). */
+void merge_reverse_device(const int* fwd, const float* fdist, int64_t n, reverse_rule const& rr, int* table, hipStream_t s);
+/** Rows ids [m, K] of the dataset's rows r0 + i without the row itself, its first k to out [m, k], -1 padded (other
+ * negative ids -1); with dist [m, K] its distances, at least 0 and +inf for -1, to out_d. */
+void drop_self(const int64_t* ids, int64_t r0, int64_t m, int K, int k, int* out, hipStream_t s);
+void drop_self(const int* ids, const float* dist, int64_t r0, int64_t m, int K, int k, int* out, float* out_d,
+               hipStream_t s);
+
 /**
  * An IVF index of one copy's projected rows y [n, w], for the reference's default cell lists (build_cells.cuh:511-516,
  * 584-596: cuVS ivf_flat with max(64, 4 sqrt(n)) lists trained on half the rows, a tenth above 4M, searched with

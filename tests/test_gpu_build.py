@@ -200,6 +200,22 @@ def test_exact_table_matches_oracle(octex, tmp_path, n, d, reverse):
     assert np.array_equal(tg, tc)
 
 
+@pytest.mark.parametrize("n,table_len,exact", [(3000, 64, True), (900, 1, True), (900, 127, True), (4000, 32, False),
+                                               (3000, 100, False), (600, 3, False)])
+def test_reverse_edges_merged_on_the_gpu_and_the_host(octex, data, monkeypatch, n, table_len, exact):
+    """The reverse edges merged by the GPU, as long as its memory holds them, and by host threads: the same table rows
+    (nearest first for the exact table; rows of one entry, of the most, and shorter than their reverse entries)."""
+    X = np.round(data[0][:n] * 2)  # many equal distances
+    kw = dict(copies=8, list_len=16, table_len=table_len, log_buckets=10, min_cell=2, member_lists=True, seed=3,
+              exact_table_max=n if exact else 0)
+    tables = []
+    for host in ("0", "1"):
+        monkeypatch.setenv("OCTEX_MERGE_HOST", host)
+        index, _ = octex.build_in_memory(X, **kw)
+        tables.append(index.array("table", np.int32))
+    assert np.array_equal(*tables)
+
+
 # The k-NN kernel's row widths: 3, 7 and 8 k steps of 16 (held fragments), 9 and 13 (not held), a partial step; rows of 0
 # and 1, of which hundreds lie at one distance (more ties at the K-th than its key lists hold), and 300 equal rows
 @pytest.mark.parametrize("n,d,top", [(700, 48, 8), (700, 112, 8), (600, 128, 8), (600, 144, 8), (400, 208, 8),
