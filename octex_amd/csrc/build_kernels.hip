@@ -1079,7 +1079,9 @@ __global__ __launch_bounds__(256) void ivf_scan_kernel(const float* __restrict__
       if (key < thr) keys[kIvfSort - kIvfBuf + atomicAdd(&nbuf, 1)] = key;
     }
     __syncthreads();
-    if (nbuf > kIvfBuf - static_cast<int>(blockDim.x)) merge();  // the next round could overflow the buffer
+    const bool full = nbuf > kIvfBuf - static_cast<int>(blockDim.x);  // the next round could overflow the buffer
+    __syncthreads();  // every thread has read nbuf before the next round adds to it: all merge, or none
+    if (full) merge();
   }
   if (nbuf > 0) merge();
   for (int k = t; k < l; k += blockDim.x) {
