@@ -887,19 +887,31 @@ __global__ __launch_bounds__(256) void kmeans_scan_update_kernel(const float* __
   }
 }
 
+/** frag[(t KS + j) 64 + l] = element 4 j + l / 16 of row 16 t + l % 16 of X [n, 4 KS] (the last row past the end): the
+ * 16x16x4 MFMA fragments of 16-row tiles, a wavefront's 64 values side by side. */
+__global__ __launch_bounds__(256) void fragments_kernel(const float* __restrict__ X, int n, int KS, int64_t total,
+                                                        float* __restrict__ frag)
+{
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (t >= total) return;
+  const int l = static_cast<int>(t & 63), j = static_cast<int>((t >> 6) % KS);
+  const int64_t row = min((t >> 6) / KS * 16 + (l & 15), static_cast<int64_t>(n) - 1);
+  frag[t]           = X[row * 4 * KS + 4 * j + (l >> 4)];
+}
+
 /**
  * The nearest row of X [n, W] to each row of Q [m, W] by |q|^2 + |x|^2 - 2 q.x, ties by row: knn_kernel's distances (the
  * same MFMA tiles and sums) with K = 1, where a lane's running minimum replaces the key lists.  A workgroup takes 16 QT
- * rows of Q, their fragments in registers; its four wavefronts share out the 16-row tiles of X, the next tile's
- * fragments loaded ahead, and combine their minima through LDS.
+ * rows of Q, their fragments in registers; its four wavefronts share out the 16-row tiles of X, given as fragments
+ * (fragments_kernel), the next tile's loaded ahead, and combine their minima through LDS.
  * 16 rows a workgroup keep the chip busy from about 4,000 rows; at 65,536 and more 64 read X a quarter as often.
- * Measured on 10,000 rows of 32 against 565: 368 us through knn_kernel, 31 us here, held by the loads of X's fragments
- * (16 rows an instruction).
+ * Measured on 10,000 rows of 32 against 565: 368 us through knn_kernel, 31 us with X's fragments loaded from its rows
+ * (each instruction touched 64 lines), 14 us here and 4 us for the fragments.
  */
 template <int W, int QT>
 __global__ __launch_bounds__(256) void nearest_kernel(const float* __restrict__ Q, const float* __restrict__ qn, int64_t m,
-                                                      const float* __restrict__ X, const float* __restrict__ xn, int n,
-                                                      int* __restrict__ out_i)
+                                                      const float* __restrict__ frag, const float* __restrict__ xn,
+                                                      int n, int* __restrict__ out_i)
 {
   constexpr int KS = W / 4;
   __shared__ unsigned long long best_key[4][16 * QT];
@@ -919,10 +931,10 @@ __global__ __launch_bounds__(256) void nearest_kernel(const float* __restrict__ 
   }
   float a[KS], an[KS], xr[4], xrn[4];
   auto load = [&](int tile) {  // the tile's fragments and norms into an, xrn (past the end: the last row)
-    const float* r = X + static_cast<int64_t>(min(tile * 16 + r16, n - 1)) * W + kq;
+    const float* r = frag + static_cast<int64_t>(min(tile, (n + 15) / 16 - 1)) * KS * 64 + lane;
 #pragma unroll
     for (int j = 0; j < KS; j++)
-      an[j] = r[4 * j];
+      an[j] = r[64 * j];
 #pragma unroll
     for (int j = 0; j < 4; j++)
       xrn[j] = xn[min(tile * 16 + 4 * kq + j, n - 1)];
@@ -1423,17 +1435,21 @@ template void knn_rows<float>(const float*, const float*, int64_t, const float*,
 
 namespace {
 
-/** out_i [m]: the nearest row of X [n, w] to each row of Q, as knn_rows with K = 1 (dtmp: its distances, if it is run). */
+/** out_i [m]: the nearest row of X [n, w] to each row of Q, as knn_rows with K = 1 (dtmp: X's fragments, or knn_rows'
+ * distances). */
 void nearest_rows(const float* Q, const float* qn, int64_t m, const float* X, const float* xn, int n, int w, int* out_i,
                   dbuf& dtmp, hipStream_t s)
 {
   if (m == 0) return;
   auto go = [&](auto w_tag) {
-    constexpr int W = decltype(w_tag)::value;
+    constexpr int W     = decltype(w_tag)::value;
+    const int64_t total = int64_t{(n + 15) / 16} * 16 * W;
+    ensure<float>(dtmp, total);
+    fragments_kernel<<<grid_for(total, 256), 256, 0, s>>>(X, n, W / 4, total, dtmp.as<float>());
     if (m >= 65536)
-      nearest_kernel<W, 4><<<grid_for(m, 64), 256, 0, s>>>(Q, qn, m, X, xn, n, out_i);
+      nearest_kernel<W, 4><<<grid_for(m, 64), 256, 0, s>>>(Q, qn, m, dtmp.as<float>(), xn, n, out_i);
     else
-      nearest_kernel<W, 1><<<grid_for(m, 16), 256, 0, s>>>(Q, qn, m, X, xn, n, out_i);
+      nearest_kernel<W, 1><<<grid_for(m, 16), 256, 0, s>>>(Q, qn, m, dtmp.as<float>(), xn, n, out_i);
   };
   switch (w) {
     case 8: go(std::integral_constant<int, 8>{}); break;
