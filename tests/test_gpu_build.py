@@ -250,6 +250,20 @@ def test_kmeans_centers_give_the_same_ivf_lists(octex, n, blocks):
         assert all(len(set(r)) == 16 for r in rows[:500])
 
 
+@pytest.mark.parametrize("n", [639, 640, 641, 1000])  # the last group of 64 rows of the lists' layout
+@pytest.mark.parametrize("blocks,list_len", [(1, 16), (4, 128), (8, 64)])
+def test_ivf_lists_over_row_groups(octex, n, blocks, list_len):
+    """Every list probed, IVF lists are the exact ones wherever the last group of rows ends and however many keys wait
+    for a sort."""
+    X = clustered(n=n, m=1, d=64, clusters=9, seed=n)[0].astype(np.float16)
+    kw = dict(copies=1, blocks=blocks, list_len=list_len, log_buckets=10, table_len=0, min_cell=3, seed=2)
+    ivf, _ = octex.build_in_memory(X, list_probes=1 << 20, **kw)
+    exact, _ = octex.build_in_memory(X, exact_lists=True, **kw)
+    a, b = (ix.array("lists", np.int32, copy=0) for ix in (ivf, exact))
+    assert a.shape == b.shape and a.size
+    assert (a != b).mean() < 5e-3  # near ties of the two distance forms
+
+
 def test_exact_table_real_valued(octex, data, tmp_path):
     """On real-valued rows the forward table holds the exact k nearest (fp64) up to near ties of the
     fp32 expanded distance |x|^2 + |y|^2 - 2 x.y, nearest first; no self, no duplicates."""
