@@ -766,12 +766,8 @@ auto build_in_memory(index_params const& params, dataset_view const& x, build_re
 
   // PCA of a sample (build_setup.cuh:40-103): every step-th row
   const int64_t step = std::max<int64_t>(1, n / 200000), ns = (n + step - 1) / step;
-  std::vector<__half> sample(static_cast<size_t>(ns) * d);
-  sample_rows(xd, ns, step, static_cast<int>(d), sample.data(), s);
   std::vector<double> mu(d, 0.0);
-  for (int64_t i = 0; i < ns; i++)
-    for (int64_t j = 0; j < d; j++)
-      mu[j] += static_cast<double>(__half2float(sample[i * d + j]));
+  sample_sums(xd, ns, step, static_cast<int>(d), mu.data(), s);
   rec.mean.resize(d);
   for (int64_t j = 0; j < d; j++)
     rec.mean[j] = static_cast<float>(mu[j] / static_cast<double>(ns));

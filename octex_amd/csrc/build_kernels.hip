@@ -36,12 +36,19 @@ __global__ void pca_sample_kernel(const __half* __restrict__ x, int64_t ns, int6
   A[t]      = static_cast<double>(__half2float(x[i * step * d + k]) - mean[k]);
 }
 
-__global__ void sample_rows_kernel(const __half* __restrict__ x, int64_t ns, int64_t step, int d,
-                                   __half* __restrict__ out)
+constexpr int kMeanRows = 256;  // sampled rows a workgroup of column_sums_kernel adds
+
+/** part[b, k] = the sum in fp64 of column k over the sampled rows b kMeanRows .. + kMeanRows - 1, in order. */
+__global__ __launch_bounds__(256) void column_sums_kernel(const __half* __restrict__ x, int64_t ns, int64_t step, int d,
+                                                          double* __restrict__ part)
 {
-  int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= ns * d) return;
-  out[t] = x[(t / d) * step * d + t % d];
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kMeanRows, i1 = min(i0 + kMeanRows, ns);
+  for (int k = threadIdx.x; k < d; k += 256) {
+    double acc = 0;
+    for (int64_t i = i0; i < i1; i++)
+      acc += static_cast<double>(__half2float(x[i * step * d + k]));
+    part[static_cast<int64_t>(blockIdx.x) * d + k] = acc;
+  }
 }
 
 /** G = A^T A (fp64) by 16 x 16 output tiles, samples staged through LDS in chunks of 64 rows. */
@@ -1360,14 +1367,19 @@ void pca_scatter(const __half* x, int64_t n, int d, int64_t step, int64_t ns, co
   OCTEX_HIP(hipStreamSynchronize(s));
 }
 
-void sample_rows(const __half* x, int64_t ns, int64_t step, int d, __half* host_out, hipStream_t s)
+void sample_sums(const __half* x, int64_t ns, int64_t step, int d, double* sums, hipStream_t s)
 {
-  if (ns * d == 0) return;
-  dbuf tmp(static_cast<size_t>(ns) * d * sizeof(__half));
-  sample_rows_kernel<<<grid_for(ns * d, 256), 256, 0, s>>>(x, ns, step, d, tmp.as<__half>());
+  const int64_t blocks = (ns + kMeanRows - 1) / kMeanRows;
+  dbuf part(static_cast<size_t>(blocks) * d * sizeof(double));
+  column_sums_kernel<<<static_cast<unsigned>(blocks), 256, 0, s>>>(x, ns, step, d, part.as<double>());
   OCTEX_HIP(hipGetLastError());
-  OCTEX_HIP(hipMemcpyAsync(host_out, tmp.ptr, tmp.size, hipMemcpyDeviceToHost, s));
+  std::vector<double> h(static_cast<size_t>(blocks) * d);
+  OCTEX_HIP(hipMemcpyAsync(h.data(), part.ptr, part.size, hipMemcpyDeviceToHost, s));
   OCTEX_HIP(hipStreamSynchronize(s));
+  std::fill(sums, sums + d, 0.0);
+  for (int64_t b = 0; b < blocks; b++)
+    for (int k = 0; k < d; k++)
+      sums[k] += h[b * d + k];
 }
 
 void project_rows(const __half* x, int64_t n, int d, const float* mean, const float* U, const float* shift, int w,

@@ -264,6 +264,16 @@ def test_ivf_lists_over_row_groups(octex, n, blocks, list_len):
     assert (a != b).mean() < 5e-3  # near ties of the two distance forms
 
 
+@pytest.mark.parametrize("n,d", [(100, 32), (255, 32), (256, 64), (257, 300), (400001, 32)])
+def test_sampled_mean(octex, n, d):
+    """The mean over every max(1, n / 200000)-th row, summed in fp64 by parts of 256 rows, is the fp64 mean rounded to
+    fp32: the sums differ by less than ns 2^-53 relative to the sum of magnitudes."""
+    X = (np.random.default_rng(n).standard_normal((n, d)) + 3).astype(np.float16)
+    ix, _ = octex.build_in_memory(X, copies=1, blocks=1, list_len=8, log_buckets=10, table_len=0, seed=2)
+    ref = X[:: max(1, n // 200000)].astype(np.float64).mean(0)
+    np.testing.assert_allclose(ix.array("mean", np.float32), ref, rtol=2.0**-23, atol=0)
+
+
 def test_exact_table_real_valued(octex, data, tmp_path):
     """On real-valued rows the forward table holds the exact k nearest (fp64) up to near ties of the
     fp32 expanded distance |x|^2 + |y|^2 - 2 x.y, nearest first; no self, no duplicates."""
