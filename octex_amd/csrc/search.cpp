@@ -1,8 +1,9 @@
 // octex::search for one MI355X (the reference: search.cu:294-518 first_round / wave_round, :619-814
 // plans, :816-961 the batch loop).  A plan holds the batch buffers of one (batch, k, search
-// parameters) and one hipGraph of the whole batch: center, projection, sketch query, probe, gather,
-// keep, then the waves (pick starts, gather rows, keep) and the best k.  Batches larger than the
-// captured size are split; the last partial batch is padded with copies of its first query.
+// parameters) and one hipGraph of a batch's stages between the first (prepare: center and sketch query, which reads
+// the queries) and the last (which writes the results): projection, probe, gather, keep, then the waves (gather rows,
+// keep).  Batches run on the caller's stream.  Batches larger than the captured size are split; the last partial
+// batch is padded with copies of its first query.
 
 #include "search.hpp"
 

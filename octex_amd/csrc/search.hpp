@@ -75,7 +75,8 @@ auto carve_buffers(index_impl const& ix, plan_shape const& sh, void* base, batch
 auto named_buffer(index_impl const& ix, plan_shape const& sh, batch_buffers const& b, std::string const& name)
   -> std::pair<const void*, size_t>;
 
-/** One plan: its shape, one block of batch buffers and the graph of a whole batch on the index's stream. */
+/** One plan: its shape, one block of batch buffers and the graph of a batch's stages between its first and
+ * last launch. */
 struct plan {
   plan_shape shape;
   dbuf block;
