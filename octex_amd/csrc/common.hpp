@@ -30,12 +30,16 @@ namespace cuvs::neighbors::octex::detail {
     if (!(cond)) ::cuvs::neighbors::octex::detail::fail(__VA_ARGS__); \
   } while (0)
 
+/** A failed call throws and leaves no last error behind: the check of the next launch (hipGetLastError) would report it
+ * again and fail a call that has nothing to do with it. */
 #define OCTEX_HIP(call)                                                                        \
   do {                                                                                         \
     hipError_t e_ = (call);                                                                    \
-    if (e_ != hipSuccess)                                                                      \
+    if (e_ != hipSuccess) {                                                                    \
+      (void)hipGetLastError();                                                                 \
       ::cuvs::neighbors::octex::detail::fail("octex: HIP error %s (%s) at %s:%d", hipGetErrorName(e_), \
                                              hipGetErrorString(e_), __FILE__, __LINE__);      \
+    }                                                                                          \
   } while (0)
 
 /** Device memory of one allocation (freed on destruction). */

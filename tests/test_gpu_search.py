@@ -397,6 +397,24 @@ def test_errors(octex, small_index):
     assert index.device_bytes[0] > 0
 
 
+def test_search_after_a_failed_allocation(octex, small_index):
+    """A search whose batch buffers do not fit the GPU is an error, and the next search runs: the failed call's error does
+    not stay behind for the next launch's check."""
+    from octex_amd._lib import OctexError
+
+    index = octex.load(small_index["path"])
+    Q = small_index["Q"][:40]
+    D1, I1 = index.search(Q, k=10, **PARAMS)
+    m = 1 + torch.cuda.get_device_properties(0).total_memory // (8 * 2048)  # 2048 (id, score) slots a query at least
+    q = torch.zeros((m, index.dim), device="cuda")
+    print(f"a batch of {m} queries", flush=True)
+    with pytest.raises(OctexError, match="hipErrorOutOfMemory"):
+        index.search(q, k=1, batch=m, read=1, starts=1, waves=0, rerank=1)
+    del q
+    D2, I2 = index.search(Q, k=10, **PARAMS)
+    assert np.array_equal(I1, I2) and np.array_equal(D1, D2)
+
+
 def test_oracle_index_with_probed_rows_only(octex, small_index):
     """The host copy that keeps only the list rows a sample's probes reach (the CPU baseline of an index
     too large for host memory) searches that sample exactly like the full copy; array ranges read the
