@@ -434,20 +434,36 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   // the batches run on the caller's stream itself, after the previous search of the index (its plan buffers may be the
   // same), which may have run on another stream.  A hop to the index's stream and back, two events and two waits, took
   // 38 us of a search of one query
+  hipStream_t s = call;
   if (call != nullptr) {
     int at = ix.device;
     OCTEX_HIP(hipStreamGetDevice(call, &at));
     OCTEX_EXPECTS(at == ix.device, "octex: the search's stream is on device %d, the index on device %d", at, ix.device);
+  } else {
+    // the null stream takes no launch while any blocking stream of the process is captured: the index's stream does
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    const hipError_t e        = hipStreamIsCapturing(call, &st);
+    if (e == hipErrorStreamCaptureImplicit) {
+      (void)hipGetLastError();
+      s = ix.stream;
+    } else {
+      OCTEX_HIP(e);
+    }
   }
-  OCTEX_HIP(hipStreamWaitEvent(call, ix.searched, 0));
+  OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));
+  if (s != call) {
+    OCTEX_HIP(hipEventRecord(ix.searched, call));
+    OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));
+  }
   // queries and results in the GPU's own memory are read and written in place by the batch's first and last kernel;
   // others are copied (each copy and its gap about 10 us of a small search)
   const bool in_place  = !resident && !host_out && on_device(queries, ix.device);
   const bool out_place = !resident && !host_out && on_device(neighbors, ix.device) && on_device(distances, ix.device);
   auto mark = [&] {  // the event the next search, and whoever frees or reads the buffers, waits for
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(call, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
-      OCTEX_HIP(hipEventRecord(ix.searched, call));
+    const hipError_t e = hipEventRecord(ix.searched, s);
+    if (e == hipSuccess) return;
+    (void)hipStreamSynchronize(s);  // no event stands for the batches: they end before the lock is given up
+    OCTEX_HIP(e);
   };
   try {
     for (int64_t b0 = 0; b0 < nq; b0 += m) {
@@ -460,11 +476,11 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
         io.distances = distances + b0 * k;
       }
       if (!resident && !in_place)
-        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, call));
-      run_batch(ix, *pl, io, call);
+        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, s));
+      run_batch(ix, *pl, io, s);
       if (!resident && !out_place) {
-        OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, call));
-        OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, call));
+        OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, s));
+        OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, s));
       }
     }
   } catch (...) {
@@ -475,9 +491,10 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
     throw;
   }
   mark();
+  if (s != call) OCTEX_HIP(hipStreamWaitEvent(call, ix.searched, 0));
   pl.reset();  // an evicted plan goes here, with the stream lock held
   run.unlock();
-  if (host_out) OCTEX_HIP(hipStreamSynchronize(call));
+  if (host_out) OCTEX_HIP(hipStreamSynchronize(s));
   OCTEX_HIP(hipSetDevice(cur));
 }
 

@@ -5,6 +5,8 @@ search returns the same ids and bit-identical distances; against exact search, r
 reference's tests (test_build.py:48-54, octex_c.cu:196).  Batch splitting / padding, graph replay, device tensors,
 sketch-rank mode and the parameter limits are covered too."""
 
+import ctypes as ct
+
 import numpy as np
 import pytest
 from conftest import exact_knn, recall
@@ -395,6 +397,36 @@ def test_errors(octex, small_index):
         octex.load(small_index["path"] + "_missing")
     assert index.size == 4000 and index.dim == 64 and index.copies == 16 and len(index.devices) == 1
     assert index.device_bytes[0] > 0
+
+
+def hip_runtime():
+    """The HIP runtime that this process has loaded."""
+    return ct.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])  # global, thread-local, relaxed
+def test_null_stream_search_while_a_blocking_stream_is_captured(octex, small_index, mode):
+    """The null stream takes no launch while a blocking stream is being captured: searches on it run on the index's
+    stream then, with the same results (host and device queries), and their work does not enter the capture."""
+    index = octex.load(small_index["path"])
+    Q = small_index["Q"][:40]
+    q = torch.from_numpy(Q).cuda()
+    D0, I0 = index.search(Q, k=10, **PARAMS)
+    torch.cuda.synchronize()
+    hip = hip_runtime()
+    stream, graph, nodes = ct.c_void_p(), ct.c_void_p(), ct.c_size_t(99)
+    assert hip.hipStreamCreate(ct.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, ct.c_int(mode)) == 0
+    try:
+        found = [index.search(Q, k=10, **PARAMS), index.search(q, k=10, **PARAMS)]
+    finally:
+        assert hip.hipStreamEndCapture(stream, ct.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ct.byref(nodes)) == 0 and nodes.value == 0
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+    torch.cuda.synchronize()
+    for D, I in found + [index.search(Q, k=10, **PARAMS)]:
+        assert np.array_equal(I0, np.asarray(torch.as_tensor(I).cpu()))
+        assert np.array_equal(D0, np.asarray(torch.as_tensor(D).cpu()))
 
 
 def test_search_after_a_failed_allocation(octex, small_index):
