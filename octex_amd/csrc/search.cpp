@@ -494,7 +494,7 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   if (s != call) OCTEX_HIP(hipStreamWaitEvent(call, ix.searched, 0));
   pl.reset();  // an evicted plan goes here, with the stream lock held
   run.unlock();
-  if (host_out) OCTEX_HIP(hipStreamSynchronize(s));
+  if (host_out) OCTEX_HIP(hipStreamSynchronize(call));  // behind s: under a capture only the null stream may be waited for
   OCTEX_HIP(hipSetDevice(cur));
 }
 
