@@ -424,8 +424,8 @@ extern "C" cuvsError_t octexIndexCopyPlanBuffer(cuvsOctexIndex_t index, const ch
     std::shared_ptr<octex::detail::plan> pl;
     {
       std::lock_guard<std::mutex> lock(ix.mu);
-      OCTEX_EXPECTS(!ix.plans.empty(), "octex: no search ran on this index yet");
-      pl = ix.plans.begin()->second;
+      pl = octex::detail::shown_plan(ix);
+      OCTEX_EXPECTS(pl != nullptr, "octex: no search ran on this index yet");
     }
     auto [src, sz] = octex::detail::named_buffer(ix, pl->shape, pl->buf, std::string(name != nullptr ? name : ""));
     if (size != nullptr) *size = static_cast<int64_t>(sz);
@@ -442,10 +442,10 @@ extern "C" cuvsError_t octexIndexPlanInfo(cuvsOctexIndex_t index, int32_t* info)
   return translate_exceptions([=] {
     auto& ix = as_index(*index)->impl();
     std::lock_guard<std::mutex> lock(ix.mu);
-    OCTEX_EXPECTS(!ix.plans.empty(), "octex: no search ran on this index yet");
-    auto const& pl = *ix.plans.begin()->second;
-    auto const& sh = pl.shape;
-    int32_t v[] = {sh.m, sh.k, sh.KO, sh.lr, sh.W, sh.W2, sh.R1, sh.R2, sh.FR, pl.graph != nullptr ? 1 : 0};
+    const auto pl = octex::detail::shown_plan(ix);
+    OCTEX_EXPECTS(pl != nullptr, "octex: no search ran on this index yet");
+    auto const& sh = pl->shape;
+    int32_t v[] = {sh.m, sh.k, sh.KO, sh.lr, sh.W, sh.W2, sh.R1, sh.R2, sh.FR, pl->graph != nullptr ? 1 : 0};
     std::memcpy(info, v, sizeof(v));
   });
 }

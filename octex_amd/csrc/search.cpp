@@ -26,12 +26,14 @@ namespace detail {
 index_impl::~index_impl()
 {
   plans.clear();
+  captured.clear();
   if (stream != nullptr) {
     (void)hipSetDevice(device);
     (void)hipStreamSynchronize(stream);
     (void)hipStreamDestroy(stream);
   }
   if (searched != nullptr) (void)hipEventDestroy(searched);
+  if (capture_end != nullptr) (void)hipEventDestroy(capture_end);
 }
 
 void index_impl::drain()
@@ -385,6 +387,12 @@ auto get_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::sha
   return pl;
 }
 
+auto shown_plan(index_impl& ix) -> std::shared_ptr<plan>
+{
+  auto const& from = !ix.plans.empty() ? ix.plans : ix.captured;
+  return from.empty() ? nullptr : from.begin()->second;
+}
+
 void run_batch(index_impl const& ix, plan const& pl, batch_io const& io, hipStream_t s)
 {
   if (pl.graph == nullptr) {
@@ -410,6 +418,78 @@ auto on_device(const void* p, int device) -> bool
   return a.type == hipMemoryTypeDevice && a.device == device;
 }
 
+/**
+ * The plan of a search under stream capture.  A capture permits no allocation, so an earlier search with the same
+ * parameters and number of queries must have made the plan.  Its first captured search takes it out of the cache: the
+ * captured graph's replays, which no event of the index covers, use its buffers.
+ */
+auto captured_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>
+{
+  const std::string key = plan_key(sp, m, k);
+  std::lock_guard<std::mutex> lock(ix.mu);
+  auto kept = ix.captured.find(key);
+  if (kept != ix.captured.end()) return kept->second;
+  auto it = ix.plans.find(key);
+  OCTEX_EXPECTS(it != ix.plans.end(),
+                "octex: a search under stream capture needs the buffers of an earlier search with the same parameters, k "
+                "and number of queries: run it once before the capture, or capture octexSearchNoAlloc");
+  auto pl = it->second;
+  ix.captured.emplace(key, pl);
+  ix.plans.erase(it);
+  return pl;
+}
+
+/** The search's batches on stream s, by the plan's graph or (direct) its kernels; resident as search_impl. */
+void run_batches(index_impl const& ix, plan const& pl, const float* queries, int64_t nq, int64_t* neighbors,
+                 float* distances, int64_t k, bool host_out, bool resident, bool direct, hipStream_t s)
+{
+  auto const& b   = pl.buf;
+  const int64_t D = ix.dim;
+  const int m     = pl.shape.m;
+  // queries and results in the GPU's own memory are read and written in place by the batch's first and last kernel;
+  // others are copied (each copy and its gap about 10 us of a small search)
+  const bool in_place  = !resident && !host_out && on_device(queries, ix.device);
+  const bool out_place = !resident && !host_out && on_device(neighbors, ix.device) && on_device(distances, ix.device);
+  for (int64_t b0 = 0; b0 < nq; b0 += m) {
+    const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
+    batch_io io;
+    io.n = n;
+    if (in_place) io.queries = queries + b0 * D;
+    if (out_place) {
+      io.neighbors = neighbors + b0 * k;
+      io.distances = distances + b0 * k;
+    }
+    if (!resident && !in_place)
+      OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, s));
+    if (direct)
+      launch_batch(ix, pl.shape, b, io, s);
+    else
+      run_batch(ix, pl, io, s);
+    if (!resident && !out_place) {
+      OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, s));
+      OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, s));
+    }
+  }
+}
+
+/**
+ * A search whose stream is being captured (stream_mu held): its kernels themselves enter the graph, since a plan's graph
+ * launched here would run once, now, and not in the replays.  Nothing waits for or records the index's events, which lie
+ * outside the capture; searches of one capture, on whatever streams, run one after another, as they share the plans.
+ */
+void search_captured(index_impl& ix, plan const& pl, const float* queries, int64_t nq, int64_t* neighbors,
+                     float* distances, int64_t k, hipStream_t s)
+{
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  unsigned long long id     = 0;
+  OCTEX_HIP(hipStreamGetCaptureInfo(s, &st, &id));
+  if (ix.capture_end == nullptr) OCTEX_HIP(hipEventCreateWithFlags(&ix.capture_end, hipEventDisableTiming));
+  else if (ix.capture_id == id) OCTEX_HIP(hipStreamWaitEvent(s, ix.capture_end, 0));
+  run_batches(ix, pl, queries, nq, neighbors, distances, k, false, false, true, s);
+  OCTEX_HIP(hipEventRecord(ix.capture_end, s));
+  ix.capture_id = id;
+}
+
 }  // namespace
 
 void search_impl(raft::resources const& res, search_params const& sp, index const& idx, const float* queries,
@@ -425,64 +505,48 @@ void search_impl(raft::resources const& res, search_params const& sp, index cons
   OCTEX_HIP(hipSetDevice(ix.device));
   const int m = static_cast<int>(std::min<int64_t>(std::max(sp.batch, 1), nq));
   std::unique_lock<std::mutex> run(ix.stream_mu);
-  if (ix.searched == nullptr)
-    OCTEX_HIP(hipEventCreateWithFlags(&ix.searched, hipEventDisableTiming | hipEventDisableSystemFence));
-  auto pl = get_plan(ix, sp, m, static_cast<int>(k));  // released before `run` on every path
-  auto const& b    = pl->buf;
-  const int64_t D  = ix.dim;
-  hipStream_t call = raft::resource::get_cuda_stream(res);
   // the batches run on the caller's stream itself, after the previous search of the index (its plan buffers may be the
   // same), which may have run on another stream.  A hop to the index's stream and back, two events and two waits, took
   // 38 us of a search of one query
-  hipStream_t s = call;
+  hipStream_t call = raft::resource::get_cuda_stream(res);
+  hipStream_t s    = call;
   if (call != nullptr) {
     int at = ix.device;
     OCTEX_HIP(hipStreamGetDevice(call, &at));
     OCTEX_EXPECTS(at == ix.device, "octex: the search's stream is on device %d, the index on device %d", at, ix.device);
-  } else {
-    // the null stream takes no launch while any blocking stream of the process is captured: the index's stream does
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    const hipError_t e        = hipStreamIsCapturing(call, &st);
-    if (e == hipErrorStreamCaptureImplicit) {
-      (void)hipGetLastError();
-      s = ix.stream;
-    } else {
-      OCTEX_HIP(e);
-    }
   }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const hipError_t e        = hipStreamIsCapturing(call, &st);
+  if (call == nullptr && e == hipErrorStreamCaptureImplicit) {
+    // the null stream takes no launch while any blocking stream of the process is captured: the index's stream does
+    (void)hipGetLastError();
+    s = ix.stream;
+  } else {
+    OCTEX_HIP(e);
+  }
+  if (st != hipStreamCaptureStatusNone) {
+    OCTEX_EXPECTS(!host_out && !resident, "octex: a search under stream capture takes device tensors");
+    auto pl = captured_plan(ix, sp, m, static_cast<int>(k));
+    search_captured(ix, *pl, queries, nq, neighbors, distances, k, call);
+    OCTEX_HIP(hipSetDevice(cur));
+    return;
+  }
+  if (ix.searched == nullptr)
+    OCTEX_HIP(hipEventCreateWithFlags(&ix.searched, hipEventDisableTiming | hipEventDisableSystemFence));
+  auto pl = get_plan(ix, sp, m, static_cast<int>(k));  // released before `run` on every path
   OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));
   if (s != call) {
     OCTEX_HIP(hipEventRecord(ix.searched, call));
     OCTEX_HIP(hipStreamWaitEvent(s, ix.searched, 0));
   }
-  // queries and results in the GPU's own memory are read and written in place by the batch's first and last kernel;
-  // others are copied (each copy and its gap about 10 us of a small search)
-  const bool in_place  = !resident && !host_out && on_device(queries, ix.device);
-  const bool out_place = !resident && !host_out && on_device(neighbors, ix.device) && on_device(distances, ix.device);
   auto mark = [&] {  // the event the next search, and whoever frees or reads the buffers, waits for
-    const hipError_t e = hipEventRecord(ix.searched, s);
-    if (e == hipSuccess) return;
+    const hipError_t err = hipEventRecord(ix.searched, s);
+    if (err == hipSuccess) return;
     (void)hipStreamSynchronize(s);  // no event stands for the batches: they end before the lock is given up
-    OCTEX_HIP(e);
+    OCTEX_HIP(err);
   };
   try {
-    for (int64_t b0 = 0; b0 < nq; b0 += m) {
-      const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
-      batch_io io;
-      io.n = n;
-      if (in_place) io.queries = queries + b0 * D;
-      if (out_place) {
-        io.neighbors = neighbors + b0 * k;
-        io.distances = distances + b0 * k;
-      }
-      if (!resident && !in_place)
-        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, s));
-      run_batch(ix, *pl, io, s);
-      if (!resident && !out_place) {
-        OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, s));
-        OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, s));
-      }
-    }
+    run_batches(ix, *pl, queries, nq, neighbors, distances, k, host_out, resident, false, s);
   } catch (...) {
     try {
       mark();

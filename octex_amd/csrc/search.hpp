@@ -91,6 +91,8 @@ struct plan {
 
 auto plan_key(search_params const& sp, int m, int k) -> std::string;
 auto get_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>;
+/** The cached plan or, when a capture took it out of the cache, a captured one; null before any search (ix.mu held). */
+auto shown_plan(index_impl& ix) -> std::shared_ptr<plan>;
 /** Where a batch's n queries come from and its results go: device memory of the index's GPU that the batch's first and
  * last kernel read and write in place.  Null queries: the plan's qbuf; null results: only bi / bd. */
 struct batch_io {

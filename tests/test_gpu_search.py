@@ -429,6 +429,79 @@ def test_null_stream_search_while_a_blocking_stream_is_captured(octex, small_ind
         assert np.array_equal(D0, np.asarray(torch.as_tensor(D).cpu()))
 
 
+def search_into(index, q, I, D, stream, **params):
+    """cuvsOctexSearch of device queries on `stream` into I and D."""
+    from octex_amd import _lib
+    from octex_amd import index as octex_index
+
+    res = _lib.Resources(stream=stream.cuda_stream)
+    tensors = [_lib.Dl(t) for t in (q, I, D)]
+    _lib.call("cuvsOctexSearch", res.h, ct.byref(octex_index.search_params(**params)), index.handle,
+              *(t.ptr for t in tensors))
+
+
+@pytest.mark.parametrize("extra", [dict(use_graph=False), dict(use_graph=True), dict(batch=17),
+                                   dict(sketch_rank=True, final_rerank=32), dict(waves=0)])
+def test_captured_search_replays(octex, small_index, extra):
+    """Two searches captured into one graph, on the captured stream and on one forked from it: every replay gives the
+    eager results of the queries then in place, beside eager searches of the same shape on another stream and after a
+    plan of another shape replaced the cached one."""
+    index = octex.load(small_index["path"])
+    params = dict(PARAMS, **extra)
+    Q = small_index["Q"][:40]
+    q, side, fork = [torch.from_numpy(Q).cuda() for _ in range(2)], torch.cuda.Stream(), torch.cuda.Stream()
+    I = [torch.full((40, 10), -7, dtype=torch.int64, device="cuda") for _ in range(2)]
+    D = [torch.full((40, 10), float("nan"), device="cuda") for _ in range(2)]
+    index.search(q[0], k=10, **params)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        fork.wait_stream(side)
+        search_into(index, q[0], I[0], D[0], side, **params)
+        search_into(index, q[1], I[1], D[1], fork, **params)
+        side.wait_stream(fork)
+    assert index.plan_info()["m"] == min(40, params.get("batch", 40))  # the captured plan's
+    torch.cuda.synchronize()
+    g = np.random.default_rng(1)
+    for rep in range(4):
+        Qr = [np.ascontiguousarray(Q[g.permutation(40)]) for _ in range(2)]
+        want = [index.search(x, k=10, **params) for x in Qr]
+        for t, x in zip(q, Qr):
+            t.copy_(torch.from_numpy(x))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            graph.replay()
+        Ds, Is = index.search(q[0], k=10, **params)  # on the null stream, beside the replay
+        index.search(Q[:7], k=5, **PARAMS)           # another plan takes its place in the cache
+        torch.cuda.synchronize()
+        print(f"replay {rep}", flush=True)
+        for (Dw, Iw), Dg, Ig in zip(want + want[:1], D + [Ds], I + [Is]):
+            assert np.array_equal(Iw, Ig.cpu().numpy()) and np.array_equal(Dw, Dg.cpu().numpy())
+
+
+def test_captured_search_without_an_earlier_one(octex, small_index):
+    """A capture allocates nothing: without an earlier search of the same shape it is refused before anything is
+    enqueued, the capture ends well, and searches go on."""
+    from octex_amd._lib import OctexError
+
+    index = octex.load(small_index["path"])
+    Q = small_index["Q"][:40]
+    want = index.search(Q, k=10, **PARAMS)
+    q, side = torch.from_numpy(Q[:39]).cuda(), torch.cuda.Stream()
+    I, D = torch.zeros((39, 10), dtype=torch.int64, device="cuda"), torch.ones((39, 10), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        D.mul_(2)
+        with pytest.raises(OctexError, match="run it once before the capture, or capture octexSearchNoAlloc"):
+            search_into(index, q, I, D, side, **PARAMS)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert (D == 2).all()
+    D1, I1 = index.search(Q, k=10, **PARAMS)
+    assert np.array_equal(I1, want[1]) and np.array_equal(D1, want[0])
+
+
 def test_search_after_a_failed_allocation(octex, small_index):
     """A search whose batch buffers do not fit the GPU is an error, and the next search runs: the failed call's error does
     not stay behind for the next launch's check."""
