@@ -38,8 +38,10 @@ index_impl::~index_impl()
 
 void index_impl::drain()
 {
+  // by way of the stream: the event is made without a system fence, so waiting for it on the host would not make what
+  // the search wrote visible to the host and to copies
+  if (searched != nullptr) OCTEX_HIP(hipStreamWaitEvent(stream, searched, 0));
   OCTEX_HIP(hipStreamSynchronize(stream));
-  if (searched != nullptr) OCTEX_HIP(hipEventSynchronize(searched));
 }
 
 plan::~plan()

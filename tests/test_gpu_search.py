@@ -502,6 +502,22 @@ def test_captured_search_without_an_earlier_one(octex, small_index):
     assert np.array_equal(I1, want[1]) and np.array_equal(D1, want[0])
 
 
+def test_plan_buffers_read_behind_a_running_search(octex, small_index):
+    """A plan buffer copied to the host while a search on another stream still runs holds that search's results."""
+    index = octex.load(small_index["path"])
+    Q = np.concatenate([small_index["Q"]] * 40)
+    q, side = torch.from_numpy(Q).cuda(), torch.cuda.Stream()
+    g = torch.Generator().manual_seed(0)
+    for _ in range(5):
+        q.copy_(q[torch.randperm(len(q), generator=g).cuda()])
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            D, I = index.search(q, k=10, **PARAMS)
+        bi, bd = index.plan_buffer("bi", np.int64), index.plan_buffer("bd", np.float32)
+        torch.cuda.synchronize()
+        assert np.array_equal(bi, I.cpu().numpy().ravel()) and np.array_equal(bd, D.cpu().numpy().ravel())
+
+
 def test_search_after_a_failed_allocation(octex, small_index):
     """A search whose batch buffers do not fit the GPU is an error, and the next search runs: the failed call's error does
     not stay behind for the next launch's check."""
