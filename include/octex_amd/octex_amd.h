@@ -104,7 +104,8 @@ cuvsError_t octexIndexCheckDirectory(const char* path, cuvsOctexLoadParams_t par
  * row major) with every per-batch buffer in a file-scope device array of 256 MiB that each GPU holds until the
  * process ends, instead of a cached plan's allocations; the batch's kernels run directly on `stream` (a
  * hipStream_t, NULL the null stream; no graph) and write neighbors [nq, k] (int64) and distances [nq, k] (float32),
- * device memory, ordered on that stream.  The queries are split into batches of min(params->batch, nq); a batch
+ * device memory, ordered on that stream.  Arrays in the memory of the index's GPU are read and written in place; others
+ * (another GPU's memory, host memory) are copied on that stream.  The queries are split into batches of min(params->batch, nq); a batch
  * whose buffers exceed 256 MiB is an error that names the bytes it needs (lower params->batch).  No call allocates
  * or frees device memory.  Every call on one GPU shares that GPU's array: calls that overlap on one GPU (other
  * streams or threads) race, and the index must not change while one runs.

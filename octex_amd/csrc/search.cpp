@@ -407,9 +407,6 @@ void run_batch(index_impl const& ix, plan const& pl, batch_io const& io, hipStre
   stages.back().launch();
 }
 
-namespace {
-
-/** p lies in the memory of `device`, where the index's kernels read and write it in place. */
 auto on_device(const void* p, int device) -> bool
 {
   hipPointerAttribute_t a{};
@@ -419,6 +416,8 @@ auto on_device(const void* p, int device) -> bool
   }
   return a.type == hipMemoryTypeDevice && a.device == device;
 }
+
+namespace {
 
 /**
  * The plan of a search under stream capture.  A capture permits no allocation, so an earlier search with the same

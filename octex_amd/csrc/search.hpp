@@ -93,6 +93,8 @@ auto plan_key(search_params const& sp, int m, int k) -> std::string;
 auto get_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>;
 /** The cached plan or, when a capture took it out of the cache, a captured one; null before any search (ix.mu held). */
 auto shown_plan(index_impl& ix) -> std::shared_ptr<plan>;
+/** p lies in the memory of `device`, where the index's kernels read and write it in place. */
+auto on_device(const void* p, int device) -> bool;
 /** Where a batch's n queries come from and its results go: device memory of the index's GPU that the batch's first and
  * last kernel read and write in place.  Null queries: the plan's qbuf; null results: only bi / bd. */
 struct batch_io {
@@ -117,9 +119,9 @@ struct profile_counters {
 void profile_batch(index_impl& ix, plan& pl, int reps, std::vector<std::string>& names, std::vector<double>& ms,
                    profile_counters& cnt);
 /**
- * The search of device queries [nq, dim] into device neighbors / distances [nq, k] on stream s with every batch
- * buffer in the library's file-scope scratch array of the index's GPU (search_noalloc.cpp): no device allocation,
- * direct launches, no graph.  A batch whose buffers exceed the array is an error.
+ * The search of queries [nq, dim] into neighbors / distances [nq, k] on stream s with every batch buffer in the
+ * library's file-scope scratch array of the index's GPU (search_noalloc.cpp): no device allocation, direct launches, no
+ * graph.  Arrays outside that GPU's memory are copied.  A batch whose buffers exceed the array is an error.
  */
 void search_no_alloc(search_params const& sp, index const& idx, const float* queries, int64_t nq, int64_t dim,
                      int64_t k, int64_t* neighbors, float* distances, hipStream_t s);

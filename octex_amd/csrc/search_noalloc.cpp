@@ -69,14 +69,27 @@ void search_no_alloc(search_params const& sp, index const& idx, const float* que
     batch_buffers b;
     carve_buffers(ix, sh, scratch_on(ix.device), &b);
     const int64_t D = ix.dim;
+    // the index's GPU's own memory is read and written in place, any other (another GPU's, host memory) is copied: the
+    // kernels cannot be trusted to reach it
+    const bool in_place  = on_device(queries, ix.device);
+    const bool out_place = on_device(neighbors, ix.device) && on_device(distances, ix.device);
     for (int64_t b0 = 0; b0 < nq; b0 += m) {
       const int n = static_cast<int>(std::min<int64_t>(m, nq - b0));
-      batch_io io;  // device pointers: read and written in place
-      io.queries   = queries + b0 * D;
-      io.neighbors = neighbors + b0 * k;
-      io.distances = distances + b0 * k;
-      io.n         = n;
+      batch_io io;
+      io.n = n;
+      if (in_place)
+        io.queries = queries + b0 * D;
+      else
+        OCTEX_HIP(hipMemcpyAsync(b.qbuf, queries + b0 * D, sizeof(float) * n * D, hipMemcpyDefault, s));
+      if (out_place) {
+        io.neighbors = neighbors + b0 * k;
+        io.distances = distances + b0 * k;
+      }
       launch_batch(ix, sh, b, io, s);
+      if (!out_place) {
+        OCTEX_HIP(hipMemcpyAsync(neighbors + b0 * k, b.bi, sizeof(int64_t) * n * k, hipMemcpyDefault, s));
+        OCTEX_HIP(hipMemcpyAsync(distances + b0 * k, b.bd, sizeof(float) * n * k, hipMemcpyDefault, s));
+      }
     }
   } catch (...) {
     (void)hipSetDevice(cur);

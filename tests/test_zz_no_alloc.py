@@ -61,6 +61,24 @@ def test_no_alloc_equals_search(octex, small_index, extra):
         assert np.array_equal(I, Ir) and np.array_equal(D, Dr)
 
 
+@pytest.mark.parametrize("pinned", [True, False])
+def test_no_alloc_copies_arrays_outside_the_gpu(octex, small_index, pinned):
+    """Queries and results that do not lie in the index's GPU's memory are copied in and out, each on its own, with
+    several batches and a partial last one."""
+    index = octex.load(small_index["path"])
+    Q = np.ascontiguousarray(small_index["Q"][:90])
+    Dr, Ir = index.search(Q, k=10, **PARAMS)
+    for hosts in ((True, True), (True, False), (False, True)):  # queries, results
+        q = torch.from_numpy(Q)
+        I, D = torch.full((90, 10), -7, dtype=torch.int64), torch.full((90, 10), float("nan"))
+        q, I, D = (t if h and not pinned else t.pin_memory() if h else t.cuda()
+                   for t, h in ((q, hosts[0]), (I, hosts[1]), (D, hosts[1])))
+        print(f"no-alloc search, host queries / results {hosts}, pinned {pinned}", flush=True)
+        call_no_alloc(index, q, I, D, **dict(PARAMS, batch=37))
+        torch.cuda.synchronize()
+        assert np.array_equal(I.cpu().numpy(), Ir) and np.array_equal(D.cpu().numpy(), Dr)
+
+
 def test_no_alloc_refuses_a_batch_beyond_the_scratch(octex, small_index):
     from octex_amd._lib import OctexError
 
