@@ -186,6 +186,11 @@ cuvsError_t octexStageFinalRerank(const int64_t* si, int32_t m, int32_t KO, int3
 /** take_k_kernel (search_kernels.cuh:672-685). */
 cuvsError_t octexStageTakeK(const int64_t* si, const float* sd, int32_t m, int32_t KO, int32_t k, int64_t* bi,
                             float* bd, void* stream);
+/** The builder's merge of reverse edges (build_table.cuh:157-252): table [n, kout] of the forward rows fwd [n, kin],
+ * their first kf entries, up to kr reverse entries (of the rows' first ks entries), then the others; with fdist
+ * [n, kin] (may be NULL) the kept entries nearest first. */
+cuvsError_t octexStageMergeReverse(const int32_t* fwd, const float* fdist, int64_t n, int32_t kin, int32_t kf,
+                                   int32_t ks, int32_t kr, int32_t kout, int32_t* table, void* stream);
 
 #ifdef __cplusplus
 }

@@ -486,13 +486,14 @@ void set_device_table(index_impl& ix, dbuf&& rows, int k)
   ix.table_len = k;
 }
 
-/** The forward rows and their merge stay on the GPU while they take at most half of its free memory (OCTEX_MERGE_HOST=1:
- * they do not; the same rows).  Measured for 250k
+/** The forward rows and their merge stay on the GPU while they take at most half of its free memory and the merge takes
+ * their number (OCTEX_MERGE_HOST=1: they do not; the same rows).  Measured for 250k
  * rows of 96 forward entries: a search pass and its merge 20 ms, with the merge on 16 host threads 125 ms. */
 auto merge_on_device(int64_t n, reverse_rule const& rr) -> bool
 {
   const char* host = std::getenv("OCTEX_MERGE_HOST");
   if (host != nullptr && std::atoi(host) != 0) return false;
+  if (n * rr.ks >= kMergeEntries) return false;
   size_t fr = 0, tot = 0;
   OCTEX_HIP(hipMemGetInfo(&fr, &tot));
   return merge_reverse_bytes(n, rr) + static_cast<size_t>(n) * (8 * rr.kin + 4 * rr.kout) <= fr / 2;

@@ -1209,22 +1209,22 @@ __global__ __launch_bounds__(256) void reverse_keys_kernel(const int* __restrict
 }
 
 /**
- * The merged row of u = blockIdx.x by one wavefront: the row's candidates in the rule's order in LDS (at most kin + kr),
+ * The merged row of u = u0 + blockIdx.x by one wavefront: the row's candidates in the rule's order in LDS (at most kin + kr),
  * an entry dropped when an earlier one holds its id (all pairs, the earlier ids by broadcast reads: 144 candidates of a
  * table of 64 take 3 x 144 steps), the rest numbered by ballots.  (key, val): the sorted reverse entries, total of them;
  * the row's are found by binary search.
  */
 __global__ __launch_bounds__(64) void merge_rows_kernel(const int* __restrict__ fwd, const float* __restrict__ fdist,
                                                         const unsigned long long* __restrict__ key,
-                                                        const int* __restrict__ val, int64_t total, reverse_rule rr,
-                                                        int* __restrict__ table)
+                                                        const int* __restrict__ val, int64_t total, int64_t u0,
+                                                        reverse_rule rr, int* __restrict__ table)
 {
   extern __shared__ int rows_lds[];
   const int cap = rr.kin + rr.kr;
   int* id       = rows_lds;                                  // [cap]
   float* dist   = reinterpret_cast<float*>(id + cap);        // [cap], with fdist
   auto* kept    = reinterpret_cast<unsigned long long*>(dist + cap);  // [kout], with fdist (2 cap words before it)
-  const int64_t u = blockIdx.x;
+  const int64_t u = u0 + blockIdx.x;
   const int lane  = threadIdx.x;
   int64_t lo = 0, hi = total;  // lanes 0 and 1: the first entry of rows u and u + 1
   const unsigned long long want = static_cast<unsigned long long>(u + (lane & 1)) << 8;
@@ -1324,7 +1324,8 @@ void merge_reverse_device(const int* fwd, const float* fdist, int64_t n, reverse
 {
   OCTEX_EXPECTS(rr.ks >= 1 && rr.ks <= 256 && rr.ks <= rr.kin && rr.kf <= rr.kin && rr.kr >= 0 && rr.kout >= 1,
                 "octex: the reverse-edge merge takes forward rows of at most 256 entries");
-  OCTEX_EXPECTS(merge_rows_lds(rr) <= 64 * 1024 && n < (int64_t{1} << 31), "octex: reverse-edge rows too long");
+  OCTEX_EXPECTS(merge_rows_lds(rr) <= 64 * 1024, "octex: reverse-edge rows too long");
+  OCTEX_EXPECTS(n * rr.ks < kMergeEntries, "octex: the reverse-edge merge on the GPU takes fewer than 2^31 entries");
   const int64_t total = n * rr.ks;
   dbuf key(static_cast<size_t>(total) * 8), skey(static_cast<size_t>(total) * 8), val(static_cast<size_t>(total) * 4),
     sval(static_cast<size_t>(total) * 4), tmp;
@@ -1334,9 +1335,12 @@ void merge_reverse_device(const int* fwd, const float* fdist, int64_t n, reverse
     return rocprim::radix_sort_pairs(p, b, key.as<unsigned long long>(), skey.as<unsigned long long>(), val.as<int>(),
                                      sval.as<int>(), static_cast<size_t>(total), 0, 8 + log2_ceil(n + 1), s);
   });
-  merge_rows_kernel<<<static_cast<unsigned>(n), 64, merge_rows_lds(rr), s>>>(fwd, fdist, skey.as<unsigned long long>(),
-                                                                            sval.as<int>(), total, rr, table);
-  OCTEX_HIP(hipGetLastError());
+  constexpr int64_t kPiece = int64_t{1} << 24;  // a launch covers fewer than 2^32 work-items, 64 a row
+  for (int64_t u0 = 0; u0 < n; u0 += kPiece) {
+    merge_rows_kernel<<<static_cast<unsigned>(std::min(kPiece, n - u0)), 64, merge_rows_lds(rr), s>>>(
+      fwd, fdist, skey.as<unsigned long long>(), sval.as<int>(), total, u0, rr, table);
+    OCTEX_HIP(hipGetLastError());
+  }
   OCTEX_HIP(hipStreamSynchronize(s));
 }
 

@@ -55,6 +55,8 @@ void make_sketch(row_source& x, int64_t n, int d, const float* mean, const float
 struct reverse_rule {
   int kin, kf, ks, kr, kout;
 };
+/** Reverse entries (n ks) below which the GPU merges: their numbers and a launch over them stay inside 32 bits. */
+constexpr int64_t kMergeEntries = int64_t{1} << 31;
 /** Device bytes of merge_reverse_device over n rows, beside its inputs and its table. */
 auto merge_reverse_bytes(int64_t n, reverse_rule const& rr) -> size_t;
 /** The table rows [n, kout] of the forward rows fwd [n, kin] with their reverse edges by the rule, -1 padded; with fdist

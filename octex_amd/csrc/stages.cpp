@@ -1,6 +1,7 @@
 // Stage entry points: one search kernel per call on caller-provided device buffers (for the parity
 // tests; see octex_amd/octex_amd.h).  Each call checks its arguments, launches, and waits.
 
+#include "build_kernels.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -248,5 +249,16 @@ extern "C" cuvsError_t octexStageTakeK(const int64_t* si, const float* sd, int32
     OCTEX_EXPECTS(k <= KO, "octex: k <= KO");
     launch_take_k(reinterpret_cast<const long long*>(si), sd, m, KO, k, reinterpret_cast<long long*>(bi), bd,
                   result_rows{}, s);
+  });
+}
+
+extern "C" cuvsError_t octexStageMergeReverse(const int32_t* fwd, const float* fdist, int64_t n, int32_t kin,
+                                              int32_t kf, int32_t ks, int32_t kr, int32_t kout, int32_t* table,
+                                              void* stream)
+{
+  return run(stream, [&](hipStream_t s) {
+    need(fwd, "fwd"), need(table, "table");
+    OCTEX_EXPECTS(n >= 1, "octex: reverse edges of at least one row");
+    merge_reverse_device(fwd, fdist, n, reverse_rule{kin, kf, ks, kr, kout}, table, s);
   });
 }

@@ -789,3 +789,20 @@ def test_selection_of_many_equal_keys_at_the_largest_width(L, ix, dix, small_ind
     for q in range(m):
         ri, rd = O.rerank_keep(ix, cand[q, : nin[q]], dist[q, : nin[q]], Q[q], R, si[q], sd[q], True)
         assert np.array_equal(host(dsi)[q], ri) and np.array_equal(host(dsd)[q], rd), f"rerank_keep query {q}"
+
+
+# ---------------------------------------------------------------- the builder's stages
+
+
+@pytest.mark.parametrize("n", [2, (1 << 24) + 1, (1 << 26) + 3])
+def test_reverse_edge_merge_of_many_rows(L, n):
+    """Rows u -> u + 1 merged with their reverse edges: [u + 1, u - 1], on either side of a launch's rows and past the
+    2^26 rows whose 64 work-items each no longer fit one launch."""
+    fwd = torch.arange(1, n + 1, dtype=torch.int32, device="cuda").remainder_(n)
+    table = torch.full((n, 2), -7, dtype=torch.int32, device="cuda")
+    print(f"merge of {n} rows", flush=True)
+    L.call("octexStageMergeReverse", P(fwd), None, i64(n), i32(1), i32(1), i32(1), i32(1), i32(2), P(table), None)
+    back = torch.arange(n - 1, 2 * n - 1, dtype=torch.int64, device="cuda").remainder_(n).int()
+    if n == 2:
+        back.fill_(-1)  # the same row twice
+    assert torch.equal(table[:, 0], fwd) and torch.equal(table[:, 1], back)
