@@ -598,10 +598,9 @@ __device__ __forceinline__ float group_sum(float x)
   return x;
 }
 
-constexpr int kChunkPitch = 18;  // float2 words of a chunk of 16 coordinates in LDS: two chunks start in other banks
-
-/** LDS words (float2) of the scales and the query sketch of S coordinates. */
-__host__ __device__ constexpr auto sketch_lds_words(int S) -> int { return S / 16 * kChunkPitch; }
+// float2 words from one chunk of 16 coordinates to the next in LDS: two chunks start in other banks, or lie side by side
+// where the slot list is in global memory and the padding does not fit (gather_impl)
+constexpr int kChunkPitch = 18, kTightPitch = 16;
 
 /**
  * Sketch scores of a query's candidates 0..n-1 (search_kernels.cuh:227-251): with LR = the next power of two >= S / 16
@@ -618,12 +617,12 @@ __host__ __device__ constexpr auto sketch_lds_words(int S) -> int { return S / 1
  * table entries (S = 96) 108, 190 and 104 -> 79, 143 and 77 us on unchanged threads, of one query 23, 30, 20 -> 15, 23,
  * 15 us; 10,000 queries of 4096 table entries over 1.5M rows 552 -> 528 us (45 G rows/s: the random-row ceiling).  The scales and the
  * query's sketch come from LDS (the same 16 bytes for every lane of a chunk, once for kRows rows); sq holds (scale, -qs),
- * a chunk every kChunkPitch.  All loads of kRows rows are issued before the first is used, unconditionally
+ * a chunk every chunk_pitch.  All loads of kRows rows are issued before the first is used, unconditionally
  * (past-the-end candidates read row 0, a chunk past S the row's first).
  */
 template <int LR, int NJ, typename IdOf, typename Put>
 __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const signed char* __restrict__ code, int S,
-                                              int pitch, const float2* sq, Put const& put)
+                                              int pitch, const float2* sq, int chunk_pitch, Put const& put)
 {
   constexpr int J     = LR < 4 ? LR : 4;  // chunks of a lane in the butterfly
   constexpr int G     = LR / J;           // lanes per candidate
@@ -676,7 +675,7 @@ __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const si
     const float4_t* coef[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++)
-      coef[j] = reinterpret_cast<const float4_t*>(sq + at + (j + 1 < NJ || has_last ? sub + G * j : 0) * kChunkPitch);
+      coef[j] = reinterpret_cast<const float4_t*>(sq + at + (j + 1 < NJ || has_last ? sub + G * j : 0) * chunk_pitch);
     float4_t next[2] = {coef[0][0], coef[0][1]};  // (scale, -qs) of two coordinates each
 #pragma unroll
     for (int p = 0; p < 4 * NJ; p++) {
@@ -1423,21 +1422,22 @@ template <bool kRows, int LR, int NJ, int NT, bool kLdsSlots, bool kBalanced>
 __global__ __launch_bounds__(NT) void gather_kernel(
   const int2* __restrict__ seg, int nseg, const long long* __restrict__ list_ptr,
   const int* __restrict__ table, int table_len, int64_t N, const signed char* __restrict__ code,
-  const float* __restrict__ scale, const float* __restrict__ qs, int S, int pitch, int W, int logW, int cap,
+  const float* __restrict__ scale, const float* __restrict__ qs, int S, int pitch, int W, int logW, int cap, int tight,
   int* __restrict__ cand, float* __restrict__ dist, int* __restrict__ nout, earlier_rows er, int* __restrict__ nknown)
 {
-  const int q = blockIdx.x;
+  const int q  = blockIdx.x;
+  const int cp = !kLdsSlots && tight ? kTightPitch : kChunkPitch;
   extern __shared__ int4 smq[];
   int* ht        = reinterpret_cast<int*>(smq);         // [W] hash set (16-byte aligned)
-  float2* sq     = reinterpret_cast<float2*>(ht + W);   // (scale, -query sketch), kChunkPitch a chunk (16-byte aligned)
-  const int** sp = reinterpret_cast<const int**>(sq + sketch_lds_words(S));  // [nseg] first entry of a segment
+  float2* sq     = reinterpret_cast<float2*>(ht + W);   // (scale, -query sketch), cp a chunk (16-byte aligned)
+  const int** sp = reinterpret_cast<const int**>(sq + S / 16 * cp);  // [nseg] first entry of a segment
   int* pre       = reinterpret_cast<int*>(sp + nseg);   // [nseg] exclusive prefix of the compacted lengths
   auto* cl       = reinterpret_cast<unsigned short*>(pre + nseg);  // [cap] slots of the candidates (kLdsSlots)
   __shared__ collect_state cs;
   int* crow   = cand + static_cast<int64_t>(q) * W;
   float* drow = dist + static_cast<int64_t>(q) * W;
   for (int i = threadIdx.x; i < S; i += blockDim.x)
-    sq[i / 16 * kChunkPitch + i % 16] = make_float2(scale[i], -qs[static_cast<int64_t>(q) * S + i]);
+    sq[i / 16 * cp + i % 16] = make_float2(scale[i], -qs[static_cast<int64_t>(q) * S + i]);
   auto keep_slot = [&](int slot, int, unsigned h) {
     if constexpr (kLdsSlots)
       cl[slot] = static_cast<unsigned short>(h);
@@ -1478,7 +1478,7 @@ __global__ __launch_bounds__(NT) void gather_kernel(
       else
         return ht[crow[j] & (W - 1)];  // a slot (< W), or an id when another group has scored j: kept inside ht
     },
-    code, S, pitch, sq,
+    code, S, pitch, sq, cp,
     [&](int j, int id, float d) {
       crow[j] = id;
       drow[j] = d;
@@ -2531,9 +2531,10 @@ auto gather_cap(int W, int nseg, int max_len) -> int
   return static_cast<int>(std::min<int64_t>(W, static_cast<int64_t>(nseg) * std::max(max_len, 1)));
 }
 
-auto gather_smem(int W, int S, int nseg, int max_len, bool lds_slots) -> size_t
+auto gather_smem(int W, int S, int nseg, int max_len, bool lds_slots, bool tight) -> size_t
 {
-  return static_cast<size_t>(nseg) * sizeof(long long) + static_cast<size_t>(W + 2 * sketch_lds_words(S) + nseg) * sizeof(int) +
+  const int cp = !lds_slots && tight ? kTightPitch : kChunkPitch;
+  return static_cast<size_t>(nseg) * sizeof(long long) + static_cast<size_t>(W + 2 * (S / 16 * cp) + nseg) * sizeof(int) +
          (lds_slots ? static_cast<size_t>(gather_cap(W, nseg, max_len)) * sizeof(unsigned short) : 0);
 }
 
@@ -2553,8 +2554,9 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
   OCTEX_EXPECTS(max_len >= 0, "octex: segment lengths are non-negative");
   OCTEX_EXPECTS(W == (1 << logW) && W <= kMaxHash, "octex: hash set size");
   OCTEX_EXPECTS(S % 16 == 0 && S >= 16 && S <= 512, "octex: sketch width: a multiple of 16, <= 512");
-  const bool lds_slots = gather_smem(W, S, nseg, max_len, true) <= kGatherLds;  // else the slots go to cand
-  const size_t smem    = gather_smem(W, S, nseg, max_len, lds_slots);
+  const bool lds_slots = gather_smem(W, S, nseg, max_len, true, false) <= kGatherLds;  // else the slots go to cand
+  const bool tight     = !lds_slots && gather_smem(W, S, nseg, max_len, false, false) > kGatherLds;
+  const size_t smem    = gather_smem(W, S, nseg, max_len, lds_slots, tight);
   OCTEX_EXPECTS(smem <= kGatherLds, "octex: gather needs %zu bytes of LDS (max 160 KiB)", smem);
   const int cap = gather_cap(W, nseg, max_len);
   OCTEX_EXPECTS(er.count >= 0 && er.count <= 2 && (er.count == 0 || rows), "octex: earlier rows of a row gather");
@@ -2579,7 +2581,7 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
     auto launch             = [&](auto kernel) {
       allow_lds(reinterpret_cast<const void*>(kernel), smem);
       kernel<<<m, wide ? 512 : 256, smem, s>>>(seg, nseg, list_ptr, table, table_len, n, code, scale, qs, S, pitch, W,
-                                               logW, cap, cand, dist, nout, er, nknown);
+                                               logW, cap, tight ? 1 : 0, cand, dist, nout, er, nknown);
     };
     if (!lds_slots)
       launch(&gather_kernel<kRowsTag, LR, NJ, 512, false, kBalanced>);

@@ -64,8 +64,9 @@ void launch_probe(const __half* Y, int m, int C, int L, int B, const float* inv_
                   const bucket_line* lines, int64_t T1, const long long* keys, int64_t Mmax, const int* base, int l,
                   int lr, int logT, int2* seg, hipStream_t s);
 /** LDS bytes of a gather over `nseg` segments per query with hash sets up to W slots; lds_slots: with the
- * candidates' 16-bit slot list in LDS too (else it is kept in the query's row of cand). */
-auto gather_smem(int W, int S, int nseg, int max_len, bool lds_slots) -> size_t;
+ * candidates' 16-bit slot list in LDS too (else it is kept in the query's row of cand); tight: without lds_slots, the
+ * query sketch without the padding between its chunks. */
+auto gather_smem(int W, int S, int nseg, int max_len, bool lds_slots, bool tight) -> size_t;
 /**
  * The distinct ids of every query's segments with their sketch scores into cand / dist [m, W] (ids in any order,
  * count in nout [m]).

@@ -589,6 +589,31 @@ def test_gather_entry_and_lane_splits(L, S, table_len, nst, lens):
         check_gather(rix, segl, qs, cand, dist, nout, rows=False)
 
 
+@pytest.mark.parametrize("nseg", [2325, 2326, 2367])
+def test_gather_fills_the_lds(L, nseg):
+    """At sketch width 512 and a hash set of 2^15 slots a gather takes up to 2,367 segments a query: 160 KiB of LDS hold
+    2,325 of them beside the query sketch's padded chunks, more beside unpadded ones."""
+    import octex_amd
+    from octex_amd._lib import OctexError
+
+    g = np.random.default_rng(nseg)
+    X = np.diag(g.uniform(1, 2, 512).astype(np.float32))  # with its negative a diagonal scatter: nothing to rotate
+    index, _ = octex_amd.build_in_memory(np.concatenate([X, -X]), copies=1, blocks=1, pca_dims=32, list_len=8, table_len=4,
+                                         log_buckets=8, sketch_width=512, member_lists=True, reverse_edges=False, seed=3)
+    rix = O.Index(index)
+    rix.sketch[:] = g.integers(-127, 128, rix.sketch.shape)
+    rdix = dict(lists=dev(rix.lists), table=dev(rix.table), sketch=dev(rix.sketch), scale=dev(rix.scale))
+    seg = np.stack([g.integers(0, rix.n, (3, nseg + 9)), np.full((3, nseg + 9), 4)], -1).astype(np.int32)
+    qs = g.standard_normal((3, 512)).astype(np.float32)
+    print(f"gather of {nseg} segments", flush=True)
+    part = np.ascontiguousarray(seg[:, :nseg])
+    cand, dist, nout = gather_gpu(L, rix, rdix, dev(part), qs, rows=1, W=1 << 15)
+    check_gather(rix, part, qs, cand, dist, nout, rows=True)
+    if nseg == 2367:
+        with pytest.raises(OctexError, match="gather needs \\d+ bytes of LDS"):
+            gather_gpu(L, rix, rdix, dev(seg), qs, rows=1, W=1 << 15)
+
+
 @pytest.mark.parametrize("R,KO", [(24, 40), (512, 64)])
 def test_rerank_keep_thread_counts_agree(L, ix, dix, small_index, R, KO):
     """A launch's queries choose its threads a query (128, 256 or 512; R D >= 2^15 takes twice as many): 20 queries alone,
