@@ -2405,10 +2405,12 @@ void with_lx(int D, F&& f)
 void launch_prepare(const float* q, int n, int m, int D, const float* mu, const float* basis, int S, float* qbuf,
                     float* qc, __half* qh, float* qs, hipStream_t s)
 {
-  if (m == 0 || D == 0) return;
-  OCTEX_EXPECTS(n >= 1 && n <= m, "octex: a batch holds at least one query");
+  if (S == 0) qs = nullptr;  // no sketch coordinates
+  if (m == 0) return;
   OCTEX_EXPECTS(qs == nullptr || (D >= 1 && 16 * static_cast<int64_t>(D) * sizeof(float) <= 64 * 1024),
-                "octex: the sketch query stages 16 query rows of at most 4096 values in LDS");
+                "octex: the sketch query stages 16 query rows of 1 to 1024 values in LDS");
+  if (D == 0 || (qbuf == nullptr && qc == nullptr && qh == nullptr && qs == nullptr)) return;
+  OCTEX_EXPECTS(n >= 1 && n <= m, "octex: a batch holds at least one query");
   // one query a thread up to 2,048 queries (512 workgroups of 4), else four
   const bool few    = m <= 2048;
   const int rows    = few ? 4 : 16;

@@ -512,6 +512,23 @@ def test_stage_errors(L):
                P(x), P(x), i32(1), None)
 
 
+def test_sketch_query_of_no_values(L):
+    """A sketch query of no coordinates or no queries writes nothing; one of rows without values, or of more than its LDS
+    holds, is refused."""
+    from octex_amd._lib import OctexError
+
+    x = torch.ones((2, 1026), device="cuda")
+    qs = torch.full((2, 4), 7.0, device="cuda")
+    L.call("octexStageSketchQuery", P(x), P(x), i32(2), i32(8), i32(0), P(qs), None)
+    L.call("octexStageSketchQuery", P(x), P(x), i32(0), i32(8), i32(4), P(qs), None)
+    assert (qs == 7).all()
+    for D in (0, 1025):
+        with pytest.raises(OctexError, match="16 query rows of 1 to 1024 values"):
+            L.call("octexStageSketchQuery", P(x), P(x), i32(2), i32(D), i32(1), P(qs), None)
+    L.call("octexStageSketchQuery", P(x), P(x), i32(2), i32(1024), i32(1), P(qs), None)
+    assert (qs.flatten()[:2] == 1024).all()
+
+
 # ---------------------------------------------------------------- lane layouts of the row kernels
 
 # (D, S): the sketch scores put a row's S / 16 chunks on that many adjacent lanes (16 and 32 lanes per row at
