@@ -191,6 +191,11 @@ cuvsError_t octexStageTakeK(const int64_t* si, const float* sd, int32_t m, int32
  * [n, kin] (may be NULL) the kept entries nearest first. */
 cuvsError_t octexStageMergeReverse(const int32_t* fwd, const float* fdist, int64_t n, int32_t kin, int32_t kf,
                                    int32_t ks, int32_t kr, int32_t kout, int32_t* table, void* stream);
+/** One k-means update of the builder's IVF lists: centers [nlist, w] = the means of the rows ys [ns, w] of each label
+ * (lab [ns], -1 for none) and cnorm [nlist] their squared norms, from the labels themselves (scan) or from the rows
+ * sorted by label: the same floats.  Centers without members stay; cnorm holds the centers' norms on entry. */
+cuvsError_t octexStageKmeansUpdate(const float* ys, int64_t ns, int32_t w, const int32_t* lab, int32_t nlist,
+                                   int32_t scan, float* centers, float* cnorm, void* stream);
 
 #ifdef __cplusplus
 }

@@ -120,7 +120,8 @@ EXPORTS = (
     "octexIndexCopyArrayRange", "octexIndexCopyArrayRanges", "octexIndexCheckDirectory", "octexSearchNoAlloc",
     "octexStageCenter", "octexStageProject", "octexStageSketchQuery", "octexStageE8", "octexStageProbe",
     "octexStageGather", "octexStageRerankKeep", "octexStageSketchKeep", "octexStagePickStarts",
-    "octexStageFinalRerank", "octexStageTakeK", "octexStageMergeReverse", "octexMeasureRowReads",
+    "octexStageFinalRerank", "octexStageTakeK", "octexStageMergeReverse", "octexStageKmeansUpdate",
+    "octexMeasureRowReads",
 )
 
 _lib = None

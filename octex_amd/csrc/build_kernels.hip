@@ -772,10 +772,11 @@ __global__ void iota_kernel(int* __restrict__ v, int64_t n)
   if (t < n) v[t] = static_cast<int>(t);
 }
 
+/** cnt[c] = the rows of label c; a row of NaN is nearest to no center and has label -1. */
 __global__ void count_labels_kernel(const int* __restrict__ lab, int64_t n, int* __restrict__ cnt)
 {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t < n) atomicAdd(&cnt[lab[t]], 1);
+  if (t < n && lab[t] >= 0) atomicAdd(&cnt[lab[t]], 1);
 }
 
 /**
@@ -1801,6 +1802,39 @@ auto cell_builder::level_streamed(const long long* key, const float* dist, int m
   return M;
 }
 
+void ivf_index::group(int64_t m, hipStream_t s)
+{
+  ensure<int>(off, nlist + 1);
+  ensure<int>(cnt, nlist + 1);
+  ensure<int>(idx, m);
+  ensure<int>(sidx, m);
+  ensure<int>(slab, m);
+  iota_kernel<<<grid_for(m, 256), 256, 0, s>>>(idx.as<int>(), m);
+  const int bits = log2_ceil(nlist) + 1;  // all ones, the low bits of -1, lie above every label
+  with_tmp(tmp, [&](void* p, size_t& b) {
+    return rocprim::radix_sort_pairs(p, b, lab.as<int>(), slab.as<int>(), idx.as<int>(), sidx.as<int>(),
+                                     static_cast<unsigned>(m), 0, bits, s);
+  });
+  OCTEX_HIP(hipMemsetAsync(cnt.ptr, 0, static_cast<size_t>(nlist + 1) * sizeof(int), s));
+  count_labels_kernel<<<grid_for(m, 256), 256, 0, s>>>(lab.as<int>(), m, cnt.as<int>());
+  with_tmp(tmp, [&](void* p, size_t& b) {
+    return rocprim::exclusive_scan(p, b, cnt.as<int>(), off.as<int>(), 0, nlist + 1, rocprim::plus<int>(), s);
+  });
+}
+
+void ivf_index::update(int64_t ns, bool scan, hipStream_t s)
+{
+  if (scan) {
+    kmeans_scan_update_kernel<<<nlist, 256, 0, s>>>(ys.as<float>(), w, lab.as<int>(), static_cast<int>(ns),
+                                                    centers.as<float>(), cnorm.as<float>());
+  } else {
+    group(ns, s);
+    kmeans_update_kernel<<<nlist, 256, 0, s>>>(ys.as<float>(), w, sidx.as<int>(), off.as<int>(), centers.as<float>());
+    row_norms<float>(centers.as<float>(), nlist, w, cnorm.as<float>(), s);
+  }
+  OCTEX_HIP(hipGetLastError());
+}
+
 void ivf_index::build(const float* y, int64_t n_, int w_, int nlist_, double train_fraction, int iters, hipStream_t s)
 {
   n = n_, w = w_, nlist = static_cast<int>(std::min<int64_t>(nlist_, n_));
@@ -1813,29 +1847,11 @@ void ivf_index::build(const float* y, int64_t n_, int w_, int nlist_, double tra
   ensure<float>(ysn, ns);
   ensure<float>(centers, int64_t{nlist} * w);
   ensure<float>(cnorm, nlist);
-  ensure<int>(off, nlist + 1);
-  ensure<int>(cnt, nlist + 1);
   take_rows_kernel<<<grid_for(ns * w, 256), 256, 0, s>>>(y, ns, step, w, ys.as<float>());
   row_norms<float>(ys.as<float>(), ns, w, ysn.as<float>(), s);
   // the first centers: evenly spaced sample rows
   take_rows_kernel<<<grid_for(int64_t{nlist} * w, 256), 256, 0, s>>>(ys.as<float>(), nlist, ns / nlist, w,
                                                                       centers.as<float>());
-  const int bits = log2_ceil(nlist) + 1;
-  auto group = [&](int64_t m) {  // sidx: 0 .. m-1 ordered by lab (stable), off: CSR of the labels
-    ensure<int>(idx, m);
-    ensure<int>(sidx, m);
-    ensure<int>(slab, m);
-    iota_kernel<<<grid_for(m, 256), 256, 0, s>>>(idx.as<int>(), m);
-    with_tmp(tmp, [&](void* p, size_t& b) {
-      return rocprim::radix_sort_pairs(p, b, lab.as<int>(), slab.as<int>(), idx.as<int>(), sidx.as<int>(),
-                                       static_cast<unsigned>(m), 0, bits, s);
-    });
-    OCTEX_HIP(hipMemsetAsync(cnt.ptr, 0, static_cast<size_t>(nlist + 1) * sizeof(int), s));
-    count_labels_kernel<<<grid_for(m, 256), 256, 0, s>>>(lab.as<int>(), m, cnt.as<int>());
-    with_tmp(tmp, [&](void* p, size_t& b) {
-      return rocprim::exclusive_scan(p, b, cnt.as<int>(), off.as<int>(), 0, nlist + 1, rocprim::plus<int>(), s);
-    });
-  };
   auto assign = [&](const float* q, const float* qn, int64_t m) {  // lab [m]: the nearest center of every row
     ensure<int>(lab, m);
     nearest_rows(q, qn, m, centers.as<float>(), cnorm.as<float>(), nlist, w, lab.as<int>(), dtmp, s);
@@ -1846,21 +1862,13 @@ void ivf_index::build(const float* y, int64_t n_, int w_, int nlist_, double tra
   row_norms<float>(centers.as<float>(), nlist, w, cnorm.as<float>(), s);
   for (int it = 0; it < iters; it++) {
     assign(ys.as<float>(), ysn.as<float>(), ns);
-    if (scan) {
-      kmeans_scan_update_kernel<<<nlist, 256, 0, s>>>(ys.as<float>(), w, lab.as<int>(), static_cast<int>(ns),
-                                                      centers.as<float>(), cnorm.as<float>());
-    } else {
-      group(ns);
-      kmeans_update_kernel<<<nlist, 256, 0, s>>>(ys.as<float>(), w, sidx.as<int>(), off.as<int>(), centers.as<float>());
-      row_norms<float>(centers.as<float>(), nlist, w, cnorm.as<float>(), s);
-    }
-    OCTEX_HIP(hipGetLastError());
+    update(ns, scan, s);
   }
   // every row to its nearest center, the rows grouped by center
   ensure<float>(yn, n);
   row_norms<float>(y, n, w, yn.as<float>(), s);
   assign(y, yn.as<float>(), n);
-  group(n);
+  group(n, s);
   rows = dbuf(static_cast<size_t>(n) * sizeof(int));
   OCTEX_HIP(hipMemcpyAsync(rows.ptr, sidx.ptr, rows.size, hipMemcpyDeviceToDevice, s));
   OCTEX_EXPECTS(w % 4 == 0, "octex: IVF lists need rows of a multiple of 4 coordinates");

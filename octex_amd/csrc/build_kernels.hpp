@@ -82,6 +82,12 @@ struct ivf_index {
   dbuf centers, cnorm, off, rows, yc;
   dbuf ys, ysn, yn, lab, slab, idx, sidx, cnt, dtmp, pd, pidx, tmp;
 
+  /** sidx: 0 .. m - 1 ordered by lab (stable; -1, a row of NaN, last), off [nlist + 1]: the CSR of the labels. */
+  void group(int64_t m, hipStream_t s);
+  /** centers [nlist, w] and their norms cnorm from the labels lab of the sample ys [ns, w], by scanning the labels
+   * (ns < 2^31) or from the rows grouped by label: the same floats.  A center without members keeps its place. */
+  void update(int64_t ns, bool scan, hipStream_t s);
+
   /** k-means of `iters` rounds over the rows y[i * step] (about train_fraction of them, at least nlist). */
   void build(const float* y, int64_t n, int w, int nlist, double train_fraction, int iters, hipStream_t s);
   /**

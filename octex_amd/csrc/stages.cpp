@@ -262,3 +262,27 @@ extern "C" cuvsError_t octexStageMergeReverse(const int32_t* fwd, const float* f
     merge_reverse_device(fwd, fdist, n, reverse_rule{kin, kf, ks, kr, kout}, table, s);
   });
 }
+
+extern "C" cuvsError_t octexStageKmeansUpdate(const float* ys, int64_t ns, int32_t w, const int32_t* lab, int32_t nlist,
+                                              int32_t scan, float* centers, float* cnorm, void* stream)
+{
+  return run(stream, [&](hipStream_t s) {
+    need(ys, "ys"), need(lab, "lab"), need(centers, "centers"), need(cnorm, "cnorm");
+    OCTEX_EXPECTS(ns >= 1 && ns < (int64_t{1} << 31) && nlist >= 1 && w >= 1 && w <= 64, "octex: k-means shape");
+    auto in = [&](dbuf& b, const void* src, size_t bytes) {
+      b = dbuf(bytes);
+      OCTEX_HIP(hipMemcpyAsync(b.ptr, src, bytes, hipMemcpyDeviceToDevice, s));
+    };
+    const size_t cb = static_cast<size_t>(nlist) * w * sizeof(float), nb = static_cast<size_t>(nlist) * sizeof(float);
+    ivf_index iv;
+    iv.w = w, iv.nlist = nlist;
+    in(iv.ys, ys, static_cast<size_t>(ns) * w * sizeof(float));
+    in(iv.lab, lab, static_cast<size_t>(ns) * sizeof(int));
+    in(iv.centers, centers, cb);
+    in(iv.cnorm, cnorm, nb);
+    iv.update(ns, scan != 0, s);
+    OCTEX_HIP(hipMemcpyAsync(centers, iv.centers.ptr, cb, hipMemcpyDeviceToDevice, s));
+    OCTEX_HIP(hipMemcpyAsync(cnorm, iv.cnorm.ptr, nb, hipMemcpyDeviceToDevice, s));
+    OCTEX_HIP(hipStreamSynchronize(s));  // before the buffers go
+  });
+}

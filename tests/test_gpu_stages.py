@@ -848,3 +848,41 @@ def test_reverse_edge_merge_of_many_rows(L, n):
     if n == 2:
         back.fill_(-1)  # the same row twice
     assert torch.equal(table[:, 0], fwd) and torch.equal(table[:, 1], back)
+
+
+@pytest.mark.parametrize("w", [8, 16, 24, 32, 40, 48, 64])  # 40, 48 and 24 do not divide a workgroup's 256 threads
+@pytest.mark.parametrize("ns,nlist", [(1, 3), (2047, 5), (2049, 64), (20_000, 300)])
+def test_kmeans_updates_agree(L, w, ns, nlist):
+    """The two k-means updates, over the labels themselves and over the rows sorted by them: the same centers and norms
+    bit for bit, with rows of no label, a center of most rows (more than the scan lists at once) and centers without
+    members, which keep their place; and the means of the rows, to the rounding of sums of that many floats."""
+    g = np.random.default_rng(ns + w)
+    ys = g.standard_normal((ns, w)).astype(np.float32)
+    lab = np.where(g.random(ns) < 0.6, 1, g.integers(-1, nlist, ns)).astype(np.int32)
+    lab[lab == 2] = -1  # a center without members
+    start = g.standard_normal((nlist, w)).astype(np.float32)
+    dys, dlab, none = dev(ys), dev(lab), dev(np.full(ns, -1, np.int32))
+    norms = torch.empty(nlist, device="cuda")
+    got = []
+    for scan in (1, 0):
+        c = dev(start)
+        n = dev(np.zeros(nlist, np.float32))
+        if scan:  # the norms of the centers that stay, as the sorted update sums them
+            L.call("octexStageKmeansUpdate", P(dys), i64(ns), i32(w), P(none), i32(nlist),
+                   i32(0), P(c), P(norms), None)
+            assert np.array_equal(host(c), start)
+            n = norms.clone()
+        print(f"k-means update, scan {scan}, {ns} x {w}, {nlist} centers", flush=True)
+        L.call("octexStageKmeansUpdate", P(dys), i64(ns), i32(w), P(dlab), i32(nlist), i32(scan), P(c), P(n), None)
+        got.append((host(c), host(n)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    c, n = got[0]
+    for k in range(nlist):
+        rows = ys[lab == k].astype(np.float64)
+        if not len(rows):
+            assert np.array_equal(c[k], start[k])
+            continue
+        # each float sum of r terms is off by at most r 2^-24 times the sum of magnitudes, the division by 2^-24
+        bound = (len(rows) + 2) * 2.0**-24 * np.abs(rows).mean(0)
+        assert (np.abs(c[k] - rows.mean(0)) <= bound).all()
+    np.testing.assert_allclose(n, (c.astype(np.float64) ** 2).sum(1), rtol=(w + 1) * 2.0**-24)
