@@ -196,6 +196,10 @@ cuvsError_t octexStageMergeReverse(const int32_t* fwd, const float* fdist, int64
  * sorted by label: the same floats.  Centers without members stay; cnorm holds the centers' norms on entry. */
 cuvsError_t octexStageKmeansUpdate(const float* ys, int64_t ns, int32_t w, const int32_t* lab, int32_t nlist,
                                    int32_t scan, float* centers, float* cnorm, void* stream);
+/** The k-means assignment of the builder's IVF lists: nearest [m] = the row of X [n, w] nearest to each row of
+ * Q [m, w] (fp32, by MFMA; ties by row), -1 for a row of NaN. */
+cuvsError_t octexStageNearest(const float* Q, int64_t m, const float* X, int32_t n, int32_t w, int32_t* nearest,
+                              void* stream);
 
 #ifdef __cplusplus
 }

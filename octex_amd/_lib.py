@@ -121,7 +121,7 @@ EXPORTS = (
     "octexStageCenter", "octexStageProject", "octexStageSketchQuery", "octexStageE8", "octexStageProbe",
     "octexStageGather", "octexStageRerankKeep", "octexStageSketchKeep", "octexStagePickStarts",
     "octexStageFinalRerank", "octexStageTakeK", "octexStageMergeReverse", "octexStageKmeansUpdate",
-    "octexMeasureRowReads",
+    "octexStageNearest", "octexMeasureRowReads",
 )
 
 _lib = None

@@ -1462,10 +1462,6 @@ template void knn_rows<__half>(const __half*, const float*, int64_t, const __hal
 template void knn_rows<float>(const float*, const float*, int64_t, const float*, const float*, int64_t, int, int,
                               float*, int*, hipStream_t);
 
-namespace {
-
-/** out_i [m]: the nearest row of X [n, w] to each row of Q, as knn_rows with K = 1 (dtmp: X's fragments, or knn_rows'
- * distances). */
 void nearest_rows(const float* Q, const float* qn, int64_t m, const float* X, const float* xn, int n, int w, int* out_i,
                   dbuf& dtmp, hipStream_t s)
 {
@@ -1494,8 +1490,6 @@ void nearest_rows(const float* Q, const float* qn, int64_t m, const float* X, co
   }
   OCTEX_HIP(hipGetLastError());
 }
-
-}  // namespace
 
 void half_to_float(const __half* x, int64_t total, float* out, hipStream_t s)
 {

@@ -68,6 +68,11 @@ void drop_self(const int64_t* ids, int64_t r0, int64_t m, int K, int k, int* out
 void drop_self(const int* ids, const float* dist, int64_t r0, int64_t m, int K, int k, int* out, float* out_d,
                hipStream_t s);
 
+/** out_i [m]: the nearest row of X [n, w] to each row of Q (squared norms qn, xn), as knn_rows with K = 1; -1 for a row
+ * of NaN.  tmp: X's fragments, or knn_rows' distances. */
+void nearest_rows(const float* Q, const float* qn, int64_t m, const float* X, const float* xn, int n, int w, int* out_i,
+                  dbuf& tmp, hipStream_t s);
+
 /**
  * An IVF index of one copy's projected rows y [n, w], for the reference's default cell lists (build_cells.cuh:511-516,
  * 584-596: cuVS ivf_flat with max(64, 4 sqrt(n)) lists trained on half the rows, a tenth above 4M, searched with

@@ -286,3 +286,17 @@ extern "C" cuvsError_t octexStageKmeansUpdate(const float* ys, int64_t ns, int32
     OCTEX_HIP(hipStreamSynchronize(s));  // before the buffers go
   });
 }
+
+extern "C" cuvsError_t octexStageNearest(const float* Q, int64_t m, const float* X, int32_t n, int32_t w,
+                                         int32_t* nearest, void* stream)
+{
+  return run(stream, [&](hipStream_t s) {
+    need(Q, "Q"), need(X, "X"), need(nearest, "nearest");
+    OCTEX_EXPECTS(m >= 0 && n >= 1 && w >= 1 && w <= 64, "octex: nearest rows' shape");
+    dbuf qn(static_cast<size_t>(m) * sizeof(float)), xn(static_cast<size_t>(n) * sizeof(float)), tmp;
+    row_norms<float>(Q, m, w, qn.as<float>(), s);
+    row_norms<float>(X, n, w, xn.as<float>(), s);
+    nearest_rows(Q, qn.as<float>(), m, X, xn.as<float>(), n, w, nearest, tmp, s);
+    OCTEX_HIP(hipStreamSynchronize(s));  // before the buffers go
+  });
+}

@@ -232,8 +232,9 @@ def test_exact_table_widths_and_ties(octex, tmp_path, n, d, top):
 
 @pytest.mark.parametrize("n,blocks", [(900, 1), (1500, 3), (70000, 4), (3000, 8)])
 def test_kmeans_centers_give_the_same_ivf_lists(octex, n, blocks):
-    """Every list probed, IVF lists hold the exact l nearest rows whatever the centers are, if every row lies in the
-    list of one center: rows lost or doubled by the assignment (16 rows a workgroup, 64 from 65,536 rows) would show."""
+    """Every list probed (900 rows), IVF lists hold the exact l nearest rows whatever the centers are, if every row lies in
+    the list of one center: rows lost or doubled by the grouping would show.  With more lists than are probed, most
+    entries are exact and a list's rows distinct.  (The assignment itself: test_nearest_rows of the stage tests.)"""
     X = clustered(n=n, m=1, d=64, clusters=9, seed=n)[0].astype(np.float16)
     kw = dict(copies=2, blocks=blocks, list_len=16, log_buckets=10, table_len=0, min_cell=3, seed=2)
     ivf, _ = octex.build_in_memory(X, list_probes=1 << 20, **kw)

@@ -850,6 +850,41 @@ def test_reverse_edge_merge_of_many_rows(L, n):
     assert torch.equal(table[:, 0], fwd) and torch.equal(table[:, 1], back)
 
 
+@pytest.mark.parametrize("w", [8, 16, 24, 32, 40, 48, 64])
+@pytest.mark.parametrize("m,n", [(1, 1), (15, 16), (17, 15), (65, 81), (65_535, 17), (65_536, 63), (65_537, 65)])
+def test_nearest_rows(L, w, m, n):
+    """The nearest of n rows to each of m, 16 rows a workgroup below 65,536 and 64 from there, whose last group and last
+    tile of 16 are full or not.  On integers every distance is exact: the first of the nearest rows; else the chosen
+    row's fp64 distance is the least up to the rounding of |q|^2 + |x|^2 - 2 q.x in fp32.  A row of NaN has none."""
+    g = np.random.default_rng(m + n + w)
+    X = g.integers(-3, 4, (n, w)).astype(np.float32)
+    Q = g.integers(-3, 4, (m, w)).astype(np.float32)
+    out = torch.full((m,), -7, dtype=torch.int32, device="cuda")
+
+    def distances(Q, X):
+        Q, X = dev(Q).double(), dev(X).double()
+        return (Q * Q).sum(1, keepdim=True) - 2 * Q @ X.T + (X * X).sum(1)[None, :]
+
+    def nearest(Q, X):
+        dq, dx = dev(Q), dev(X)
+        print(f"nearest of {n} rows of {w} to {m}", flush=True)
+        L.call("octexStageNearest", P(dq), i64(m), P(dx), i32(n), i32(w), P(out), None)
+        return out.long()
+
+    d = distances(Q, X)
+    first = torch.where(d == d.min(1, keepdim=True).values, torch.arange(n, device="cuda")[None, :], n).min(1).values
+    assert torch.equal(nearest(Q, X), first)
+    X, Q = (g.standard_normal(a.shape).astype(np.float32) for a in (X, Q))
+    d = distances(Q, X)
+    got = nearest(Q, X)
+    assert ((got >= 0) & (got < n)).all()
+    # the dot product and both norms: sums of w terms, each off by (w + 2) 2^-24 of the sum of magnitudes at most
+    scale = dev(Q).double().square().sum(1) + dev(X).double().square().sum(1).max()
+    assert (d.gather(1, got[:, None])[:, 0] - d.min(1).values <= 4 * (w + 2) * 2.0**-24 * scale).all()
+    Q[m // 2, w - 1] = np.nan
+    assert int(nearest(Q, X)[m // 2]) == -1
+
+
 @pytest.mark.parametrize("w", [8, 16, 24, 32, 40, 48, 64])  # 40, 48 and 24 do not divide a workgroup's 256 threads
 @pytest.mark.parametrize("ns,nlist", [(1, 3), (2047, 5), (2049, 64), (20_000, 300)])
 def test_kmeans_updates_agree(L, w, ns, nlist):
