@@ -602,6 +602,9 @@ __device__ __forceinline__ float group_sum(float x)
 // where the slot list is in global memory and the padding does not fit (gather_impl)
 constexpr int kChunkPitch = 18, kTightPitch = 16;
 
+/** The most chunks of a row that a lane of sketch_scores takes (a power of two). */
+__host__ __device__ constexpr auto lane_chunks(int LR) -> int { return LR >= 8 ? 4 : LR == 4 ? 2 : 1; }
+
 /**
  * Sketch scores of a query's candidates 0..n-1 (search_kernels.cuh:227-251): with LR = the next power of two >= S / 16
  * (at most 32), the 16-element chunks sub, sub + LR, ... of a row are summed as u = fma(code, scale, -qs),
@@ -613,6 +616,10 @@ constexpr int kChunkPitch = 18, kTightPitch = 16;
  * arithmetic, 3 instructions a code, and small batches by a wavefront's rows in flight: an LR-lane group with one chunk a
  * lane leaves lanes without a chunk idle (2 of 8 at S = 96), spends a butterfly of log2 LR steps on every 64 / LR rows and
  * has 32 rows in flight a wavefront (LR = 8).  Four chunks a lane leave one step (S <= 128) on 32 rows, 64 in flight.
+ * Shorter rows keep more lanes on a row, one at S <= 32 and two chunks a lane at 48 and 64, since a lane that reads a whole
+ * row has every load touch 64 lines: 10,000 queries of 1,100 list entries (S = 48, rows in the caches) 119 us with three
+ * chunks a lane, 108 with two, 108 with one; 1,600 at S = 32 97 us with two, 91 with one; at S = 96 4096 table entries 203 us
+ * with four, 208 with two, 219 with one.
  * Measured with the entries' loads overlapped too (collect_candidates): the gathers of 1,000 queries of 3840 list and 8192
  * table entries (S = 96) 108, 190 and 104 -> 79, 143 and 77 us on unchanged threads, of one query 23, 30, 20 -> 15, 23,
  * 15 us; 10,000 queries of 4096 table entries over 1.5M rows 552 -> 528 us (45 G rows/s: the random-row ceiling).  The scales and the
@@ -624,7 +631,7 @@ template <int LR, int NJ, typename IdOf, typename Put>
 __device__ __forceinline__ void sketch_scores(int n, IdOf const& id_of, const signed char* __restrict__ code, int S,
                                               int pitch, const float2* sq, int chunk_pitch, Put const& put)
 {
-  constexpr int J     = LR < 4 ? LR : 4;  // chunks of a lane in the butterfly
+  constexpr int J     = lane_chunks(LR);  // chunks of a lane in the butterfly
   constexpr int G     = LR / J;           // lanes per candidate
   constexpr int kRows = 2;                // candidates per group in flight
   constexpr int GPW   = 64 / G;           // groups per wavefront
@@ -2569,12 +2576,16 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
   int Lr = 1;  // the reference's lanes per candidate: the next power of two >= S / 16, at most 32
   while (Lr < S / 16 && Lr < 32)
     Lr <<= 1;
-  // 512 threads a query; 256 for few entries, whose small hash sets leave room for more workgroups.  Measured, 256 / 512
-  // threads: 800 list entries a query 129 / 162 us and 1024 table entries 111 / 179 us (10,000 queries of 128 codes);
-  // 1440 list entries 280 / 279 us; 6400 list entries 74 / 57 us (1,000 queries), 3200 79 / 69 us.  1024 threads leave
-  // one workgroup a CU: 280 -> 506 us.
-  const bool wide = static_cast<int64_t>(nseg) * max_len > kGatherFew || !lds_slots || !kBalanced;
-  const int G  = std::max(1, Lr / 4);         // lanes per candidate and
+  // 256 or 512 threads a query.  A hash set of 8,192 slots and its lists leave room for three workgroups a CU, which need
+  // 512 threads to fill it; below, six and more of 256 hide each other's barriers better, from about two queries a CU.
+  // Fewer queries than that leave CUs to a workgroup or two, and 512 threads shorten its chain when it has more than 1,024
+  // entries.  Measured, 256 / 512 threads, 10,000 queries: 1,100 list entries 129 / 154 us, 1,600 table entries 113 / 174,
+  // 2,600 list entries 175 / 208, 3,200 228 / 204, 4,800 260 / 233, 4096 table entries 215 / 203 (S = 96, rows in the caches);
+  // 1,000 queries of 1,100 list entries 22.0 / 25.9 us, 640 (S = 128) 19.7 / 19.1, 512 17.5 / 16.4, 300 15.8 / 15.0; 300 of 400
+  // 12.3 / 12.2.  1024 threads leave one workgroup a CU: 280 -> 506 us for 10,000 queries of 1,440.
+  const bool wide =
+    W >= kGatherBigSet || !lds_slots || (m <= kGatherFewQueries && static_cast<int64_t>(nseg) * max_len > kGatherFew);
+  const int G  = Lr / lane_chunks(Lr);        // lanes per candidate and
   const int nj = (S / 16 + G - 1) / G;        // chunks a lane: sketch_scores
   auto go = [&](auto rows_tag, auto lr_tag, auto nj_tag) {
     constexpr bool kRowsTag = decltype(rows_tag)::value;
@@ -2589,7 +2600,7 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
       launch(&gather_kernel<kRowsTag, LR, NJ, 512, false, kBalanced>);
     else if (wide)
       launch(&gather_kernel<kRowsTag, LR, NJ, 512, true, kBalanced>);
-    else if constexpr (kBalanced)
+    else
       launch(&gather_kernel<kRowsTag, LR, NJ, 256, true, kBalanced>);
   };
   auto by_nj = [&](auto rows_tag, auto lr_tag) {
@@ -2601,8 +2612,8 @@ void gather_impl(bool rows, const int2* seg, int nseg, int max_len, int m, const
   auto by_lr = [&](auto rows_tag) {
     switch (Lr) {
       case 1: go(rows_tag, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
-      case 2: go(rows_tag, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}); break;
-      case 4: by_nj(rows_tag, std::integral_constant<int, 4>{}); break;
+      case 2: go(rows_tag, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{}); break;
+      case 4: go(rows_tag, std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{}); break;
       case 8: by_nj(rows_tag, std::integral_constant<int, 8>{}); break;
       case 16: by_nj(rows_tag, std::integral_constant<int, 16>{}); break;
       default: by_nj(rows_tag, std::integral_constant<int, 32>{}); break;

@@ -18,7 +18,9 @@ constexpr int kMaxKeepSort    = 1024;   // kept + reranked keys sorted together
 constexpr int kMaxSketchKO    = 1024;   // kept entries of the sketch merge
 constexpr int kPickHash       = 8192;   // hash set of the expanded start points
 constexpr int kMaxExpanded    = 6144;   // start points expanded by earlier waves
-constexpr int kGatherFew      = 1024;   // entries a query up to which a gather takes 256 threads (gather_impl)
+constexpr int kGatherFew      = 1024;   // a gather's threads (gather_impl): entries a query up to which 256 always do
+constexpr int kGatherFewQueries = 512;  // queries up to which more entries take 512, and
+constexpr int kGatherBigSet   = 8192;   // slots of the hash set from which any do
 constexpr int kKeepThreads    = 256;
 
 /** log2 of the hash set of a query reading `total` entries: ceil(log2(1.5 total)) in [11, log_cap]. */

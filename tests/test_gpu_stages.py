@@ -606,6 +606,29 @@ def test_gather_entry_and_lane_splits(L, S, table_len, nst, lens):
         check_gather(rix, segl, qs, cand, dist, nout, rows=False)
 
 
+# a gather's threads: 512 for a set of 8,192 slots, and for more than 1,024 entries of up to 512 queries; 256 otherwise
+@pytest.mark.parametrize("nst,W,m", [(64, 2048, 512), (65, 2048, 512), (65, 2048, 513), (170, 4096, 513), (170, 8192, 513)])
+@pytest.mark.parametrize("S", [32, 64])
+def test_gather_thread_rule(L, S, nst, W, m):
+    import octex_amd
+
+    X, Q = clustered(n=1200, m=8, d=64, clusters=6, seed=S + nst)
+    index, _ = octex_amd.build_in_memory(X, copies=3, blocks=2, pca_dims=32, list_len=8, table_len=16, log_buckets=8,
+                                         sketch_width=S, member_lists=True, reverse_edges=False, seed=3)
+    rix = O.Index(index)
+    rdix = dict(lists=dev(rix.lists), table=dev(rix.table), sketch=dev(rix.sketch), scale=dev(rix.scale))
+    g = np.random.default_rng(S + nst)
+    seg = np.stack([g.integers(0, rix.n, (8, nst)), np.full((8, nst), 16)], -1).astype(np.int32)
+    qs = g.standard_normal((8, S)).astype(np.float32)
+    at = np.arange(m) % 8
+    cand, dist, nout = gather_gpu(L, rix, rdix, dev(seg[at]), np.ascontiguousarray(qs[at]), rows=1, W=W)
+    ref = [O.gather(rix, seg[q], qs[q], rows=True) for q in range(8)]
+    for q in range(m):
+        rc, rd = ref[at[q]]
+        order = np.argsort(cand[q, : nout[q]])
+        assert np.array_equal(cand[q, order], rc) and np.array_equal(dist[q, order], rd)
+
+
 @pytest.mark.parametrize("nseg", [2325, 2326, 2367])
 def test_gather_fills_the_lds(L, nseg):
     """At sketch width 512 and a hash set of 2^15 slots a gather takes up to 2,367 segments a query: 160 KiB of LDS hold
