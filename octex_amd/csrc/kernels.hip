@@ -499,15 +499,25 @@ __global__ __launch_bounds__(256) void probe_kernel(const __half* __restrict__ Y
   }
 }
 
-constexpr int kProbeGroup     = 8;            // lanes of an item in probe_levels_kernel
-constexpr int64_t kProbeLevels = 65536;        // items up to which probe_levels_kernel is taken
+constexpr int kProbeGroup = 8;  // lanes of an item in probe_levels_kernel
+
+/** Items up to which probe_levels_kernel is taken for L levels. */
+constexpr auto probe_levels_items(int L) -> int64_t
+{
+  const int64_t items = int64_t{8192} * (2 * L - 1);
+  return items < 65536 ? items : 65536;
+}
 
 /**
  * probe_kernel for few items: a group of kProbeGroup lanes takes one (query, copy) item, each lane another level, and the
  * finest level that holds the cell wins; more than kProbeGroup levels go in rounds.  All levels cost what the deepest
  * does, so an item takes one decode and one lookup in time, at up to L of them in work: with few wavefronts to run, the
- * chain of levels is what counts.  Measured at 120 items 26 -> 9.5 us, 3,200 items
- * 28 -> 8.6, 60,000 items 32 -> 19; 100,000 items 32 / 29, 120,000 33 / 36, 200,000 35 / 47 us.
+ * chain of levels is what counts, and the longer it is the more items gain.  Measured (a lane an item / a lane a level, us):
+ * one level 5,000 items 8.9 / 8.3, 10,000 9.0 / 9.2, 65,000 10.5 / 18.9; two 24,000 13.1 / 11.0, 48,000 14.5 / 17.0; three
+ * 48,000 18.6 / 16.8, 100,000 21 / 25.5; four 65,000 23.3 / 19.5, 120,000 27 / 28.5; five 120 26 / 9.5, 65,000 27.4 / 19.2,
+ * 100,000 29.6 / 26; eight 150,000 50 / 39.  The line (probe_levels_items) rises with the levels as the crossings do.  It
+ * ends at 65,536 items: where most cells are found at the first of five levels the walk is short, and the crossing is at
+ * 85,000 already (100,000: 21.0 / 24.0).
  */
 template <int B, bool kLines>
 __global__ __launch_bounds__(256) void probe_levels_kernel(const __half* __restrict__ Y, int m, int C, int L,
@@ -2495,7 +2505,7 @@ void launch_probe(const __half* Y, int m, int C, int L, int B, const float* inv_
   const int64_t chunk = std::max<int64_t>(64, (tot + int64_t{24} * cus - 1) / (int64_t{24} * cus));
   const int64_t waves = (tot + chunk - 1) / chunk;
   auto g              = grid_for(waves * 64, 256);
-  if (tot <= kProbeLevels) {
+  if (tot <= probe_levels_items(L)) {
     const unsigned gl = grid_for(tot * kProbeGroup, 256);
 #define OCTEX_PROBE_LEVELS(b)                                                                                         \
   (lines != nullptr ? probe_levels_kernel<b, true><<<gl, 256, 0, s>>>(Y, m, C, L, inv_f, off, lines, T1, keys, Mmax,  \

@@ -247,6 +247,24 @@ def test_probe_few_and_many_items(L, tmp_path, blocks, spacings, stage):
     assert np.array_equal(seg, np.tile(ref, (rep, 1, 1)))
 
 
+@pytest.mark.parametrize("spacings", [[2.5], [2.0, 3.2], [2.0, 2.5, 3.2]])
+def test_probe_on_both_sides_of_its_line(L, tmp_path, spacings):
+    """The items up to which the probe takes a lane a level, 8,192 (2 levels - 1), and the next batch above them."""
+    X, _ = clustered(n=1500, m=10, d=48, clusters=8, seed=12)
+    path = str(tmp_path / "probe")
+    O.build(X, path, copies=8, blocks=2, pca_dims=48, spacings=spacings, list_len=8, table_len=0, log_buckets=5,
+            min_cell=2, member_lists=True, seed=4)
+    pix = O.Index(path)
+    pdix = dict(inv_f=dev(pix.inv_f), offsets=dev(pix.offsets), keys=dev(pix.keys), base=dev(pix.base))
+    Y = queries_Y(pix, X[:200], extra_random=56)
+    ref = O.probe(pix, Y, read=pix.list_len)
+    line = 8192 * (2 * len(spacings) - 1) // 8  # queries of 8 copies
+    for m in (line, line + 1):
+        at = np.arange(m) % len(Y)
+        seg = host(run_probe(L, pix, pdix, np.ascontiguousarray(Y[at]), pix.list_len, PROBES[0]))
+        assert np.array_equal(seg, ref[at])
+
+
 def gather_gpu(L, ix, dix, seg, qs, rows, W=4096):
     m, nseg = seg.shape[0], seg.shape[1]
     cand = torch.full((m, W), -5, dtype=torch.int32, device="cuda")
