@@ -1391,8 +1391,9 @@ void project_rows(const __half* x, int64_t n, int d, const float* mean, const fl
                   float* y, hipStream_t s)
 {
   OCTEX_EXPECTS(w <= kMaxW, "octex: blocks must be at most 8");
-  const size_t smem = static_cast<size_t>(d * w + d) * sizeof(float);  // the largest projection taken
-  OCTEX_EXPECTS(smem <= 160 * 1024, "octex: dimension x 8 blocks too large for the projection kernel");
+  // the builder's limit on a copy's projection: 160 KiB of U and mean, once staged in LDS; no limit of this kernel
+  OCTEX_EXPECTS(static_cast<size_t>(d * w + d) * sizeof(float) <= 160 * 1024,
+                "octex: dimension x 8 blocks too large for the projection kernel");
   if (n == 0) return;
   const unsigned g = grid_for(n, 64);
   auto go          = [&](auto w_tag) {

@@ -1929,14 +1929,13 @@ __device__ __forceinline__ int hist_slot(int* hs, int slots, int v, bool insert)
  * becomes the KO smallest distinct keys of every key merged so far, so an id an earlier round reranked has its exact key
  * either in the kept list already (merging it again changes nothing) or above all KO kept keys (it cannot enter):
  * dropping it leaves the merge's result unchanged.  It is neither read nor merged; nskip [m] (when not null) gets the
- * count.
+ * count.  The window's ids are loaded as the kernel starts and their set (hslots slots, at least twice the window)
+ * cleared, so neither waits after the selection.
  *
  * With next.seg2 the next wave's start points are taken from the merged list (next_starts), with k > 0 (the batch's last
  * round) its first k go to ki / kd and `out`: launches of their own took 4 to 20 us each, here at most 10 (measured, 16
  * queries at the defaults 117 -> 111 us, 10,000 at the deep point 1649 -> 1634).  sketch_keep_kernel does not: its 512
  * threads lost more (227 -> 264 us a wave of 10,000) than the launches cost.
-  The window's ids are loaded as the kernel starts and their set (hslots slots, at least twice the window)
- * cleared, so neither waits after the selection.
  */
 // Eight waves a SIMD: the selection's 64-bit tie bounds took the kernel to about 100 SGPRs, which allow seven (the
 // excess spills to VGPR lanes); measured at 10M rows, the first round's launch went from 94 to 84 us.  Merges of 8
