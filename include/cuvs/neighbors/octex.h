@@ -162,11 +162,10 @@ cuvsError_t cuvsOctexLoad(cuvsResources_t res, const char* path, cuvsOctexLoadPa
  * host or all device.  Host results are complete on return; device results are ordered on the
  * stream of `res`.
  *
- * While that stream is being captured into a graph, device tensors are taken whose parameters, k and number of queries
- * an earlier search had (it allocated the buffers; the capture allocates nothing), and the search's kernels enter the
- * graph, whatever use_graph says.  The index keeps those buffers, apart from other searches', until it is destroyed, and
- * replays are valid as long.  Replays that share them (of one graph, or of searches captured with the same parameters,
- * k and number of queries) must run one after another, and after the searches before the capture.
+ * While that stream is being captured into a graph, device tensors are taken and the search's kernels enter the graph,
+ * whatever use_graph says.  The index keeps the buffers of each captured parameters, k and number of queries, apart from
+ * other searches', until it is destroyed, and replays are valid as long.  Replays that share them (of one graph, or of
+ * searches captured alike) must run one after another, and after the searches before the capture.
  */
 cuvsError_t cuvsOctexSearch(cuvsResources_t res, cuvsOctexSearchParams_t params, cuvsOctexIndex_t index,
                             DLManagedTensor* queries, DLManagedTensor* neighbors, DLManagedTensor* distances);

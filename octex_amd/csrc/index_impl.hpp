@@ -108,8 +108,8 @@ struct index_impl {
   // invalidate, that graph.
   std::mutex stream_mu;
   hipEvent_t searched = nullptr;  // recorded behind every search on its caller's stream; every search waits for it first
-  // Searches under a caller's stream capture (search.cpp, captured_plan): their plans leave the cache, so that no other
-  // search shares the buffers which the captured graph's replays use, and live as long as the index.
+  // The plans of searches under a caller's stream capture (search.cpp, captured_plan): outside the cache, so that no other
+  // search shares the buffers which the captured graph's replays use, for as long as the index lives.
   std::map<std::string, std::shared_ptr<plan>> captured;
   hipEvent_t capture_end        = nullptr;  // recorded behind the last captured search, inside its capture
   unsigned long long capture_id = 0;        // that capture

@@ -419,10 +419,18 @@ auto on_device(const void* p, int device) -> bool
 
 namespace {
 
+/** The calling thread may allocate and wait for other streams while it captures one (its own stream's work is not meant). */
+struct relaxed_capture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  relaxed_capture() { OCTEX_HIP(hipThreadExchangeStreamCaptureMode(&mode)); }
+  relaxed_capture(relaxed_capture const&) = delete;
+  ~relaxed_capture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 /**
- * The plan of a search under stream capture.  A capture permits no allocation, so an earlier search with the same
- * parameters and number of queries must have made the plan.  Its first captured search takes it out of the cache: the
- * captured graph's replays, which no event of the index covers, use its buffers.
+ * The plan of a search under stream capture: that of an earlier search with the same parameters and number of queries,
+ * whose first captured search takes it out of the cache, or a new one (its allocation and first run, on the index's own
+ * stream, lie outside the capture).  The captured graph's replays, which no event of the index covers, use its buffers.
  */
 auto captured_plan(index_impl& ix, search_params const& sp, int m, int k) -> std::shared_ptr<plan>
 {
@@ -431,12 +439,17 @@ auto captured_plan(index_impl& ix, search_params const& sp, int m, int k) -> std
   auto kept = ix.captured.find(key);
   if (kept != ix.captured.end()) return kept->second;
   auto it = ix.plans.find(key);
-  OCTEX_EXPECTS(it != ix.plans.end(),
-                "octex: a search under stream capture needs the buffers of an earlier search with the same parameters, k "
-                "and number of queries: run it once before the capture, or capture octexSearchNoAlloc");
-  auto pl = it->second;
+  std::shared_ptr<plan> pl;
+  if (it != ix.plans.end()) {
+    pl = it->second;
+    ix.plans.erase(it);
+  } else {
+    relaxed_capture guard;
+    search_params direct = sp;
+    direct.use_graph     = false;  // its kernels themselves are captured
+    pl                   = make_plan(ix, direct, m, k);
+  }
   ix.captured.emplace(key, pl);
-  ix.plans.erase(it);
   return pl;
 }
 

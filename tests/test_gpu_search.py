@@ -479,27 +479,33 @@ def test_captured_search_replays(octex, small_index, extra):
             assert np.array_equal(Iw, Ig.cpu().numpy()) and np.array_equal(Dw, Dg.cpu().numpy())
 
 
-def test_captured_search_without_an_earlier_one(octex, small_index):
-    """A capture allocates nothing: without an earlier search of the same shape it is refused before anything is
-    enqueued, the capture ends well, and searches go on."""
-    from octex_amd._lib import OctexError
-
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+@pytest.mark.parametrize("searched", [False, True])
+def test_captured_search_without_an_earlier_one(octex, small_index, mode, searched):
+    """A search captured without an earlier one of its shape, as the index's first search or after others: its buffers
+    are allocated beside the capture, which goes on, and every replay gives the eager results."""
     index = octex.load(small_index["path"])
     Q = small_index["Q"][:40]
-    want = index.search(Q, k=10, **PARAMS)
-    q, side = torch.from_numpy(Q[:39]).cuda(), torch.cuda.Stream()
-    I, D = torch.zeros((39, 10), dtype=torch.int64, device="cuda"), torch.ones((39, 10), device="cuda")
+    if searched:
+        index.search(Q[:5], k=10, **PARAMS)
+    q, side = torch.from_numpy(Q).cuda(), torch.cuda.Stream()
+    I, D = torch.zeros((40, 10), dtype=torch.int64, device="cuda"), torch.ones((40, 10), device="cuda")
+    other = torch.ones(100, device="cuda")
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=side):
-        D.mul_(2)
-        with pytest.raises(OctexError, match="run it once before the capture, or capture octexSearchNoAlloc"):
-            search_into(index, q, I, D, side, **PARAMS)
-    graph.replay()
-    torch.cuda.synchronize()
-    assert (D == 2).all()
-    D1, I1 = index.search(Q, k=10, **PARAMS)
-    assert np.array_equal(I1, want[1]) and np.array_equal(D1, want[0])
+    print(f"capture mode {mode}, searched {searched}", flush=True)
+    with torch.cuda.graph(graph, stream=side, capture_error_mode=mode):
+        other.mul_(2)
+        search_into(index, q, I, D, side, **PARAMS)
+        other.add_(1)
+    for rep in range(3):
+        Qr = np.ascontiguousarray(np.roll(Q, rep, axis=0))
+        q.copy_(torch.from_numpy(Qr))
+        Dw, Iw = index.search(Qr, k=10, **PARAMS)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(Iw, I.cpu().numpy()) and np.array_equal(Dw, D.cpu().numpy())
+    assert (other == 2 ** 3 + 2**2 + 2 + 1).all()
 
 
 def test_plan_buffers_read_behind_a_running_search(octex, small_index):
